@@ -219,6 +219,20 @@ __device__ inline u32x4 nibbles_to_magic_paired(uint32_t w, uint32_t mask, uint3
   return out;
 }
 
+// The widened B operands of two packed dwords (16 codes): (MAGIC | q) pairs in
+// pair order (dword s holds elements s and s + 4 of its 8). The three shifts of
+// each dword are shared between the two as 64-bit funnel shifts; bits shifted
+// in from the high dword land outside the 0x000f000f mask.
+template <int DT>
+__device__ inline void widen_pair(uint32_t lo, uint32_t hi, uint32_t mask, uint32_t magic, u32x4& b0, u32x4& b1) {
+  const uint64_t v = (static_cast<uint64_t>(hi) << 32) | lo;
+  const uint64_t v4 = v >> 4, v8 = v >> 8, v12 = v >> 12;
+  b0 = u32x4{and_or(lo, mask, magic), and_or(static_cast<uint32_t>(v4), mask, magic),
+             and_or(static_cast<uint32_t>(v8), mask, magic), and_or(static_cast<uint32_t>(v12), mask, magic)};
+  b1 = u32x4{and_or(hi, mask, magic), and_or(static_cast<uint32_t>(v4 >> 32), mask, magic),
+             and_or(static_cast<uint32_t>(v8 >> 32), mask, magic), and_or(static_cast<uint32_t>(v12 >> 32), mask, magic)};
+}
+
 // 8 consecutive 16-bit values (4 dwords) reordered 0,4,1,5,2,6,3,7.
 __device__ inline u32x4 permute_x8(u32x4 v) {
   u32x4 out;

@@ -644,6 +644,11 @@ LnqStatus launch_int4_gemv_tiles(const void* xt, const uint8_t* packed, const vo
                                  const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
 LnqStatus launch_x_tiles(const void* x, void* xt, int rows, int K, hipStream_t stream);
 
+// Defined in int4_stream.hip: the streaming few-row product.
+bool int4_stream_supports(int K);
+LnqStatus launch_int4_stream(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
+                             const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
+
 // The split GEMV's workgroup shape for K: past K = 4096 (where the few-row
 // GEMV stops), 64-row blocks and the fewest K chunks of at most 16 slices of
 // 256 inputs, if that leaves a chunk 8 or more (K = 14336: 4 chunks of 14;
@@ -673,8 +678,8 @@ static bool split_shape(int K, int& u8, int& S) {
 // only over the widest outputs (N = 128256 at 32 rows 109.9 against 117.5 for
 // the unsplit 32-row GEMV; N = 28672: 31.5 against 30.6, N = 4096: 11.7 against
 // 11.5, so the rest keep their kernels).
-static bool split_preferred(int M, int N, int K) {
-  if (M < 16 || M > 64 || N % 4 != 0) return false;
+static bool split_preferred(int M, int N, int K, int G) {
+  if (M < 16 || M > 64 || N % 4 != 0 || (G != 128 && G % 256 != 0)) return false;
   if (K > 4096) return true;
   return K == 4096 && M > 16 && N >= 65536;
 }
@@ -779,6 +784,17 @@ static int choose_int4_kernel(int M, int N, int K, int G, int dtype, int kernel,
   return kernel;
 }
 
+// The few-token GEMV's rows: 1..4 on the one-workgroup-per-CU GEMVs, 5..16 on the
+// streaming kernel (bf16, group 128, K = 4096, us on the GEMV / streaming: N = 14336 6 rows
+// 10.6 / 9.7, 16 rows 12.4 / 11.0; N = 4096 6 rows 5.7 / 5.3, 16 rows 7.4 / 6.0; N = 28672
+// 16 rows 22.4 / 19.4; at 4 rows N = 4096 4.8 / 5.1, N = 28672 16.5 / 16.8), 17..32 on the
+// 32-row GEMV, whose products the x-tile entry repeats bit for bit.
+static LnqStatus launch_few_tokens(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
+                                   const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t s) {
+  if (M >= 5 && M <= 16) return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
+  return launch_int4_gemv(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
+}
+
 }  // namespace lnq
 
 using namespace lnq;
@@ -804,13 +820,13 @@ LNQ_API LnqStatus lnq_int4_linear(const void* x, const uint8_t* packed, const vo
   const int code = choose_int4_kernel(M, N, K, G, dtype, kernel, x, packed, scale, zero);
   if (code < 0) return LNQ_ERROR;
   if (code == LNQ_KERNEL_GEMV) {
-    if (M <= 32) return launch_int4_gemv(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
+    if (M <= 32) return launch_few_tokens(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
     // 33..64 rows over a wide output: the few-token GEMV once per 32-row chunk.
     const size_t xrow = static_cast<size_t>(K) * 2, yrow = static_cast<size_t>(N) * 2;
     for (int c = 0; c < M; c += 32) {
       const int rc = M - c < 32 ? M - c : 32;
-      const LnqStatus st = launch_int4_gemv(static_cast<const uint8_t*>(x) + c * xrow, packed, scale, zero, bias,
-                                            static_cast<uint8_t*>(y) + c * yrow, rc, N, K, G, dtype, s);
+      const LnqStatus st = launch_few_tokens(static_cast<const uint8_t*>(x) + c * xrow, packed, scale, zero, bias,
+                                             static_cast<uint8_t*>(y) + c * yrow, rc, N, K, G, dtype, s);
       if (st != LNQ_OK) return st;
     }
     return LNQ_OK;
@@ -820,6 +836,10 @@ LNQ_API LnqStatus lnq_int4_linear(const void* x, const uint8_t* packed, const vo
   if (code == LNQ_KERNEL_TILED_128 || code == LNQ_KERNEL_TILED_256)
     return launch_int4_tiled(x, packed, scale, zero, bias, y, M, N, K, G, dtype,
                              code == LNQ_KERNEL_TILED_256 ? 256 : 128, s);
+  // The rest of the few-row calls (LNQ_KERNEL_SKINNY as the plan names them) stream; the
+  // skinny kernel runs when it is asked for, and past the streaming kernel's widest layer.
+  if (kernel == LNQ_KERNEL_AUTO && int4_stream_supports(K))
+    return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
   if (dtype == LNQ_BF16)
     return launch_skinny<LNQ_BF16>(x, packed, scale, zero, bias, y, M, N, K, G, s);
   return launch_skinny<LNQ_F16>(x, packed, scale, zero, bias, y, M, N, K, G, s);
@@ -858,7 +878,7 @@ LNQ_API LnqStatus lnq_int4_linear_workspace(int64_t rows, int64_t in_features, i
   const int M = static_cast<int>(rows), N = static_cast<int>(out_features), K = static_cast<int>(in_features);
   int u8 = 0, S = 0;
   const bool shaped = rows > 0 && split_shape(K, u8, S);
-  if (kernel == LNQ_KERNEL_SPLIT || (kernel == LNQ_KERNEL_AUTO && shaped && split_preferred(M, N, K))) {
+  if (kernel == LNQ_KERNEL_SPLIT || (kernel == LNQ_KERNEL_AUTO && shaped && split_preferred(M, N, K, static_cast<int>(group)))) {
     static const uint8_t* const kAligned = reinterpret_cast<const uint8_t*>(static_cast<uintptr_t>(256));
     LNQ_REQUIRE(rows == 0 || (shaped && rows <= 64 &&
                               int4_gemv_split_supports(M < 32 ? M : 32, N, K, static_cast<int>(group), u8, S,

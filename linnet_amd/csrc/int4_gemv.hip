@@ -123,20 +123,6 @@ struct GemvPrologue {
     return base + w * wb + (T % P) * 2048;                                                        \
   }
 
-// The widened B operands of two packed dwords (16 codes): (MAGIC | q) pairs in
-// pair order (dword s holds elements s and s + 4 of its 8). The three shifts of
-// each dword are shared between the two as 64-bit funnel shifts; bits shifted
-// in from the high dword land outside the 0x000f000f mask.
-template <int DT>
-__device__ inline void widen_pair(uint32_t lo, uint32_t hi, uint32_t mask, uint32_t magic, u32x4& b0, u32x4& b1) {
-  const uint64_t v = (static_cast<uint64_t>(hi) << 32) | lo;
-  const uint64_t v4 = v >> 4, v8 = v >> 8, v12 = v >> 12;
-  b0 = u32x4{and_or(lo, mask, magic), and_or(static_cast<uint32_t>(v4), mask, magic),
-             and_or(static_cast<uint32_t>(v8), mask, magic), and_or(static_cast<uint32_t>(v12), mask, magic)};
-  b1 = u32x4{and_or(hi, mask, magic), and_or(static_cast<uint32_t>(v4 >> 32), mask, magic),
-             and_or(static_cast<uint32_t>(v8 >> 32), mask, magic), and_or(static_cast<uint32_t>(v12 >> 32), mask, magic)};
-}
-
 // Workgroup: NW = K / 256 waves, R = 8 * U8 rows. G128: group 128 (a wave's two
 // halves have consecutive groups, scales loaded as one dword); otherwise G is
 // a multiple of 256 (both halves share one group).
@@ -676,14 +662,12 @@ __global__ __launch_bounds__(64 * gemv::MAX_WAVES) void int4_gemv_slices_kernel(
   }
 }
 
-// A few tokens (2..MX rows, MX = 4 or 16): the one-token kernel's workgroup
+// A few tokens (2..MX rows, MX = 4; more stream, stream.hpp): the one-token kernel's workgroup
 // shape and weight streams, with A-operand row m of every MFMA holding x row m
 // (lane col = m). The order of the inputs within a wave's 256 is free as long
 // as A and B agree, so MFMA t of half H takes inputs 128 H + 32 t + 8 j .. + 7
-// in lane (col, j): at 16 rows each lane loads its own A operands straight from
-// x, an instruction reading 16 rows x 64 contiguous bytes (rows past M read
-// zeros through the range check; up to 4 rows the loads are two rows x 512
-// bytes, put in operand order through LDS). The B operands follow: lane (col,
+// in lane (col, j): x loads are two rows x 512 bytes, put in operand order through
+// LDS (rows past M read zeros through the range check). The B operands follow: lane (col,
 // j) reads dword j of the 16-byte pieces 4 H + t of its weight row. The output
 // registers of a tile hold rows 4 (lane / 16) + i; the fold takes each row's sum
 // of x from the lanes that loaded it, and after a barrier the 16 waves' partial
@@ -735,25 +719,15 @@ __global__ __launch_bounds__(64 * gemv::MAX_WAVES) void int4_gemv_rows_kernel(
     zv16 = __builtin_amdgcn_raw_buffer_load_b8(rz, srow * groups + g0, 0, 0);
   }
   __builtin_amdgcn_sched_barrier(0);
-  // 16 rows: each lane loads its A operands. Up to 4 rows, loads of two rows
-  // x 256 inputs (lanes 0..31 row 2 i, 32..63 row 2 i + 1) move x to registers
+  // Loads of two rows x 256 inputs (lanes 0..31 row 2 i, 32..63 row 2 i + 1) move x to registers
   // with fewer instructions, and one pass through a wave-private LDS slot puts
   // it in operand order (A rows past 4 are zeros).
   u32x4 xa[2][4];
   u32x4 xc[2];
-  if constexpr (MX == 16) {
 #pragma unroll
-    for (int H = 0; H < 2; ++H)
-#pragma unroll
-      for (int t = 0; t < 4; ++t)
-        xa[H][t] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, (col * K + k0 + 128 * H + 32 * t + 8 * j) * 2, 0, 0));
-  } else {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      xc[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                            rx, ((2 * i + (lane >> 5)) * K + k0 + 8 * (lane & 31)) * 2, 0, 0));
-  }
+  for (int i = 0; i < 2; ++i)
+    xc[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                          rx, ((2 * i + (lane >> 5)) * K + k0 + 8 * (lane & 31)) * 2, 0, 0));
   __builtin_amdgcn_sched_barrier(0);
   {
     const int a = lane >> 4, b = lane & 15;
@@ -771,24 +745,21 @@ __global__ __launch_bounds__(64 * gemv::MAX_WAVES) void int4_gemv_rows_kernel(
   // halves, then the A operands in pair order.
   wait_vm<U8>();
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (MX != 16) {
-    static_assert(MX == 4, "4 or 16 rows");
-    __shared__ __attribute__((aligned(16))) uint16_t Xst[gemv::MAX_WAVES][4 * 256];
-    uint16_t* Xw = Xst[wave];
-    *reinterpret_cast<u32x4*>(Xw + 256 * (lane >> 5) + 8 * (lane & 31)) = xc[0];
-    *reinterpret_cast<u32x4*>(Xw + 256 * (2 + (lane >> 5)) + 8 * (lane & 31)) = xc[1];
+  __shared__ __attribute__((aligned(16))) uint16_t Xst[gemv::MAX_WAVES][4 * 256];
+  uint16_t* Xw = Xst[wave];
+  *reinterpret_cast<u32x4*>(Xw + 256 * (lane >> 5) + 8 * (lane & 31)) = xc[0];
+  *reinterpret_cast<u32x4*>(Xw + 256 * (2 + (lane >> 5)) + 8 * (lane & 31)) = xc[1];
+#pragma unroll
+  for (int H = 0; H < 2; ++H)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) xa[H][t] = u32x4{0u, 0u, 0u, 0u};
+  // Only the reads are under the lane condition.
+  if (col < 4) {
 #pragma unroll
     for (int H = 0; H < 2; ++H)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) xa[H][t] = u32x4{0u, 0u, 0u, 0u};
-    // Only the reads are under the lane condition.
-    if (col < 4) {
-#pragma unroll
-      for (int H = 0; H < 2; ++H)
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          xa[H][t] = *reinterpret_cast<const u32x4*>(Xw + 256 * col + 128 * H + 32 * t + 8 * j);
-    }
+      for (int t = 0; t < 4; ++t)
+        xa[H][t] = *reinterpret_cast<const u32x4*>(Xw + 256 * col + 128 * H + 32 * t + 8 * j);
   }
   // The sums of x over each half on the matrix core (A = x, B = ones): lane
   // (col, j) register i is the sum of x row 4 j + i, the row its output
@@ -1585,9 +1556,6 @@ LnqStatus launch_int4_gemv(const void* x, const uint8_t* packed, const void* sca
   } else if (M <= 4) {
     if (dtype == LNQ_BF16) launch_rows_dt<LNQ_BF16, 4>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
     else launch_rows_dt<LNQ_F16, 4>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
-  } else if (M <= 16) {
-    if (dtype == LNQ_BF16) launch_rows_dt<LNQ_BF16, 16>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
-    else launch_rows_dt<LNQ_F16, 16>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
   } else {
     if (dtype == LNQ_BF16) launch_rows32_dt<LNQ_BF16, false>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
     else launch_rows32_dt<LNQ_F16, false>(x, packed, scale, zero, bias, y, M, N, K, G, stream);

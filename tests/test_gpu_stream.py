@@ -1,0 +1,73 @@
+"""The streaming few-row product (`csrc/stream.hpp`) in every weight format, against the f64
+product of the exactly dequantized weight: row counts at the edges of its forms (4, 8, 16,
+32 rows of x a workgroup, chunks of 32), K that ends inside a wave's share or a 256-input
+line, a partial last tile and workgroup, groups within, of and over a 128-input step,
+scales and zero points at odd addresses, and rows of x past the last.
+
+Bound: half a unit in the last place of the result (one rounding; one more with a bias),
+plus 16 f32 units of the sum of the products' magnitudes as they are added -- int4 codes
+carry 128 (f16: 1024) plus the zero point, int8 in bf16 carries 128, until the fold."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from linnet_amd.torch import kernels
+from oracle import linear, quant
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+ULP = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}
+BF16, F16 = torch.bfloat16, torch.float16
+
+
+def _x(rows: int, width: int, dtype: torch.dtype) -> torch.Tensor:
+    return torch.randn(rows, width, generator=torch.Generator().manual_seed(rows + width)).to(dtype)
+
+
+def _check(got: torch.Tensor, x: torch.Tensor, w: np.ndarray, carried: np.ndarray, bias: torch.Tensor | None = None) -> None:
+    """`w` [Out, In] f64; `carried` the magnitudes the kernel adds up for each weight."""
+    xd = x.double().numpy()
+    ref = xd @ w.T
+    bound = ULP[x.dtype] * np.abs(ref)
+    if bias is not None:
+        ref = ref + bias.double().numpy()
+        bound = bound + ULP[x.dtype] * np.abs(ref)
+    bound = bound + 2.0**-20 * (np.abs(xd) @ carried.T) + 2.0**-24
+    err = np.abs(got.double().cpu().numpy() - ref)
+    print(f"max err / bound {float((err / bound).max()):.3f}", flush=True)
+    assert got.shape == ref.shape and np.all(err <= bound)
+
+
+@pytest.mark.parametrize(("rows", "out", "width", "group", "dtype"), [
+    (1, 40, 128, 32, BF16),  # one step, one wave, a partial tile
+    (4, 300, 1152, 64, F16),  # 9 steps: an odd last unit; 4-row form
+    (5, 2049, 1024, 128, BF16),  # GEMV's rows 5..16, a ragged last workgroup
+    (8, 96, 2176, 128, F16),  # 17 groups: scale rows at odd addresses
+    (9, 4100, 640, 32, BF16),  # 32 rows a workgroup, its last of 4
+    (16, 520, 3072, 384, F16),  # a group of three steps
+    (17, 130, 4352, 256, BF16),  # 32-row form, a group of two steps
+    (33, 24, 14336, 64, BF16),  # two chunks; long K; 8 rows a workgroup
+    (16, 14336, 4096, 64, F16),  # every wave two units, 56 rows a workgroup, one workgroup a CU
+    (64, 20000, 256, 64, F16),  # more workgroups than CUs, one unit of weights
+    (20, 512, 8192, 32, BF16),  # scales past the LDS beside 32 rows: fewer rows a workgroup
+])
+def test_int4(rows: int, out: int, width: int, group: int, dtype: torch.dtype) -> None:
+    print(f"int4 stream rows={rows} out={out} in={width} group={group} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(out + width)
+    groups = width // group
+    packed = torch.randint(0, 256, (out, groups, group // 2), generator=g, dtype=torch.uint8)
+    scale = (torch.rand(out * groups + 1, generator=g) * 0.02 + 0.001).to(dtype)[1:].view(out, groups)
+    zero = torch.randint(0, 16, (out * groups + 3,), generator=g, dtype=torch.uint8)[3:].view(out, groups)
+    bias = torch.randn(out, generator=g).to(dtype) if rows % 2 else None
+    # Contiguous views one scale and three zero points into their buffers on the GPU.
+    sd = torch.cat([scale.reshape(-1)[:1], scale.reshape(-1)]).to(DEV)[1:].view(out, groups)
+    zd = torch.cat([zero.reshape(-1)[:3], zero.reshape(-1)]).to(DEV)[3:].view(out, groups)
+    x = _x(rows, width, dtype)
+    got = kernels.int4_linear(x.to(DEV), packed.to(DEV), sd, zd, None if bias is None else bias.to(DEV))
+    q = quant.unpack_int4_codes(packed.numpy()).reshape(out, groups, group).astype(np.float64)
+    s, z = scale.double().numpy()[..., None], zero.double().numpy()[..., None]
+    offset = 128.0 if dtype == BF16 else 1024.0
+    _check(got, x, ((q - z) * s).reshape(out, width), ((q + z + 2 * offset) * s).reshape(out, width), bias)
