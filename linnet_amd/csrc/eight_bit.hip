@@ -9,6 +9,7 @@
 //                 its block-scaled FP8 form: fp8_block.hip);
 //   - int8_quantize: symmetric group-wise int8 rounding, bit-exact with numpy.
 #include "eight_bit.hpp"
+#include "stream.hpp"
 
 namespace lnq {
 
@@ -77,18 +78,14 @@ __device__ inline void widen4(uint32_t w, uint32_t& d0, uint32_t& d1) {
 // feeds MFMA t (t = 0, 1) elements 8t..8t+7 of them. A group (of `group`
 // inputs, or the whole row when the scale is per row) closes with
 //   acc += s * (C - offset * Cx),  Cx = sum of x over the group (B = ones).
-// ONE (one row of x, MT = 1): x is staged in LDS once (dynamic shared memory
-// of K 16-bit values) and the ring holds only weight bytes, 16 chunks deep.
-template <int DT, int FP8, int MT, bool ONE = false>
+template <int DT, int FP8, int MT>
 __global__ __launch_bounds__(256) void w8_skinny_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ weight,
     const float* __restrict__ scale, uint16_t* __restrict__ y, int M, int N, int K, int G,
     int row_block, int scale_cols) {
   using E = Elem<DT>;
   constexpr float offset = FP8 ? 0.0f : 128.0f;
-  static_assert(!ONE || MT == 1, "the one-row form has one x tile");
   __shared__ f32x4 red[4][MT][64];
-  extern __shared__ __attribute__((aligned(16))) uint16_t xl[];
 
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -128,28 +125,20 @@ __global__ __launch_bounds__(256) void w8_skinny_kernel(
   // A ring of D chunks in flight per wave: the weight bytes (streamed once,
   // non-temporal) and the x values they meet, requested D chunks ahead so the
   // wave keeps D loads of each in flight instead of waiting on every chunk.
-  constexpr int D = ONE ? 16 : MT == 1 ? 8 : MT == 2 ? 4 : 2;
+  constexpr int D = MT == 1 ? 8 : MT == 2 ? 4 : 2;
   u32x4 rw[D];
-  u32x4 rx[ONE ? 1 : D][MT][2];
+  u32x4 rx[D][MT][2];
   auto fetch = [&](int slot, int c) {
     rw[slot] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow + 64 * c + 16 * j));
-    if constexpr (!ONE) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
-          rx[slot][mt][t] = *reinterpret_cast<const u32x4*>(xrow[mt] + 64 * c + 16 * j + 8 * t);
-    }
+      for (int t = 0; t < 2; ++t)
+        rx[slot][mt][t] = *reinterpret_cast<const u32x4*>(xrow[mt] + 64 * c + 16 * j + 8 * t);
   };
 #pragma unroll
   for (int i = 0; i < D; ++i)
     if (cb + i < ce) fetch(i, cb + i);
-  if constexpr (ONE) {
-    // Staged while the first D weight chunks are in flight.
-    for (int i = 8 * threadIdx.x; i < K; i += 8 * 256)
-      *reinterpret_cast<u32x4*>(&xl[i]) = *reinterpret_cast<const u32x4*>(&x[i]);
-    __syncthreads();
-  }
   for (int c0 = cb; c0 < ce; c0 += D) {
 #pragma unroll
     for (int i = 0; i < D; ++i) {
@@ -157,17 +146,10 @@ __global__ __launch_bounds__(256) void w8_skinny_kernel(
       if (c >= ce) break;
       const u32x4 w = rw[i];
       u32x4 xa[MT][2];
-      if constexpr (ONE) {
-        // Every lane takes row 0: the 15 copies of it land in output rows
-        // past M, which are not stored.
 #pragma unroll
-        for (int t = 0; t < 2; ++t) xa[0][t] = *reinterpret_cast<const u32x4*>(&xl[64 * c + 16 * j + 8 * t]);
-      } else {
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) xa[mt][t] = mok[mt] ? rx[i][mt][t] : u32x4{0u, 0u, 0u, 0u};
-      }
+        for (int t = 0; t < 2; ++t) xa[mt][t] = mok[mt] ? rx[i][mt][t] : u32x4{0u, 0u, 0u, 0u};
       if (c + D < ce) fetch(i, c + D);
       const uint32_t words[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -215,9 +197,8 @@ __global__ __launch_bounds__(256) void w8_skinny_kernel(
 }
 
 // =================================================================== one row
-// One row of x (a decoding step), groups a multiple of 128 inputs, K % 512 == 0.
-// The skinny kernel's workgroups (16 output features, 4 waves each a quarter of
-// K, x staged in LDS) with wider reads: a wave instruction reads 8 rows x 128
+// One row of x (a decoding step), groups a multiple of 128 inputs.
+// The skinny kernel's workgroups (16 output features) with wider reads: a wave instruction reads 8 rows x 128
 // contiguous bytes (lane: row l % 8, 16-byte piece l / 8) instead of 16 rows x 64
 // bytes, which streams faster (a 235 MB pure read in this workgroup shape: 34-35
 // against 39 us). Lane l then holds, for B column c = l % 16, piece 2 (l / 16) +
@@ -225,162 +206,12 @@ __global__ __launch_bounds__(256) void w8_skinny_kernel(
 // of the same 8 rows, so A row 0 takes x at the even pieces and A row 1 at the
 // odd ones, and row r's sum is C[0][r] + C[1][8 + r]. Two loads (rows 0-7 and
 // 8-15) per 128 inputs, each two MFMA 16x16x32 (bytes 0-7 and 8-15 of a piece).
-//
-// NW waves split K; D loads in flight per wave. K = 4096 runs
-// w8_row_slices_kernel below instead.
-template <int DT, int FP8, int NW = 4, int D = 16>
-__global__ __launch_bounds__(64 * NW) void w8_row_kernel(const uint16_t* __restrict__ x,
-                                                         const uint8_t* __restrict__ weight,
-                                                         const float* __restrict__ scale,
-                                                         uint16_t* __restrict__ y, int N, int K, int G,
-                                                         int row_block, int scale_cols) {
-  using E = Elem<DT>;
-  constexpr float offset = FP8 ? 0.0f : 128.0f;
-  constexpr int THREADS = 64 * NW;
-  __shared__ float red[NW][16];
-  extern __shared__ __attribute__((aligned(16))) uint16_t xl[];
-
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int col = lane & 15;
-  const int j = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int steps = K >> 7;  // 128 inputs a step
-  const int per_wave = steps / NW;
-  const int sb = wave * per_wave, se = sb + per_wave;
-  const int steps_per_group = G >> 7;
-
-  // Load rows: half h reads rows n0 + 8h + l % 8 (clamped: rows past N are not stored).
-  const uint8_t* wrow[2];
-  const float* srow[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    wrow[h] = weight + static_cast<size_t>(min(n0 + 8 * h + (lane & 7), N - 1)) * K + 16 * (lane >> 3);
-    // The scale of this lane's B column (row n0 + 8h + col % 8).
-    const int srow_n = min(n0 + 8 * h + (col & 7), N - 1);
-    srow[h] = scale + static_cast<size_t>(srow_n / row_block) * scale_cols;
-  }
-  u32x4 ones;
-  ones.x = ones.y = ones.z = ones.w = E::ONE2;
-  f32x4 acc[2], C[2], Cx;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-    C[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  Cx = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  u32x4 rw[D];
-  auto fetch = [&](int slot, int step) {
-    rw[slot] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wrow[slot & 1] + 128 * step));
-  };
-  // x and the scales of the wave's first group into registers first, then the
-  // ring's weight loads, and only then x into LDS: a store of x right after its
-  // load would hold every weight load back by x's round trip. (Loads retire in
-  // issue order, so x and the scales land ahead of the weights.)
-  constexpr int XR = 8192 / (8 * THREADS);  // x chunks a thread loads (K <= 8192 from registers)
-  u32x4 xr[XR];
-#pragma unroll
-  for (int r = 0; r < XR; ++r) {
-    const int i = 8 * (threadIdx.x + THREADS * r);
-    xr[r] = i < K ? *reinterpret_cast<const u32x4*>(&x[i]) : u32x4{0u, 0u, 0u, 0u};
-  }
-  const int g_first = sb / steps_per_group;
-  float s_first[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) s_first[h] = srow[h][g_first];
-  __asm__ volatile("" ::: "memory");
-  // (Unconditional: a wave with fewer than D / 2 steps re-reads its last one,
-  // unused, so that the number of loads in flight is known where x is stored.)
-#pragma unroll
-  for (int i = 0; i < D; ++i) fetch(i, min(sb + (i >> 1), se - 1));
-  __asm__ volatile("" ::: "memory");
-#pragma unroll
-  for (int r = 0; r < XR; ++r) {
-    const int i = 8 * (threadIdx.x + THREADS * r);
-    if (i < K) *reinterpret_cast<u32x4*>(&xl[i]) = xr[r];
-  }
-  for (int i = 8 * (threadIdx.x + THREADS * XR); i < K; i += 8 * THREADS)
-    *reinterpret_cast<u32x4*>(&xl[i]) = *reinterpret_cast<const u32x4*>(&x[i]);
-  __syncthreads();
-  // A row m (lane m = l % 16): x at piece 2 j + (m & 1); rows 2..15 repeat rows
-  // 0 / 1 and their outputs are not used.
-  const int apiece = 2 * j + (col & 1);
-  for (int s0 = sb; s0 < se; s0 += D / 2) {
-#pragma unroll
-    for (int i = 0; i < D / 2; ++i) {
-      const int step = s0 + i;
-      if (step >= se) break;
-      u32x4 xa[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) xa[t] = *reinterpret_cast<const u32x4*>(&xl[128 * step + 16 * apiece + 8 * t]);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const u32x4 w = rw[2 * i + h];
-        if (step + D / 2 < se) fetch(2 * i + h, step + D / 2);
-        const uint32_t words[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          uint32_t b0, b1, b2, b3;
-          widen4<DT, FP8>(words[2 * t], b0, b1);
-          widen4<DT, FP8>(words[2 * t + 1], b2, b3);
-          C[h] = mfma16x16x32<DT>(xa[t], u32x4{b0, b1, b2, b3}, C[h]);
-        }
-      }
-      if constexpr (!FP8) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t) Cx = mfma16x16x32<DT>(xa[t], ones, Cx);
-      }
-      // A group closes at its last step or where this wave's quarter of K ends.
-      if ((step + 1) % steps_per_group == 0 || step + 1 == se) {
-        const int g = step / steps_per_group;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float sc = s_first[h];
-          if (g != g_first) {
-            // (The asm keeps this load in its branch: loaded speculatively, the
-            // wait for it would add a round trip to every group's end.)
-            __asm__ volatile("" ::: "memory");
-            sc = srow[h][g];
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float d = FP8 ? C[h][r] : fmaf(-offset, Cx[r], C[h][r]);
-            acc[h][r] = fmaf(sc, d, acc[h][r]);
-          }
-          C[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        Cx = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-    }
-  }
-  // Lane col (j = 0) holds A row 0 in register 0 and row 1 in register 1: row
-  // col % 8 of half h is C[0][col % 8] + C[1][8 + col % 8].
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const float mine = col < 8 ? acc[h][0] : acc[h][1];
-    const float v = mine + __shfl_xor(mine, 8, 64);
-    if (j == 0 && col < 8) red[wave][8 * h + col] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x < 16) {
-    const int n = n0 + threadIdx.x;
-    float v = red[0][threadIdx.x];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) v += red[w][threadIdx.x];
-    if (n < N) y[n] = E::from_f32(v);
-  }
-}
-
-// One row of x at K = 4096 (config 1's int8 4096 x 4096 GEMV): the workgroups
-// and loads of w8_row_kernel (16 output features, lane l reading row l % 8,
-// piece l / 8 of a 128-input step), with K split over 16 waves of 2 steps, so
-// every load of a CU is in flight at once and each wave multiplies as soon as
+// K = 4096 (config 1's int8 4096 x 4096 GEMV), split over 16 waves of 2 steps: every
+// load of a CU is in flight at once and each wave multiplies as soon as
 // its own loads land. Each wave loads just the 256 inputs of x its steps use,
 // straight into its MFMA A-operand registers (32 bytes of x a lane a step,
 // issued before the weights): no LDS stage of x and no workgroup barrier ahead of
-// the products (6.2 -> 5.6 us for config 1). The sums are w8_row_kernel's, in
-// the same order (the same bits).
+// the products (6.2 -> 5.6 us for config 1).
 template <int DT, int FP8>
 __global__ __launch_bounds__(1024) void w8_row_slices_kernel(const uint16_t* __restrict__ x,
                                                              const uint8_t* __restrict__ weight,
@@ -464,7 +295,7 @@ __global__ __launch_bounds__(1024) void w8_row_slices_kernel(const uint16_t* __r
       for (int h = 0; h < 2; ++h) {
         float sc = s_first[h];
         if (g != g_first) {
-          // (The asm keeps this load in its branch, as in w8_row_kernel.)
+          // (The asm keeps this load in its branch.)
           __asm__ volatile("" ::: "memory");
           sc = srow[h][g];
         }
@@ -478,7 +309,7 @@ __global__ __launch_bounds__(1024) void w8_row_slices_kernel(const uint16_t* __r
       Cx = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
-  // Row col % 8 of half h is C[0][col % 8] + C[1][8 + col % 8] (w8_row_kernel).
+  // Row col % 8 of half h is C[0][col % 8] + C[1][8 + col % 8].
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const float mine = col < 8 ? acc[h][0] : acc[h][1];
@@ -697,26 +528,22 @@ __global__ __launch_bounds__(256) void int8_quantize_kernel(const float* __restr
 
 // ================================================================ launchers
 
+// Defined in fp8_stream.hip, int8_stream.hip: the streaming few-row product.
+LnqStatus launch_fp8_stream(const void* x, const uint8_t* w, const float* scale, void* y, int M, int N, int K, int group,
+                            int row_block, int dtype, hipStream_t stream);
+LnqStatus launch_int8_stream(const void* x, const uint8_t* w, const float* scale, void* y, int M, int N, int K, int group,
+                             int row_block, int dtype, hipStream_t stream);
+
+// The row kernel (one row, K = 4096, scales of 128 k inputs), or the skinny kernel where
+// the streaming product does not reach (stream::MAX_K).
 template <int DT, int FP8>
-static void launch_w8_skinny(const void* x, const uint8_t* w, const float* s, void* y, int M,
+static void launch_w8_few(const void* x, const uint8_t* w, const float* s, void* y, int M,
                              int N, int K, int G, int rb, int cols, hipStream_t stream) {
   const auto* xs = static_cast<const uint16_t*>(x);
   auto* ys = static_cast<uint16_t*>(y);
-  if (M == 1 && K == 4096 && G % 128 == 0)
+  if (M == 1 && K == 4096)
     hipLaunchKernelGGL((w8_row_slices_kernel<DT, FP8>), dim3((N + 15) / 16), dim3(1024), 0, stream, xs, w, s, ys, N, G,
                        rb, cols);
-  else if (M == 1 && K <= 32768 && K % 512 == 0 && G % 128 == 0)
-    hipLaunchKernelGGL((w8_row_kernel<DT, FP8>), dim3((N + 15) / 16), dim3(256), K * 2, stream, xs, w, s, ys, N, K, G,
-                       rb, cols);
-  else if (M == 1 && K <= 32768)
-    hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 1, true>), dim3((N + 15) / 16, 1), dim3(256), K * 2, stream,
-                       xs, w, s, ys, M, N, K, G, rb, cols);
-  else if (M <= 16)
-    hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 1>), dim3((N + 15) / 16, 1), dim3(256), 0, stream,
-                       xs, w, s, ys, M, N, K, G, rb, cols);
-  else if (M <= 32)
-    hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 2>), dim3((N + 15) / 16, 1), dim3(256), 0, stream,
-                       xs, w, s, ys, M, N, K, G, rb, cols);
   else
     hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 4>), dim3((N + 15) / 16, (M + 63) / 64), dim3(256),
                        0, stream, xs, w, s, ys, M, N, K, G, rb, cols);
@@ -780,14 +607,22 @@ LNQ_API LnqStatus lnq_w8a16(const void* x, const uint8_t* weight, const float* s
   const int rb = group == 0 ? 1 : (int)row_block;
   const int cols = group == 0 ? 1 : (int)(in_features / group);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // Several rows, and one where the row kernels do not take it, on the streaming product (a
+  // decode batch of 8 at 8192 -> 28672 FP8 69 us on the skinny kernel, 24 rows at 4096 ->
+  // 14336 int8 in groups 46: it reads all of x for each 16 outputs).
+  // One row at K = 4096 over a narrow output keeps the row kernel, which loads a wave's
+  // whole share at once (N = 4096 int8 5.9 against 6.4 us, N = 6144 FP8 7.9 against 7.1).
+  const bool row_kernel = M == 1 && K == 4096 && N <= 4096 && G % 128 == 0;
+  if (!row_kernel && K <= stream::MAX_K)
+    return (fp8 ? launch_fp8_stream : launch_int8_stream)(x, weight, scale, y, M, N, K, (int)group, rb, dtype, s);
   if (dtype == LNQ_BF16) {
-    if (fp8) launch_w8_skinny<LNQ_BF16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
-    else launch_w8_skinny<LNQ_BF16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    if (fp8) launch_w8_few<LNQ_BF16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    else launch_w8_few<LNQ_BF16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
   } else {
-    if (fp8) launch_w8_skinny<LNQ_F16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
-    else launch_w8_skinny<LNQ_F16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    if (fp8) launch_w8_few<LNQ_F16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    else launch_w8_few<LNQ_F16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
   }
-  return launched("w8_skinny");
+  return launched("w8_few");
 }
 
 LNQ_API LnqStatus lnq_dequantize8(const uint8_t* weight, const float* scale, void* out,

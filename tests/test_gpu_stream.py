@@ -71,3 +71,32 @@ def test_int4(rows: int, out: int, width: int, group: int, dtype: torch.dtype) -
     s, z = scale.double().numpy()[..., None], zero.double().numpy()[..., None]
     offset = 128.0 if dtype == BF16 else 1024.0
     _check(got, x, ((q - z) * s).reshape(out, width), ((q + z + 2 * offset) * s).reshape(out, width), bias)
+
+
+@pytest.mark.parametrize("fp8", [True, False])
+@pytest.mark.parametrize(("rows", "out", "width", "group", "row_block", "dtype"), [
+    (1, 72, 640, 0, 1, BF16),  # one row, a scale a row, 5 steps
+    (3, 5000, 4096, 0, 1, F16),
+    (8, 100, 2176, 64, 1, BF16),  # two groups a step
+    (16, 264, 1280, 128, 1, F16),
+    (31, 48, 3840, 384, 1, BF16),  # a group of three steps
+    (33, 60, 1152, 192, 5, F16),  # groups of 1.5 steps, a scale row for 5 weight rows
+    (64, 1024, 1024, 128, 128, BF16),  # block scales
+])
+def test_eight_bit(fp8: bool, rows: int, out: int, width: int, group: int, row_block: int, dtype: torch.dtype) -> None:
+    print(f"w8 stream fp8={fp8} rows={rows} out={out} in={width} group={group}/{row_block} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(out + width)
+    if fp8:
+        weight = (torch.randn(out, width, generator=g) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+        w = weight.float().double().numpy()
+    else:
+        weight = torch.randint(-128, 128, (out, width), generator=g, dtype=torch.int8)
+        w = weight.double().numpy()
+    shape = (out // row_block, width // group) if group else (out,)
+    scale = torch.rand(shape, generator=g) * 0.01 + 0.001
+    s = scale.double().numpy()
+    s = np.repeat(np.repeat(s, row_block, 0), group, 1) if group else s[:, None]
+    x = _x(rows, width, dtype)
+    got = kernels.w8a16(x.to(DEV), weight.to(DEV), scale.to(DEV), fp8, group, row_block)
+    carried = np.abs(w) + (256.0 if not fp8 and dtype == BF16 else 0.0)
+    _check(got, x, w * s, carried * s)
