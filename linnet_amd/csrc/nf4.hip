@@ -33,7 +33,7 @@
 // sums (ROWS x rows of x) go through LDS, [output][lane] with the lanes
 // contiguous, and 256 / (ROWS * MR) lanes add each output's 256 partial sums in
 // a fixed order.
-#include "common.hpp"
+#include "stream.hpp"
 
 namespace lnq {
 
@@ -61,10 +61,7 @@ __constant__ float kNf4Values[16] = {
 
 // The values' 16-bit patterns in x's type as byte planes: byte c of lo[] (c = 4
 // * dword + byte) is the low byte of value c, hi[] the high bytes.
-struct Nf4Planes {
-  uint32_t lo[4];
-  uint32_t hi[4];
-};
+using Nf4Planes = stream::Planes;
 
 // ---------------------------------------------------------------- dequantize
 // Thread i widens UNIT_BYTES bytes (2 * UNIT_BYTES inputs) of the weight,
@@ -322,6 +319,25 @@ Nf4Planes planes_for(int dtype) {
   return p;
 }
 
+// Whether the streaming product (stream.hpp) takes the call: past 4 rows (2 where In > 4096
+// gives the GEMV's lanes several units; 4096 -> 14336, block 64: 4 rows 14.0 us on the GEMV
+// against 14.9, 5 rows 20.9 against 14.1, 16 rows 42.9 against 15.4; 14336 -> 4096: 2 rows
+// 13.9 against 14.1, 4 rows 19.1 against 14.5), blocks its
+// steps hold whole (32, 64 or 128 k inputs), 32 rows of x below 1 GiB.
+bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride,
+                  int64_t y_stride) {
+  return rows > (in_features <= nf4::UNIT * nf4::THREADS ? 4 : 2) && rows <= INT32_MAX && (block == 32 || block == 64 || block % 128 == 0) &&
+         in_features <= stream::MAX_K && x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
+}
+
+template <int DT>
+void launch_stream(stream::Args& a, int block, hipStream_t s) {
+  a.span = block % 128 == 0 ? block / 128 : 1;
+  if (block == 32) stream::launch<DT, stream::NF4, 4>(a, s);
+  else if (block == 64) stream::launch<DT, stream::NF4, 2>(a, s);
+  else stream::launch<DT, stream::NF4, 1, stream::SPAN>(a, s);
+}
+
 }  // namespace
 
 }  // namespace lnq
@@ -403,6 +419,26 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
   const int slots = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
   const Nf4Planes planes = planes_for(dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (stream_takes(rows, out_features, in_features, block, x_stride, y_stride)) {
+    stream::Args a{};
+    a.x = static_cast<const uint16_t*>(x);
+    a.w = codes;
+    a.scale = absmax;
+    a.bias = static_cast<const uint16_t*>(bias);
+    a.y = static_cast<uint16_t*>(y);
+    a.x_stride = static_cast<int>(x_stride);
+    a.y_stride = static_cast<int>(y_stride);
+    a.row_bytes = static_cast<int>(in_features / 2);
+    a.M = static_cast<int>(rows);
+    a.N = static_cast<int>(out_features);
+    a.K = static_cast<int>(in_features);
+    a.cols = static_cast<int>(in_features / block);
+    a.row_block = 1;
+    a.planes = planes;
+    if (dtype == LNQ_BF16) launch_stream<LNQ_BF16>(a, static_cast<int>(block), s);
+    else launch_stream<LNQ_F16>(a, static_cast<int>(block), s);
+    return launched("nf4_stream");
+  }
   const int O = static_cast<int>(out_features), K = static_cast<int>(in_features), B = static_cast<int>(block);
   // Up to 8 rows of x a launch (4 past In = 8192); more rows take more launches
   // over the same weight.

@@ -820,6 +820,21 @@ def nf4_gemv_fits(rows: int, in_features: int, block: int, dtype: torch.dtype) -
             and 0 < in_features <= NF4_GEMV_MAX_IN)
 
 
+# Rows up to which `nf4_linear` reads the stored weight at all: past NF4_GEMV_ROWS on the
+# streaming kernel, 32 rows a pass.
+NF4_STREAM_ROWS = 96
+NF4_STREAM_MAX_IN = 65536
+
+
+def _nf4_reads_stored(rows: int, in_features: int, block: int, dtype: torch.dtype) -> bool:
+    """Whether `nf4_linear` multiplies by the stored weight (`lnq_nf4_linear`) rather than
+    the widened one."""
+    if nf4_gemv_fits(rows, in_features, block, dtype):
+        return True
+    return (dtype in _HALF and rows <= NF4_STREAM_ROWS and (block in (32, 64) or block % 128 == 0)
+            and in_features % block == 0 and 0 < in_features <= NF4_STREAM_MAX_IN)
+
+
 def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: int,
              bias: torch.Tensor | None = None) -> torch.Tensor:
     """x [..., In] (bf16 / f16) times the NF4 weight's transpose (+ bias), the
@@ -854,7 +869,7 @@ def nf4_linear(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block
     _on_gpu("nf4_linear", x, codes, absmax, bias)
     out_features, in_features = _nf4_operands("nf4_linear", codes, absmax, block)
     rows = x.numel() // max(in_features, 1) if x.dim() else 0
-    if nf4_gemv_fits(rows, in_features, block, x.dtype):
+    if _nf4_reads_stored(rows, in_features, block, x.dtype):
         return nf4_gemv(x, codes, absmax, block, bias)
     weight = nf4_dequantize(codes, absmax, block, x.dtype)
     return torch.nn.functional.linear(x, weight, bias)

@@ -100,3 +100,26 @@ def test_eight_bit(fp8: bool, rows: int, out: int, width: int, group: int, row_b
     got = kernels.w8a16(x.to(DEV), weight.to(DEV), scale.to(DEV), fp8, group, row_block)
     carried = np.abs(w) + (256.0 if not fp8 and dtype == BF16 else 0.0)
     _check(got, x, w * s, carried * s)
+
+
+@pytest.mark.parametrize(("rows", "out", "width", "block", "dtype"), [
+    (3, 40, 8256, 64, BF16),  # In ends inside a step
+    (5, 300, 1088, 64, F16),
+    (9, 2050, 4096, 32, BF16),
+    (17, 130, 1024, 128, F16),
+    (24, 72, 14336, 64, BF16),
+    (96, 1000, 1536, 512, BF16),
+])
+def test_nf4(rows: int, out: int, width: int, block: int, dtype: torch.dtype) -> None:
+    print(f"nf4 stream rows={rows} out={out} in={width} block={block} {dtype}", flush=True)
+    rng = np.random.default_rng(out + width)
+    codes = rng.integers(0, 256, (out, width // 2)).astype(np.uint8)
+    absmax = (rng.random((out, width // block)) * 0.1 + 0.01).astype(np.float32)
+    x = _x(rows, width, dtype)
+    bias = _x(1, out, dtype)[0] if rows % 2 else None
+    got = kernels.nf4_linear(x.to(DEV), torch.from_numpy(codes).to(DEV), torch.from_numpy(absmax).to(DEV), block,
+                             None if bias is None else bias.to(DEV))
+    # The codes' values as the kernel holds them, rounded to x's type.
+    values = torch.from_numpy(quant.NF4_VALUES.copy()).to(dtype).double().numpy()
+    w = values[np.stack([codes & 15, codes >> 4], axis=-1).reshape(out, width)] * np.repeat(absmax.astype(np.float64), block, 1)
+    _check(got, x, w, np.abs(w), bias)
