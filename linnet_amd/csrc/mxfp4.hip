@@ -19,7 +19,9 @@
 // (buffer loads: rows past Out, blocks past G and the rows of an out-of-range
 // expert read zeros through the range check). A row's sum is the lanes' partial
 // sums added across the wave (fixed order).
-#include "common.hpp"
+#include <cmath>
+
+#include "stream.hpp"
 
 namespace lnq {
 
@@ -135,6 +137,98 @@ __global__ __launch_bounds__(64 * mx::WAVES) void mxfp4_experts_kernel(
   }
 }
 
+// Many pairs: the pairs of one expert together, so that its weights are read and widened
+// once for all of them (the kernel above reads an expert's bytes again for each of its
+// pairs: 32 tokens, top 4 of 32 experts, 2880 -> 5760 took 213 us, four times the bytes'
+// time). Workgroup (n block, expert): the pairs that chose the expert, in order, are
+// listed in LDS, then the streaming product (stream.hpp) runs over them 4 XI (16 MT) at a
+// time, x rows gathered and output rows scattered by pair. One expert more lists the pairs
+// whose choice is out of range and clears their rows.
+namespace mx {
+constexpr int MAX_PAIRS = 2048;  // pairs of a launch (the list's LDS)
+constexpr int GROUP_WAVES = 4;
+}
+
+struct ExpertArgs {
+  stream::Args a;  // w, scale: every expert's; M unused
+  const int64_t* experts;
+  int num_experts, pairs, chosen, x_row_stride, x_slot_stride;
+  uint32_t x_bytes;
+};
+
+template <int DT, int MT, int XI>
+__global__ __launch_bounds__(64 * mx::GROUP_WAVES, MT == 1 ? 4 : 2) void mxfp4_grouped_kernel(ExpertArgs g) {
+  using E = Elem<DT>;
+  constexpr int NT = 4, THREADS = 64 * mx::GROUP_WAVES;
+  LNQ_STREAM_STAGES(mx::GROUP_WAVES, XI, MT, NT);
+  __shared__ uint16_t list[mx::MAX_PAIRS];
+  __shared__ int found[mx::GROUP_WAVES];
+  extern __shared__ __attribute__((aligned(16))) uint8_t SC[];
+  const int e = blockIdx.y;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int count = 0;
+  for (int p0 = 0; p0 < g.pairs; p0 += THREADS) {
+    const int p = p0 + threadIdx.x;
+    const int64_t id = p < g.pairs ? g.experts[p] : -1;
+    const bool known = id >= 0 && id < g.num_experts;
+    const bool mine = p < g.pairs && (known ? id == e : e == g.num_experts);
+    const uint64_t mask = __ballot(mine);
+    if (lane == 0) found[wave] = __popcll(mask);
+    __syncthreads();
+    int at = count;
+#pragma unroll
+    for (int w = 0; w < mx::GROUP_WAVES; ++w) {
+      if (w < wave) at += found[w];
+      count += found[w];
+    }
+    if (mine) list[at + __popcll(mask & ((uint64_t{1} << lane) - 1))] = static_cast<uint16_t>(p);
+    __syncthreads();
+  }
+  if (count == 0) return;
+  stream::Args a = g.a;
+  a.w += static_cast<int64_t>(e) * a.N * a.row_bytes;
+  a.scale = static_cast<const uint8_t*>(a.scale) + static_cast<int64_t>(e) * a.N * a.cols;
+  const int n0 = blockIdx.x * a.R, n_end = min(a.N, n0 + a.R);
+  if (e == g.num_experts) {
+    const int width = n_end - n0;
+    for (int i = threadIdx.x; i < count * width; i += THREADS)
+      a.y[static_cast<int64_t>(list[i / width]) * a.N + n0 + i % width] = 0;
+    return;
+  }
+  constexpr int ROWS = MT == 1 ? 4 * XI : 16 * MT;
+  for (int m0 = 0; m0 < count; m0 += ROWS) {
+    const int live = min(count - m0, ROWS);
+    stream::product<mx::GROUP_WAVES, DT, stream::FP4, 4, MT, XI, NT, stream::ONE_STEP>(
+        a, n0, n_end, a.x, g.x_bytes, X0, X1, X2, X3, SC,
+        [&](int i) -> int {
+          if (i >= live) return -1;
+          const int p = list[m0 + i], r = p / g.chosen;
+          return r * g.x_row_stride + (p - r * g.chosen) * g.x_slot_stride;
+        },
+        [&](int m, int n, float v) {
+          if (m < live) a.y[static_cast<int64_t>(list[m0 + m]) * a.N + n] = E::from_f32(v);
+        });
+    __syncthreads();  // the stages and scales are read before the next rows' loads
+  }
+}
+
+template <int DT, int MT, int XI>
+static void launch_grouped(const ExpertArgs& g, hipStream_t stream) {
+  const int lds = stream::scale_lds(stream::FP4, false, false, g.a.R, g.a.cols, 1);
+  hipLaunchKernelGGL((mxfp4_grouped_kernel<DT, MT, XI>),
+                     dim3(static_cast<unsigned>((g.a.N + g.a.R - 1) / g.a.R), static_cast<unsigned>(g.num_experts + 1)),
+                     dim3(64 * mx::GROUP_WAVES), static_cast<size_t>(lds), stream, g);
+}
+
+template <int DT>
+static void launch_grouped_dt(const ExpertArgs& g, hipStream_t stream) {
+  // Rows of x a pass by the pairs an expert has on average.
+  if (g.pairs <= g.num_experts) launch_grouped<DT, 1, 1>(g, stream);
+  else if (g.pairs <= 3 * g.num_experts) launch_grouped<DT, 1, 2>(g, stream);
+  else if (g.pairs <= 12 * g.num_experts) launch_grouped<DT, 1, 4>(g, stream);
+  else launch_grouped<DT, 2, 8>(g, stream);
+}
+
 }  // namespace lnq
 
 using namespace lnq;
@@ -161,13 +255,55 @@ LNQ_API LnqStatus lnq_mxfp4_experts(const void* x, int64_t x_row_stride, int64_t
   LNQ_REQUIRE(aligned(x, 16) && aligned(blocks, 16) && x_row_stride % 8 == 0 && x_slot_stride % 8 == 0,
               "lnq_mxfp4_experts: x (with its row and slot strides) and blocks must be 16-byte aligned");
   const int groups = static_cast<int>(in_features / 32);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const auto* xs = static_cast<const uint16_t*>(x);
+  auto* ys = static_cast<uint16_t*>(y);
+  const int64_t pairs = rows * chosen;
+  // The grouped kernel costs about 4 us more than this one for what it reads once (the
+  // list, its barriers), so it is taken where it saves 16 MB of weights read again: the
+  // pairs past the experts that evenly spread choices would name (2880 -> 5760, 32
+  // experts, top 4: 6 tokens 45.2 against 48.6 us, 8 53.8 / 61.9, 16 66.8 / 113, 32 79 /
+  // 214, 64 93 / 409; 1056 -> 1501, 8 experts, top 2: 8 tokens 8.1 / 7.1, 16 8.6 / 11.4).
+  // x as the range-checked buffers need it: below 1 GiB, rows and slots forward.
+  const int64_t x_span = (rows - 1) * x_row_stride + (chosen - 1) * x_slot_stride + in_features;
+  const double named = static_cast<double>(num_experts) * (1.0 - std::pow(1.0 - 1.0 / static_cast<double>(num_experts), static_cast<double>(pairs)));
+  const double again = (static_cast<double>(pairs) - named) * static_cast<double>(out_features * groups * 17);
+  if (in_features >= 32 && again > 16e6 && x_row_stride >= 0 && x_slot_stride >= 0 &&
+      x_span < (int64_t{1} << 29) && num_experts < 65535 && out_features <= (1 << 24) &&
+      chosen <= mx::MAX_PAIRS) {
+    ExpertArgs g{};
+    g.a.w = blocks;
+    g.a.scale = scales;
+    g.a.row_bytes = groups * 16;
+    g.a.N = static_cast<int>(out_features);
+    g.a.K = static_cast<int>(in_features);
+    g.a.R = stream::MAX_R;
+    g.a.span = 1;
+    g.a.cols = groups;
+    g.a.row_block = 1;
+    g.num_experts = static_cast<int>(num_experts);
+    g.chosen = static_cast<int>(chosen);
+    g.x_row_stride = static_cast<int>(x_row_stride);
+    g.x_slot_stride = static_cast<int>(x_slot_stride);
+    const int64_t part = mx::MAX_PAIRS / chosen;
+    for (int64_t r0 = 0; r0 < rows; r0 += part) {
+      const int64_t rc = rows - r0 < part ? rows - r0 : part;
+      g.a.x = xs + r0 * x_row_stride;
+      g.x_bytes = static_cast<uint32_t>(((rc - 1) * x_row_stride + (chosen - 1) * x_slot_stride + in_features) * 2);
+      g.a.y = ys + r0 * chosen * out_features;
+      g.experts = experts + r0 * chosen;
+      g.pairs = static_cast<int>(rc * chosen);
+      if (dtype == LNQ_BF16) launch_grouped_dt<LNQ_BF16>(g, s);
+      else launch_grouped_dt<LNQ_F16>(g, s);
+      const LnqStatus st = launched("mxfp4_grouped");
+      if (st != LNQ_OK) return st;
+    }
+    return LNQ_OK;
+  }
   const int slots = (groups + 63) / 64;
   const int per_wg = mx::WAVES * mx::ROWS;
   const dim3 grid(static_cast<unsigned>(rows * chosen), static_cast<unsigned>((out_features + per_wg - 1) / per_wg));
   LNQ_REQUIRE(grid.y <= 65535, "lnq_mxfp4_experts: too many output features");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const auto* xs = static_cast<const uint16_t*>(x);
-  auto* ys = static_cast<uint16_t*>(y);
   const int C = static_cast<int>(chosen), NE = static_cast<int>(num_experts), O = static_cast<int>(out_features);
 #define LNQ_MX(DT, S)                                                                                                 \
   hipLaunchKernelGGL((mxfp4_experts_kernel<DT, S>), grid, dim3(64 * mx::WAVES), 0, s, xs, x_row_stride, x_slot_stride, \

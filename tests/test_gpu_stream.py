@@ -123,3 +123,63 @@ def test_nf4(rows: int, out: int, width: int, block: int, dtype: torch.dtype) ->
     values = torch.from_numpy(quant.NF4_VALUES.copy()).to(dtype).double().numpy()
     w = values[np.stack([codes & 15, codes >> 4], axis=-1).reshape(out, width)] * np.repeat(absmax.astype(np.float64), block, 1)
     _check(got, x, w, np.abs(w), bias)
+
+
+@pytest.mark.parametrize("dtype", [BF16, F16])
+@pytest.mark.parametrize(("rows", "chosen", "count", "out", "width", "skew"), [
+    (40, 4, 8, 1500, 2880, False),  # In ends inside a step; 20 pairs an expert on average
+    (24, 2, 4, 3000, 1056, True),  # one expert takes most pairs (several passes), some are out of range
+    (600, 4, 2, 70, 256, False),  # more pairs than a launch lists
+    (16, 4, 16, 2048, 2048, False),  # 4 pairs an expert: the 8-row form
+])
+def test_mxfp4_grouped(dtype: torch.dtype, rows: int, chosen: int, count: int, out: int, width: int, skew: bool) -> None:
+    print(f"mxfp4 grouped rows={rows} chosen={chosen} E={count} out={out} in={width} {dtype}", flush=True)
+    rng = np.random.default_rng(out + width)
+    blocks = rng.integers(0, 256, (count, out, width // 32, 16)).astype(np.uint8)
+    scales = rng.integers(118, 136, (count, out, width // 32)).astype(np.uint8)
+    experts = rng.integers(0, count, (rows, chosen)).astype(np.int64)
+    if skew:
+        experts[rng.random((rows, chosen)) < 0.8] = 1
+        experts[0, 0], experts[3, 1] = -1, count
+    x = torch.randn(rows, width, generator=torch.Generator().manual_seed(rows)).to(dtype)
+    xs = x.to(DEV)[:, None].expand(rows, chosen, width)
+    args = [torch.from_numpy(t).to(DEV) for t in (blocks, scales, experts)]
+    got = kernels.mxfp4_experts(xs, *args).cpu()
+    for r, k in ((0, 0), (3, 1), (rows // 2, 0), (rows - 1, chosen - 1)):
+        e = int(experts[r, k])
+        if not 0 <= e < count:
+            assert not got[r, k].any()
+            continue
+        w = quant.dequantize_mxfp4(blocks[e], scales[e]).astype(np.float64)
+        _check(got[r, k][None], x[r][None], w, np.abs(w))
+    # Every pair against the pair kernel's answer for its row alone (one row's pairs stay on it).
+    for r in range(0, rows, max(1, rows // 12)):
+        alone = kernels.mxfp4_experts(xs[r:r + 1], args[0], args[1], args[2][r:r + 1]).cpu()[0].double()
+        top = alone.abs().amax().item()
+        assert (got[r].double() - alone).abs().max().item() <= 2 * ULP[dtype] * top
+
+
+def test_replayed_from_a_graph() -> None:
+    """A captured call of each format replays to the eager bits with work between."""
+    x = _x(12, 1024, BF16).to(DEV)
+    g = torch.Generator().manual_seed(0)
+    w8 = torch.randint(-128, 128, (512, 1024), generator=g, dtype=torch.int8).to(DEV)
+    s8 = (torch.rand(512, 8, generator=g) * 0.01).to(DEV)
+    codes = torch.randint(0, 256, (512, 512), generator=g, dtype=torch.uint8).to(DEV)
+    absmax = torch.rand(512, 16, generator=g).to(DEV)
+    packed = codes.view(512, 16, 32)
+    scale, zero = torch.rand(512, 16, generator=g).to(BF16).to(DEV), torch.randint(0, 16, (512, 16), generator=g, dtype=torch.uint8).to(DEV)
+    calls = [lambda: kernels.w8a16(x, w8, s8, False, 128), lambda: kernels.nf4_linear(x, codes, absmax, 64),
+             lambda: kernels.int4_linear(x, packed, scale, zero)]
+    want = [c().clone() for c in calls]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = [c() for c in calls]
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+        torch.randn(1 << 20, device=DEV).sum().item()
