@@ -79,6 +79,8 @@ SIGNATURES: dict[str, list[object]] = {
 }
 
 _lock = threading.Lock()
+# The loaded library's entry points by name (cleared when another library is loaded).
+_entries: dict[str, object] = {}
 _lib: ctypes.CDLL | None = None
 
 
@@ -112,6 +114,7 @@ def load() -> ctypes.CDLL:
             function = getattr(lib, name)
             function.restype = ctypes.c_int32
             function.argtypes = argtypes
+        _entries.clear()
         _lib = lib
         return lib
 
@@ -122,7 +125,11 @@ def last_error() -> str:
 
 def call(name: str, *args: object) -> None:
     """Calls entry point `name`; raises LinnetError with the library's message on failure."""
-    status = getattr(load(), name)(*args)
+    entry = _entries.get(name)
+    if entry is None or _lib is None:
+        entry = getattr(load(), name)
+        _entries[name] = entry
+    status = entry(*args)
     if status != LNQ_OK:
         kind = "unavailable" if status == LNQ_UNAVAILABLE else "failed"
         raise LinnetError(f"{name} {kind}: {last_error()}")

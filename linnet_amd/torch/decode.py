@@ -11,7 +11,7 @@ import torch
 
 from .. import _lib
 from ..errors import LinnetError
-from .kernels import SplitParts, XTiles, _on_gpu, _ptr, _stream
+from .kernels import SplitParts, XTiles, _on, _on_gpu, _ptr, _stream
 
 
 def _bf16(what: str, *tensors: torch.Tensor) -> None:
@@ -43,18 +43,18 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-5, delta: tor
         if parts.data.dim() != 3 or tuple(parts.data.shape[1:]) != (rows, x.shape[-1]) or not parts.data.is_contiguous():
             raise LinnetError("rmsnorm: split parts are a contiguous f32 [splits, rows, hidden]")
         out = XTiles.empty(rows, x.shape[-1], x.dtype, device) if tiles else torch.empty_like(x)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_rmsnorm_parts", _ptr(x), _ptr(parts.data), parts.data.shape[0], _ptr(weight),
                       _ptr(out.data if tiles else out), int(tiles), rows, x.shape[-1], float(eps), _stream(device))
         return out
     if tiles:
         xt = XTiles.empty(rows, x.shape[-1], x.dtype, device)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_rmsnorm_tiles", _ptr(x), _ptr(delta), _ptr(weight), _ptr(xt.data), rows, x.shape[-1],
                       float(eps), _stream(device))
         return xt
     h = torch.empty_like(x)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_rmsnorm", _ptr(x), _ptr(delta), _ptr(weight), _ptr(h), rows, x.shape[-1],
                   float(eps), _stream(device))
     return h
@@ -90,7 +90,7 @@ def prefill_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: torch.T
     q_out = torch.empty(1, heads, prompt, hd, dtype=q.dtype, device=device)
     k_out = torch.empty(1, kvh, prompt, hd, dtype=q.dtype, device=device)
     v_out = torch.empty(1, kvh, prompt, hd, dtype=q.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_prefill_rope", _ptr(q), _ptr(k), _ptr(v), stride, _ptr(cos), _ptr(sin), _ptr(q_out),
                   _ptr(k_out), _ptr(v_out), _ptr(kt_cache), _ptr(v_cache), prompt, heads, kvh, hd, cap, _stream(device))
     return q_out, k_out, v_out
@@ -146,13 +146,13 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
         work = torch.empty(max(floats, 1), dtype=torch.float32, device=device)
         if tiles:
             xt = XTiles.empty(rows, heads * hd, q.dtype, device)
-            with torch.cuda.device(device):
+            with _on(device):
                 _lib.call("lnq_decode_attention_tiles", _ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin),
                           _ptr(kt_cache), _ptr(v_cache), _ptr(xt.data), _ptr(work), work.numel(), rows, heads, kvh,
                           hd, cap, 0, _ptr(pos), q.stride(0), k.stride(0), _stream(device))
             return xt
         out = torch.empty_like(q)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_decode_attention_at", _ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(kt_cache),
                       _ptr(v_cache), _ptr(out), _ptr(work), work.numel(), rows, heads, kvh, hd, cap, _ptr(pos),
                       q.stride(0), k.stride(0), _stream(device))
@@ -163,13 +163,13 @@ def decode_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cos: tor
     work = torch.empty(max(floats, 1), dtype=torch.float32, device=device)
     if tiles:
         xt = XTiles.empty(rows, heads * hd, q.dtype, device)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_decode_attention_tiles", _ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(kt_cache),
                       _ptr(v_cache), _ptr(xt.data), _ptr(work), work.numel(), rows, heads, kvh, hd, cap, pos, None,
                       q.stride(0), k.stride(0), _stream(device))
         return xt
     out = torch.empty_like(q)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_decode_attention", _ptr(q), _ptr(k), _ptr(v), _ptr(cos), _ptr(sin), _ptr(kt_cache),
                   _ptr(v_cache), _ptr(out), _ptr(work), work.numel(), rows, heads, kvh, hd, cap, pos, q.stride(0),
                   k.stride(0), _stream(device))
@@ -190,20 +190,20 @@ def silu_mul(g: torch.Tensor, u: torch.Tensor, tiles: bool = False) -> torch.Ten
         if g.dim() != 2 or g.stride(1) != 1 or u.stride(1) != 1:
             g, u = g.contiguous(), u.contiguous()
         xt = XTiles.empty(g.shape[0], g.shape[1], g.dtype, device)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_silu_mul_tiles", _ptr(g), _ptr(u), _ptr(xt.data), g.shape[0], g.shape[1], g.stride(0),
                       u.stride(0), _stream(device))
         return xt
     if g.is_contiguous() and u.is_contiguous():
         a = torch.empty_like(g)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call("lnq_silu_mul", _ptr(g), _ptr(u), _ptr(a), g.numel(), _stream(device))
         return a
     if g.dim() != 2 or g.stride(1) != 1 or u.stride(1) != 1:
         g, u = g.contiguous(), u.contiguous()
     rows, width = g.shape
     a = torch.empty(rows, width, dtype=g.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_silu_mul_rows", _ptr(g), _ptr(u), _ptr(a), rows, width, g.stride(0), u.stride(0),
                   _stream(device))
     return a

@@ -70,11 +70,13 @@ def _int4_linear(
     With the fused 3-tuple, any number of rows runs one HIP kernel (few rows the
     skinny MFMA kernel, many the tiled dequant-GEMM) with the bias added in its
     epilogue; with the 1-tuple, `F.linear` over the dequantized weight."""
-    flat = x.reshape(-1, x.shape[-1])
     if len(packed) == 3 and x.dtype == scale.dtype:
         p, s, z = packed
-        y = kernels.int4_linear(flat, p, s, z, bias)
+        if x.dim() == 2:
+            return kernels.int4_linear(x, p, s, z, bias)
+        y = kernels.int4_linear(x.reshape(-1, x.shape[-1]), p, s, z, bias)
         return y.reshape(*x.shape[:-1], y.shape[-1])
+    flat = x.reshape(-1, x.shape[-1])
     if not x.is_cuda:
         raise LinnetError("_int4_linear: linnet_amd runs on the GPU; x is on " + str(x.device))
     weight = packed[0] if len(packed) == 1 else kernels.int4_weight(raw, scale, zero)

@@ -34,27 +34,51 @@ KERNELS = {
 _KERNEL_NAMES = {code: name for name, code in KERNELS.items()}
 
 
-def _ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+# A call's host time is longer than a small kernel's (a 4096 x 4096 layer at one token: 4.3
+# us on the GPU, 12.5 us from call to call with torch.cuda.device, current_stream and a
+# ctypes object a pointer), so these are the direct forms: plain integers, and the device
+# guard only where the call's device is not the current one.
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _ptr(t: torch.Tensor | None) -> int | None:
+    return None if t is None else t.data_ptr()
+
+
+def _stream(device: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _Here:
+    """The device guard of a call on the current device."""
+
+    def __enter__(self) -> None:
+        return None
+
+    def __exit__(self, *exc: object) -> None:
+        return None
+
+
+_HERE = _Here()
+
+
+def _on(device: torch.device) -> _Here | torch.cuda.device:
+    return _HERE if device.index == torch._C._cuda_getDevice() else torch.cuda.device(device)
 
 
 def _on_gpu(what: str, *tensors: torch.Tensor | None) -> torch.device:
-    device: torch.device | None = None
+    first: torch.Tensor | None = None
+    index = -1
     for t in tensors:
         if t is None:
             continue
         if not t.is_cuda:
             raise LinnetError(f"{what}: the HIP kernels take GPU tensors, got one on {t.device}")
-        if device is None:
-            device = t.device
-        elif t.device != device:
-            raise LinnetError(f"{what}: tensors on {device} and {t.device}")
-    assert device is not None
-    return device
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise LinnetError(f"{what}: tensors on {first.device} and {t.device}")
+    assert first is not None
+    return first.device
 
 
 def _code(dtype: torch.dtype, what: str, allowed: tuple[torch.dtype, ...] = _HALF) -> int:
@@ -103,12 +127,12 @@ def int4_linear(
         raise LinnetError(f"int4_linear: packed {tuple(packed.shape)} does not hold In={depth}")
     if packed.dtype != torch.uint8 or zero.dtype != torch.uint8:
         raise LinnetError("int4_linear: packed and zero are uint8")
-    if tuple(scale.shape) != (width, groups) or tuple(zero.shape) != (width, groups):
+    if scale.shape != (width, groups) or zero.shape != (width, groups):
         raise LinnetError(f"int4_linear: scale and zero are [{width}, {groups}]")
     code = _code(x.dtype, "int4_linear")
     if scale.dtype != x.dtype or (bias is not None and bias.dtype != x.dtype):
         raise LinnetError("int4_linear: scale and bias have x's dtype")
-    if bias is not None and tuple(bias.shape) != (width,):
+    if bias is not None and bias.shape != (width,):
         raise LinnetError(f"int4_linear: bias is [{width}]")
     if kernel not in KERNELS:
         raise LinnetError(f"int4_linear: kernel is one of {', '.join(KERNELS)}")
@@ -118,21 +142,21 @@ def int4_linear(
     if out is None:
         y = torch.empty(rows, width, dtype=x.dtype, device=device)
     else:
-        if tuple(out.shape) != (rows, width) or out.dtype != x.dtype or out.device != device or not out.is_contiguous():
+        if out.shape != (rows, width) or out.dtype != x.dtype or out.device != device or not out.is_contiguous():
             raise LinnetError(f"int4_linear: out is a contiguous [{rows}, {width}] {x.dtype} tensor on {device}")
         y = out
     if order is not None:
-        if order.dtype != torch.int32 or tuple(order.shape) != (depth,):
+        if order.dtype != torch.int32 or order.shape != (depth,):
             raise LinnetError(f"int4_linear: order is [{depth}] int32")
         order = order.contiguous()
         taken = torch.empty_like(x)
-        with torch.cuda.device(device):
+        with _on(device):
             _lib.call(
                 "lnq_int4_linear_ordered", _ptr(x), _ptr(order), _ptr(packed), _ptr(scale), _ptr(zero), _ptr(bias),
                 _ptr(y), _ptr(taken), rows, depth, width, group, code, KERNELS[kernel], _stream(device),
             )
         return y
-    with torch.cuda.device(device):
+    with _on(device):
         _, need = _workspace(rows, depth, width, group, code, KERNELS[kernel])
         if need:
             # The split GEMV's partial sums: memory of torch's caching allocator
@@ -189,7 +213,7 @@ def x_tiles(x: torch.Tensor) -> XTiles:
         raise LinnetError("x_tiles: x is a [rows, width] tensor of a 16-bit type")
     x = x.contiguous()
     xt = XTiles.empty(x.shape[0], x.shape[1], x.dtype, device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_x_tiles", _ptr(x), _ptr(xt.data), x.shape[0], x.shape[1], _stream(device))
     return xt
 
@@ -217,10 +241,10 @@ def int4_linear_tiles(xt: XTiles, packed: torch.Tensor, scale: torch.Tensor, zer
     if out is None:
         y = torch.empty(rows, width, dtype=xt.dtype, device=device)
     else:
-        if tuple(out.shape) != (rows, width) or out.dtype != xt.dtype or out.device != device or not out.is_contiguous():
+        if out.shape != (rows, width) or out.dtype != xt.dtype or out.device != device or not out.is_contiguous():
             raise LinnetError(f"int4_linear_tiles: out is a contiguous [{rows}, {width}] {xt.dtype} tensor on {device}")
         y = out
-    with torch.cuda.device(device):
+    with _on(device):
         need = 0
         if kernel == "split" or depth > 4096:
             _, need = _workspace(rows, depth, width, group, code, _lib.KERNEL_SPLIT)
@@ -262,7 +286,7 @@ def int4_linear_tiles_parts(xt: XTiles, packed: torch.Tensor, scale: torch.Tenso
     if scale.dtype != xt.dtype:
         raise LinnetError("int4_linear_tiles_parts: scale has x's dtype")
     packed, scale, zero = packed.contiguous(), scale.contiguous(), zero.contiguous()
-    with torch.cuda.device(device):
+    with _on(device):
         _, need = _workspace(rows, depth, width, group, code, _lib.KERNEL_SPLIT)
         parts = torch.empty(max(need, 16) // 4, dtype=torch.float32, device=device)
         splits = ctypes.c_int32(0)
@@ -290,16 +314,16 @@ def _prologue_linear(what: str, prologue: int, x: torch.Tensor, operand: torch.T
     width, groups, half = packed.shape
     if groups * 2 * half != depth or packed.dtype != torch.uint8 or zero.dtype != torch.uint8:
         raise LinnetError(f"{what}: packed {tuple(packed.shape)} (uint8) does not hold In={depth}")
-    if scale.dtype != torch.bfloat16 or tuple(scale.shape) != (width, groups) or tuple(zero.shape) != (width, groups):
+    if scale.dtype != torch.bfloat16 or scale.shape != (width, groups) or zero.shape != (width, groups):
         raise LinnetError(f"{what}: scale is [{width}, {groups}] bf16 and zero [{width}, {groups}] uint8")
-    if bias is not None and (bias.dtype != torch.bfloat16 or tuple(bias.shape) != (width,)):
+    if bias is not None and (bias.dtype != torch.bfloat16 or bias.shape != (width,)):
         raise LinnetError(f"{what}: bias is [{width}] bf16")
     x, operand = x.contiguous(), operand.contiguous()
     packed, scale, zero = packed.contiguous(), scale.contiguous(), zero.contiguous()
     bias = None if bias is None else bias.contiguous()
     if out is None:
         y = torch.empty(rows, width, dtype=x.dtype, device=device)
-    elif tuple(out.shape) != (rows, width) or out.dtype != x.dtype or out.device != device or not out.is_contiguous():
+    elif out.shape != (rows, width) or out.dtype != x.dtype or out.device != device or not out.is_contiguous():
         raise LinnetError(f"{what}: out is a contiguous [{rows}, {width}] bf16 tensor on {device}")
     else:
         y = out
@@ -307,7 +331,7 @@ def _prologue_linear(what: str, prologue: int, x: torch.Tensor, operand: torch.T
     # group, an In no one-token kernel takes); one row's is a few KB.
     staged = torch.empty_like(x)
     norm = prologue == _lib.PROLOGUE_RMSNORM
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_linear_prologue", _ptr(x), None if norm else _ptr(operand), _ptr(operand) if norm else None,
                   float(eps), prologue, _ptr(packed), _ptr(scale), _ptr(zero), _ptr(bias), _ptr(y), _ptr(staged),
                   rows, depth, width, 2 * half, _lib.BF16, _lib.KERNEL_AUTO, _stream(device))
@@ -323,7 +347,7 @@ def int4_linear_rmsnorm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, 
     to bf16 where `decode.rmsnorm` rounds x * r * w); more rows normalise first.
     With one row, `bias` = the residual stream's row gives residual + product (the
     residual add of the next layer, rounded as it rounds)."""
-    if norm_weight.dtype != torch.float32 or tuple(norm_weight.shape) != (x.shape[-1],):
+    if norm_weight.dtype != torch.float32 or norm_weight.shape != (x.shape[-1],):
         raise LinnetError("int4_linear_rmsnorm: norm_weight is f32 [In]")
     return _prologue_linear("int4_linear_rmsnorm", _lib.PROLOGUE_RMSNORM, x, norm_weight, eps, packed, scale, zero,
                             bias, out)
@@ -349,11 +373,11 @@ def take_inputs(x: torch.Tensor, order: torch.Tensor) -> torch.Tensor:
     device = _on_gpu("take_inputs", x, order)
     code = _code(x.dtype, "take_inputs", (torch.bfloat16, torch.float16, torch.float32))
     n = x.shape[-1] if x.dim() else 0
-    if x.dim() == 0 or order.dtype != torch.int32 or tuple(order.shape) != (n,):
+    if x.dim() == 0 or order.dtype != torch.int32 or order.shape != (n,):
         raise LinnetError(f"take_inputs: order is [{n}] int32 over x's last axis")
     x, order = x.contiguous(), order.contiguous()
     taken = torch.empty_like(x)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_take_inputs", _ptr(x), _ptr(order), _ptr(taken), x.numel() // max(n, 1), n, code,
                   _stream(device))
     return taken
@@ -380,11 +404,11 @@ def int4_weight(raw: torch.Tensor, scale: torch.Tensor, zero: torch.Tensor) -> t
     code = _code(scale.dtype, "int4_weight", (torch.bfloat16, torch.float16, torch.float32))
     if raw.dtype != torch.uint8 or zero.dtype != torch.uint8:
         raise LinnetError("int4_weight: packed and zero are uint8")
-    if tuple(scale.shape) != (width, groups) or tuple(zero.shape) != (width, groups):
+    if scale.shape != (width, groups) or zero.shape != (width, groups):
         raise LinnetError(f"int4_weight: scale and zero are [{width}, {groups}]")
     raw, scale, zero = raw.contiguous(), scale.contiguous(), zero.contiguous()
     out = torch.empty(width, groups * 2 * half, dtype=scale.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_dequantize", _ptr(raw), _ptr(scale), _ptr(zero), _ptr(out),
                   width, groups * 2 * half, 2 * half, code, _stream(device))
     return out
@@ -404,7 +428,7 @@ def quantize_int4(weight: torch.Tensor, group: int) -> tuple[torch.Tensor, torch
     packed = torch.empty(width, depth // group, group // 2, dtype=torch.uint8, device=device)
     scale = torch.empty(width, depth // group, dtype=torch.float32, device=device)
     zero = torch.empty(width, depth // group, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_quantize", _ptr(w), _ptr(packed), _ptr(scale), _ptr(zero),
                   width, depth, group, _stream(device))
     return packed, scale, zero
@@ -420,7 +444,7 @@ def pack4(codes: torch.Tensor) -> torch.Tensor:
         codes = codes.trunc().to(torch.int64)
     as_bytes = (codes.to(torch.int64) & 15).to(torch.uint8).contiguous()
     out = torch.empty(*codes.shape[:-1], codes.shape[-1] // 2, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_pack", _ptr(as_bytes), _ptr(out), out.numel(), _stream(device))
     return out
 
@@ -436,7 +460,7 @@ def unpack4(packed: torch.Tensor, kind: str) -> torch.Tensor:
     packed = packed.contiguous()
     dtype = torch.int8 if kind == "i4" else torch.uint8
     out = torch.empty(*packed.shape[:-1], 2 * packed.shape[-1], dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_unpack", _ptr(packed), _ptr(out), packed.numel(), int(kind == "i4"), _stream(device))
     return out
 
@@ -461,7 +485,7 @@ def int4_row_prepare(weight: torch.Tensor, scale: torch.Tensor, group: int = 128
     packed = torch.empty(width, depth // group, group // 2, dtype=torch.uint8, device=device)
     group_scale = torch.empty(width, depth // group, dtype=scale.dtype, device=device)
     zero = torch.empty(width, depth // group, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_row_prepare", _ptr(weight), _ptr(scale), _ptr(packed), _ptr(group_scale), _ptr(zero),
                   width, depth, group, code, _stream(device))
     return packed, group_scale, zero
@@ -493,10 +517,10 @@ def int4_repack(
     if group <= 0 or in_features % group or group % 2:
         raise LinnetError(f"int4_repack: {in_features} inputs do not make even groups of {group}")
     groups = in_features // group
-    if in_features % 8 or tuple(qzeros.shape) != (groups, out_features // 8):
+    if in_features % 8 or qzeros.shape != (groups, out_features // 8):
         raise LinnetError(f"int4_repack: qzeros is [{groups}, {out_features // 8}], got {tuple(qzeros.shape)}")
     if order is not None:
-        if packing != "gptq" or order.dtype != torch.int32 or tuple(order.shape) != (in_features,):
+        if packing != "gptq" or order.dtype != torch.int32 or order.shape != (in_features,):
             raise LinnetError(f"int4_repack: an order is GPTQ's, [{in_features}] int32")
         order = order.contiguous()
         # The kernel reads whatever input an entry names (an entry out of range as
@@ -513,7 +537,7 @@ def int4_repack(
     qweight, qzeros = qweight.contiguous(), qzeros.contiguous()
     packed = torch.empty(out_features, groups, group // 2, dtype=torch.uint8, device=device)
     zero = torch.empty(out_features, groups, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int4_repack", _ptr(qweight), _ptr(qzeros), _ptr(order), kinds[packing], zero_offset,
                   in_features, out_features, groups, _ptr(packed), _ptr(zero), _stream(device))
     return packed, zero
@@ -535,9 +559,9 @@ def mxfp4_experts(x: torch.Tensor, blocks: torch.Tensor, scales: torch.Tensor, e
     count, out_features, groups, sixteen = blocks.shape
     if sixteen != 16 or blocks.dtype != torch.uint8 or scales.dtype != torch.uint8:
         raise LinnetError("mxfp4_experts: blocks are [E, Out, G, 16] and scales [E, Out, G], both uint8")
-    if tuple(scales.shape) != (count, out_features, groups) or width != groups * 32:
+    if scales.shape != (count, out_features, groups) or width != groups * 32:
         raise LinnetError(f"mxfp4_experts: x's In={width}, blocks {tuple(blocks.shape)}, scales {tuple(scales.shape)}")
-    if tuple(experts.shape) != (rows, chosen) or experts.is_floating_point():
+    if experts.shape != (rows, chosen) or experts.is_floating_point():
         raise LinnetError(f"mxfp4_experts: experts are integers [{rows}, {chosen}]")
     code = _code(x.dtype, "mxfp4_experts")
     if (x.stride(2) != 1 or x.data_ptr() % 16 or x.stride(0) % 8 or x.stride(1) % 8):
@@ -545,7 +569,7 @@ def mxfp4_experts(x: torch.Tensor, blocks: torch.Tensor, scales: torch.Tensor, e
     blocks, scales = blocks.contiguous(), scales.contiguous()
     ids = experts.to(torch.int64).contiguous()
     y = torch.empty(rows, chosen, out_features, dtype=x.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_mxfp4_experts", _ptr(x), x.stride(0), x.stride(1), _ptr(blocks), _ptr(scales), _ptr(ids),
                   _ptr(y), rows, chosen, count, out_features, width, code, _stream(device))
     return y
@@ -562,7 +586,7 @@ def _scale_columns(weight: torch.Tensor, scale: torch.Tensor, group: int, row_bl
     else:
         if depth % group or width % row_block:
             raise LinnetError(f"scales of {row_block}x{group} blocks do not tile [{width}, {depth}]")
-        if tuple(scale.shape) != (width // row_block, depth // group):
+        if scale.shape != (width // row_block, depth // group):
             raise LinnetError(f"scale is [{width // row_block}, {depth // group}], got {tuple(scale.shape)}")
 
 
@@ -590,7 +614,7 @@ def w8a16(x: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, fp8: bool,
         raise LinnetError("w8a16: scales are f32 (the operands' form)")
     x, wb, scale = x.contiguous(), _bytes(weight), scale.contiguous()
     y = torch.empty(rows, width, dtype=x.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_w8a16", _ptr(x), _ptr(wb), _ptr(scale), _ptr(y), rows, width, depth,
                   int(fp8), group, row_block, code, _stream(device))
     return y
@@ -612,7 +636,7 @@ def dequantize8(weight: torch.Tensor, scale: torch.Tensor, fp8: bool, group: int
     code = _code(dtype, "dequantize8", (torch.bfloat16, torch.float16, torch.float32))
     wb, scale = _bytes(weight), scale.to(torch.float32).contiguous()
     out = torch.empty(width, depth, dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_dequantize8", _ptr(wb), _ptr(scale), _ptr(out), width, depth, int(fp8),
                   group, row_block, code, _stream(device))
     return out
@@ -625,7 +649,7 @@ def _rows8(x: torch.Tensor, fp8: bool) -> tuple[torch.Tensor, torch.Tensor]:
     x = x.contiguous()
     q = torch.empty(rows, depth, dtype=torch.float8_e4m3fn if fp8 else torch.int8, device=device)
     scale = torch.empty(rows, 1, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_rows8", _ptr(x), _ptr(q), _ptr(scale), rows, depth, int(fp8), code, _stream(device))
     return q, scale
 
@@ -657,7 +681,7 @@ def _mm8(q: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor, scale: to
     xs = x_scale.to(torch.float32).contiguous()
     ws = scale.to(torch.float32).contiguous()
     y = torch.empty(rows, width, dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_mm8_tiles", _ptr(qb), _ptr(wb), _ptr(xs), _ptr(ws), _ptr(y), rows, width, depth,
                   int(fp8), code, tile_n, _stream(device))
     return y
@@ -696,7 +720,7 @@ def fp8_groups(x: torch.Tensor, group: int, padded: int) -> tuple[torch.Tensor, 
     x = x.contiguous()
     q = torch.empty(padded, depth, dtype=torch.float8_e4m3fn, device=device)
     scale = torch.empty(depth // group, padded, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_fp8_groups", _ptr(x), _ptr(q), _ptr(scale), rows, padded, depth, group, code, _stream(device))
     return q, scale.t()
 
@@ -714,9 +738,9 @@ def fp8_block_mm(q: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor, s
     width = weight.shape[0]
     if weight.shape[1] != depth or depth % 128 or width % 128:
         raise LinnetError(f"fp8_block_mm: weight {tuple(weight.shape)} against In={depth} (both % 128 == 0)")
-    if tuple(scale.shape) != (width // 128, depth // 128):
+    if scale.shape != (width // 128, depth // 128):
         raise LinnetError(f"fp8_block_mm: scale is [{width // 128}, {depth // 128}], got {tuple(scale.shape)}")
-    if tuple(x_scale.shape) != (rows, depth // 128):
+    if x_scale.shape != (rows, depth // 128):
         raise LinnetError(f"fp8_block_mm: x_scale is [{rows}, {depth // 128}], got {tuple(x_scale.shape)}")
     code = _code(dtype, "fp8_block_mm")
     # The kernel reads x_scale[b * stride + row]: a column-major [rows, In/128] view.
@@ -727,7 +751,7 @@ def fp8_block_mm(q: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor, s
     qb, wb = _bytes(q.contiguous()), _bytes(weight.contiguous())
     ws = scale.to(torch.float32).contiguous()
     y = torch.empty(rows, width, dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_mm8_block", _ptr(qb), _ptr(wb), _ptr(xs), stride, _ptr(ws), _ptr(y), rows, width, depth,
                   code, _stream(device))
     return y
@@ -767,7 +791,7 @@ def quantize_int8(weight: torch.Tensor, group: int, dtype: str) -> tuple[torch.T
     w = weight.to(torch.float32).contiguous()
     q = torch.empty(width, depth, dtype=torch.int8, device=device)
     scale = torch.empty(width, depth // group, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_int8_quantize", _ptr(w), _ptr(q), _ptr(scale), width, depth, group, codes[dtype], _stream(device))
     return q, scale
 
@@ -797,7 +821,7 @@ def nf4_dequantize(codes: torch.Tensor, absmax: torch.Tensor, block: int, dtype:
     code = _code(dtype, "nf4_dequantize", (torch.bfloat16, torch.float16, torch.float32))
     codes, absmax = codes.contiguous(), absmax.contiguous()
     out = torch.empty(out_features, in_features, dtype=dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_nf4_dequant", _ptr(codes), _ptr(absmax), _ptr(out), out_features, in_features, block, code,
                   _stream(device))
     return out
@@ -847,7 +871,7 @@ def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: 
     if bias is not None and (bias.dtype != x.dtype or bias.numel() != out_features):
         raise LinnetError(f"nf4_gemv: bias is [{out_features}] {x.dtype}")
     lead = x.shape[:-1]
-    x2 = x.reshape(-1, in_features)
+    x2 = x if x.dim() == 2 else x.reshape(-1, in_features)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16 or (x2.shape[0] > 1 and x2.stride(0) < in_features):
         x2 = x2.contiguous()
         if in_features % 8:
@@ -855,10 +879,10 @@ def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: 
     codes, absmax = codes.contiguous(), absmax.contiguous()
     bias = None if bias is None else bias.contiguous()
     y = torch.empty(x2.shape[0], out_features, dtype=x.dtype, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_nf4_linear", _ptr(x2), max(x2.stride(0), in_features), x2.shape[0], _ptr(codes), _ptr(absmax),
                   _ptr(bias), _ptr(y), out_features, out_features, in_features, block, code, _stream(device))
-    return y.reshape(*lead, out_features)
+    return y if x.dim() == 2 else y.reshape(*lead, out_features)
 
 
 def nf4_linear(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: int,
@@ -910,7 +934,7 @@ def nf4_repack(packed: torch.Tensor, absmax: torch.Tensor, out_features: int, in
     nested_map = None if nested_map is None else nested_map.contiguous()
     codes = torch.empty(out_features, in_features // 2, dtype=torch.uint8, device=device)
     scale = torch.empty(out_features, in_features // block, dtype=torch.float32, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _lib.call("lnq_nf4_repack", _ptr(packed), _ptr(absmax), _ptr(nested_absmax), _ptr(nested_map),
                   nested_block, ctypes.c_float(offset), _ptr(codes), _ptr(scale), out_features, in_features, block,
                   _stream(device))

@@ -66,7 +66,8 @@ def _weight_only(flat: torch.Tensor, weight: torch.Tensor, scale: torch.Tensor, 
 
 
 def _finish(x: torch.Tensor, y: torch.Tensor, bias: torch.Tensor | None) -> torch.Tensor:
-    y = y.reshape(*x.shape[:-1], y.shape[-1])
+    if x.dim() != 2:
+        y = y.reshape(*x.shape[:-1], y.shape[-1])
     return y if bias is None else y + bias
 
 
@@ -85,7 +86,7 @@ def fp8_operands(weight: torch.Tensor, scale: torch.Tensor, rounded: int) -> Fp8
 def fp8_linear(x: torch.Tensor, operands: Fp8Operands, bias: torch.Tensor | None) -> torch.Tensor:
     """`quantized.py:123-135`."""
     weight, fp8, scale, rounded, fast = operands
-    flat = x.reshape(-1, x.shape[-1])
+    flat = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if fast and flat.dtype in _HALF:
         if rounded and fast == 2 and flat.shape[0] > FEW_ROWS:
             q, rows = kernels.fp8_rows(flat)
@@ -117,7 +118,7 @@ def fp8_block_linear(x: torch.Tensor, operands: Fp8BlockOperands, bias: torch.Te
     FP8 per 128 inputs (`fp8_groups`) and the block-scaled FP8 product; else the
     weight-only kernels."""
     weight, fp8, scale, block, rounded, fast = operands
-    flat = x.reshape(-1, x.shape[-1])
+    flat = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if fast and flat.dtype in _HALF:
         rows = flat.shape[0]
         if rounded and fast == 2 and rows > FEW_ROWS:
@@ -141,7 +142,7 @@ def int8_operands(weight: torch.Tensor, scale: torch.Tensor, rounded: int) -> In
 def int8_linear(x: torch.Tensor, operands: Int8Operands, bias: torch.Tensor | None) -> torch.Tensor:
     """`quantized.py:183-194`."""
     weight, scale, rounded, fast = operands
-    flat = x.reshape(-1, x.shape[-1])
+    flat = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if fast and flat.dtype in _HALF:
         if rounded and flat.shape[0] > FEW_ROWS:
             q, rows = kernels.int8_rows(flat)
@@ -166,7 +167,7 @@ def int8_group_operands(weight: torch.Tensor, scale: torch.Tensor) -> Int8GroupO
 def int8_group_linear(x: torch.Tensor, operands: Int8GroupOperands, bias: torch.Tensor | None) -> torch.Tensor:
     """`quantized.py:206-218`."""
     weight, scale, group, fast = operands
-    flat = x.reshape(-1, x.shape[-1])
+    flat = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if fast and flat.dtype in _HALF:
         y = _weight_only(flat, weight, scale, False, group)
     else:
