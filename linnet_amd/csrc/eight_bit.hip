@@ -737,6 +737,11 @@ LNQ_API LnqStatus lnq_mm8_tiles(const uint8_t* qx, const uint8_t* weight, const 
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto* ys = static_cast<uint16_t*>(y);
   const int bn = tile_n == 0 ? mm8_kernel_for(M, N, K, fp8 != 0) : tile_n;
+  // Chosen, not asked for, and too few large tiles for the chip: small ones where they win.
+  if (tile_n == 0 && (bn == 128 || bn == LNQ_MM8_STREAM)) {
+    const int bm = mm8_small_rows(M, N, K, false);
+    if (bm) return launch_mm8_small(bm, qx, weight, x_scale, scale, y, M, N, K, fp8, dtype, s);
+  }
   if (bn == LNQ_MM8_PERSISTENT) {
     const int tiles = ((M + mm8p::BM - 1) / mm8p::BM) * (N / mm8p::BN);
     const dim3 grid(tiles < compute_units() ? tiles : compute_units());

@@ -882,4 +882,13 @@ __global__ __launch_bounds__(mm8p::THREADS, 1) void mm8p_kernel(
   wait_vm<0>();
 }
 
+// mm8_small.hip: tiles of 32 to 128 rows by 64 columns. mm8_small_rows chooses (0: use the
+// 256-row tiles); the launches expect lnq_mm8's / lnq_mm8_block's checks to have passed.
+int mm8_small_rows(int M, int N, int K, bool blk);
+LnqStatus launch_mm8_small(int bm, const uint8_t* qx, const uint8_t* weight, const float* x_scale,
+                           const float* scale, void* y, int M, int N, int K, int fp8, int dtype, hipStream_t s);
+LnqStatus launch_mm8_block_small(int bm, const uint8_t* qx, const uint8_t* weight, const float* x_scale,
+                                 int xs_stride, const float* scale, void* y, int M, int N, int K, int dtype,
+                                 hipStream_t s);
+
 }  // namespace lnq

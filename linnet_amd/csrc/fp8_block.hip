@@ -99,6 +99,8 @@ LNQ_API LnqStatus lnq_mm8_block(const uint8_t* qx, const uint8_t* weight, const 
               "lnq_mm8_block: operands exceed the 2 GiB buffer range");
   hipStream_t s = static_cast<hipStream_t>(stream);
   auto* ys = static_cast<uint16_t*>(y);
+  if (const int bm = mm8_small_rows(M, N, K, true))
+    return launch_mm8_block_small(bm, qx, weight, x_scale, static_cast<int>(xs_stride), scale, y, M, N, K, dtype, s);
   const int tiles = ((M + mm8::BM - 1) / mm8::BM) * (N / 128);
   if (dtype == LNQ_BF16)
     hipLaunchKernelGGL((mm8_kernel<LNQ_BF16, 1, 128, true>), dim3(tiles), dim3(mm8::THREADS), 0, s, qx, weight,

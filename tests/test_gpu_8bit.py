@@ -231,6 +231,41 @@ def test_fp8_block_product(rows: int, out: int, width: int, dtype: torch.dtype) 
     assert np.all(np.abs(y - want) <= 8e-3 * np.abs(want) + 1e-3 * top)
 
 
+# Edges of the 32-, 64- and 128-row tiles, a partial last column tile, one step to many
+# (fewer than the stages, and no multiple of them), rows past a tile's last.
+@pytest.mark.parametrize(("rows", "out", "width"), [(1, 64, 128), (33, 65, 256), (48, 2048, 1152), (64, 7000, 640),
+                                                    (97, 4097, 2048), (129, 2050, 4096), (600, 700, 3200), (257, 14336, 512)])
+@pytest.mark.parametrize("fp8", [True, False])
+def test_mm8_small_tiles(rows: int, out: int, width: int, fp8: bool) -> None:
+    """The chosen form (small tiles where they win) has the bits of the 256-row tiles."""
+    g = torch.Generator().manual_seed(rows + out)
+    xs, ws = torch.rand(rows, generator=g).to(DEV), torch.rand(out, generator=g).to(DEV)
+    q, w = (torch.randint(-127, 128, (n, width), generator=g, dtype=torch.int8) for n in (rows, out))
+    mm = kernels.int8_mm
+    if fp8:
+        mm, q, w = kernels.fp8_mm, q.float().to(torch.float8_e4m3fn), w.float().to(torch.float8_e4m3fn)
+    q, w = q.to(DEV), w.to(DEV)
+    for dtype in (torch.bfloat16, torch.float16):
+        assert torch.equal(mm(q, w, xs * 1e-2, ws * 1e-2, dtype), mm(q, w, xs * 1e-2, ws * 1e-2, dtype, tile_n=128))
+
+
+@pytest.mark.parametrize(("rows", "out", "width"), [(33, 128, 128), (65, 4096, 640), (129, 2048, 1152), (200, 7168, 2048), (500, 640, 4096)])
+def test_fp8_block_small_tiles(rows: int, out: int, width: int) -> None:
+    """Small tiles' block fold. Whole codes up to 8 and scales of powers of two: every sum is
+    exact in f32, so the result is the f64 product rounded once."""
+    g = torch.Generator().manual_seed(rows)
+    q, w = (torch.randint(-8, 9, (n, width), generator=g).float().to(torch.float8_e4m3fn) for n in (rows, out))
+    xs = torch.randint(-1, 3, (width // 128, rows + 3), generator=g).float().exp2()[:, :rows].t()
+    ws = torch.randint(-1, 3, (out // 128, width // 128), generator=g).float().exp2()
+    xd = q.double() * xs.double().repeat_interleave(128, 1)
+    wd = w.double() * ws.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    assert float(xd.abs().amax() * wd.abs().amax()) * width <= 2.0**22  # in units of 1/4: 2^24
+    q, w, xs, ws = q.to(DEV), w.to(DEV), xs.to(DEV), ws.to(DEV)
+    for dtype in (torch.bfloat16, torch.float16):
+        got = kernels.fp8_block_mm(q, w, xs / 64, ws / 64, dtype).cpu()
+        assert torch.equal(got, ((xd @ wd.t()) / 4096).to(dtype))
+
+
 def test_fp8_block_product_takes_row_major_scales() -> None:
     """x scales given row-major [rows, In/128] (not `fp8_groups`' view) give the same product."""
     g = torch.Generator().manual_seed(3)
