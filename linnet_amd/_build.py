@@ -45,7 +45,7 @@ FLAGS = [
 # one with AGPRs has it split in half, and the GEMV kernels then spill.
 EXTRA = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"]
          for name in ("int4.hip", "int4_gemv.hip", "int4_stream.hip", "fp8_stream.hip", "int8_stream.hip", "nf4.hip",
-                      "mxfp4.hip", "fp8_block.hip", "mm8_small.hip")}
+                      "mxfp4.hip", "fp8_block.hip", "mm8_small.hip", "int4_mid.hip")}
 
 
 def hipcc() -> str:

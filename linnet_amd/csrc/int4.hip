@@ -644,6 +644,11 @@ LnqStatus launch_int4_gemv_tiles(const void* xt, const uint8_t* packed, const vo
                                  const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
 LnqStatus launch_x_tiles(const void* x, void* xt, int rows, int K, hipStream_t stream);
 
+// Defined in int4_mid.hip: the dequant-GEMM in 64 x 128 tiles with K split inside a workgroup.
+bool int4_mid_preferred(int M, int N);
+LnqStatus launch_int4_mid(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero, const void* bias,
+                          void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
+
 // Defined in int4_stream.hip: the streaming few-row product.
 bool int4_stream_supports(int K);
 LnqStatus launch_int4_stream(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
@@ -833,6 +838,9 @@ LNQ_API LnqStatus lnq_int4_linear(const void* x, const uint8_t* packed, const vo
   }
   if (code == LNQ_KERNEL_PERSISTENT)
     return launch_int4_persistent(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
+  // Chosen, not asked for: small tiles where they give no CU a second one.
+  if (kernel == LNQ_KERNEL_AUTO && code == LNQ_KERNEL_TILED_128 && int4_mid_preferred(M, N))
+    return launch_int4_mid(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
   if (code == LNQ_KERNEL_TILED_128 || code == LNQ_KERNEL_TILED_256)
     return launch_int4_tiled(x, packed, scale, zero, bias, y, M, N, K, G, dtype,
                              code == LNQ_KERNEL_TILED_256 ? 256 : 128, s);

@@ -159,6 +159,36 @@ def test_mxfp4_grouped(dtype: torch.dtype, rows: int, chosen: int, count: int, o
         assert (got[r].double() - alone).abs().max().item() <= 2 * ULP[dtype] * top
 
 
+@pytest.mark.parametrize(("rows", "out", "width", "group", "dtype"), [
+    (65, 40, 128, 128, BF16),  # half of the only step, a partial tile, rows past the last
+    (66, 130, 384, 64, F16),  # a step and a half, a second column tile of 2
+    (129, 384, 1152, 32, BF16),  # two scales a chunk
+    (128, 256, 1024, 128, F16),  # 8 groups at once
+    (200, 700, 13 * 1024, 128, BF16),  # 52 steps: both scale sets on either side of the unrolled twelve
+    (257, 129, 3328, 128, BF16),  # 13 steps, 26 groups: one a step
+    (300, 514, 2048, 256, F16),
+    (96, 2050, 768, 32, F16),
+])
+def test_int4_mid(rows: int, out: int, width: int, group: int, dtype: torch.dtype) -> None:
+    """The automatic choice at 65 rows up to a tile a CU: products of x and the weight rounded
+    to x's type, as the prefill kernels' -- that rounding is in the reference here."""
+    print(f"int4 mid rows={rows} out={out} in={width} group={group} {dtype}", flush=True)
+    rng = np.random.default_rng(rows + out)
+    codes = rng.integers(0, 16, (out, width)).astype(np.uint8)
+    packed = (codes[:, 0::2] | (codes[:, 1::2] << 4)).reshape(out, width // group, group // 2)
+    scale = torch.from_numpy((rng.random((out, width // group)) * 0.02 + 0.001).astype(np.float32)).to(dtype)
+    zero = rng.integers(0, 16, (out, width // group)).astype(np.uint8)
+    wide = scale.double().numpy().repeat(group, 1) * (codes.astype(np.float64) - zero.repeat(group, 1))
+    w = torch.from_numpy(wide).float().to(dtype).double().numpy()
+    x = _x(rows, width, dtype)
+    bias = _x(1, out, dtype)[0] if rows % 2 else None
+    args = [t.to(DEV) for t in (x, torch.from_numpy(packed), scale, torch.from_numpy(zero))]
+    bias_d = None if bias is None else bias.to(DEV)
+    got = kernels.int4_linear(*args, bias_d)
+    _check(got, x, w, np.abs(w), bias)
+    _check(kernels.int4_linear(*args, bias_d, kernel="tiled128"), x, w, np.abs(w), bias)
+
+
 def test_replayed_from_a_graph() -> None:
     """A captured call of each format replays to the eager bits with work between."""
     x = _x(12, 1024, BF16).to(DEV)
