@@ -15,6 +15,7 @@ import dataclasses
 import functools
 
 import torch
+from torch.autograd import forward_ad
 
 from .. import _lib
 from ..errors import LinnetError
@@ -847,16 +848,26 @@ def nf4_gemv_fits(rows: int, in_features: int, block: int, dtype: torch.dtype) -
 # Rows up to which `nf4_linear` reads the stored weight at all: past NF4_GEMV_ROWS on the
 # streaming kernel, 32 rows a pass.
 NF4_STREAM_ROWS = 96
-NF4_STREAM_MAX_IN = 65536
 
 
-def _nf4_reads_stored(rows: int, in_features: int, block: int, dtype: torch.dtype) -> bool:
+def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor | None, rows: int, block: int) -> bool:
     """Whether `nf4_linear` multiplies by the stored weight (`lnq_nf4_linear`) rather than
-    the widened one."""
-    if nf4_gemv_fits(rows, in_features, block, dtype):
+    the widened one. Past the GEMV's rows the widened product takes whatever that entry
+    refuses (wide or huge weights, operands off their alignment, a broadcast bias) and what
+    needs an operator that autograd and vmap know."""
+    out_features, in_features = codes.shape[0], 2 * codes.shape[1]
+    if nf4_gemv_fits(rows, in_features, block, x.dtype):
         return True
-    return (dtype in _HALF and rows <= NF4_STREAM_ROWS and (block in (32, 64) or block % 128 == 0)
-            and in_features % block == 0 and 0 < in_features <= NF4_STREAM_MAX_IN)
+    if not (x.dtype in _HALF and rows <= NF4_STREAM_ROWS and (block in (32, 64) or block % 128 == 0)
+            and in_features % block == 0 and 0 < in_features <= NF4_GEMV_MAX_IN
+            and out_features * in_features < 1 << 32):
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
+        return False
+    if torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0:
+        return False
+    return (bias is None or (bias.dtype == x.dtype and bias.numel() == out_features)) and (
+        (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))
 
 
 def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: int,
@@ -893,7 +904,7 @@ def nf4_linear(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block
     _on_gpu("nf4_linear", x, codes, absmax, bias)
     out_features, in_features = _nf4_operands("nf4_linear", codes, absmax, block)
     rows = x.numel() // max(in_features, 1) if x.dim() else 0
-    if _nf4_reads_stored(rows, in_features, block, x.dtype):
+    if _nf4_reads_stored(x, codes, bias, rows, block):
         return nf4_gemv(x, codes, absmax, block, bias)
     weight = nf4_dequantize(codes, absmax, block, x.dtype)
     return torch.nn.functional.linear(x, weight, bias)

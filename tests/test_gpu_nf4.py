@@ -245,3 +245,28 @@ def test_import_rejects_other_bitsandbytes_types(tmp_path: Path) -> None:
     with pytest.raises(lquant.LinnetError, match="load_in_4bit"):
         lquant.import_quantized(tmp_path / "bnb.safetensors", tmp_path / "o.safetensors",
                                 config={"quant_method": "bitsandbytes"})
+
+
+@pytest.mark.parametrize("form", ["wide", "offset", "grad", "vmap", "broadcast"])
+def test_widened_where_the_stored_product_refuses(form: str) -> None:
+    """Past the GEMV's rows, calls the stored product does not take keep the widened one."""
+    g = torch.Generator().manual_seed(1)
+    rows, out, width = 20, 8, 33024 if form == "wide" else 256
+    codes = torch.randint(0, 256, (out, width // 2), generator=g, dtype=torch.uint8).to("cuda")
+    absmax = torch.rand(out, width // 64, generator=g).to("cuda")
+    bias = torch.ones(1, dtype=torch.bfloat16, device="cuda") if form == "broadcast" else None
+    x = torch.randn(rows * width + 1, generator=g).to(torch.bfloat16).to("cuda")
+    x = (x[1:] if form == "offset" else x[:-1]).view(rows, width)
+    if form == "grad":
+        x.requires_grad_()
+    weight = kernels.nf4_dequantize(codes, absmax, 64, torch.bfloat16)
+    if form == "vmap":
+        both = torch.stack([x, -x])
+        got = torch.vmap(lambda t: kernels.nf4_linear(t, codes, absmax, 64))(both)
+        want = torch.nn.functional.linear(both, weight)
+    else:
+        got, want = kernels.nf4_linear(x, codes, absmax, 64, bias), torch.nn.functional.linear(x, weight, bias)
+    torch.testing.assert_close(got, want, rtol=1e-2, atol=1e-2 * want.abs().max().item())
+    if form == "grad":
+        got.sum().backward()
+        assert x.grad is not None and bool(x.grad.abs().sum() > 0)
