@@ -26,6 +26,7 @@
 //   200 rows 14336 -> 4096   122.9 -> 59.1  (15.8)   512 rows 14336 -> 4096  152.0 -> 79.2
 // group 64, 200 rows 8192 -> 8192: 84.3 -> 53.6; group 32, 200 rows 4096 -> 4096: 40.1 -> 30.5.
 #include "common.hpp"
+#include "stream.hpp"
 
 namespace lnq {
 
@@ -49,13 +50,30 @@ __device__ inline f32x16 mid_mfma(u32x4 a, u32x4 b, f32x16 c) {
 // SC, how a lane gets the scales and zero points of its column (lane l: column l of the wave's
 // 64; a swap of the wave's halves hands out the two blocks): 8 groups of 128 at once, one for
 // four steps (In % 1024 == 0); one a step (groups of 64 and more); two a step (groups of 32).
-enum class Scales { BLOCK, ONE, TWO };
+// NF4 (lnq_nf4_linear): the codes' values in x's type are the MFMA operand, x the other, so a
+// lane holds one column of the product; each 64 inputs' partial tile (a block is 64 or more)
+// is folded in f32 with the column's absmax.
+enum class Scales { BLOCK, ONE, TWO, NF4 };
+
+struct MidArgs {
+  const uint16_t* x;
+  const uint8_t* packed;
+  const void* scale;  // x's type; NF4: f32 absmax
+  const uint8_t* zero;
+  const uint16_t* bias;
+  uint16_t* y;
+  int M, N, K, gshift, x_stride, y_stride;
+  stream::Planes planes;
+};
 
 template <int DT, Scales SC>
-__global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
-    const uint16_t* __restrict__ x, const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scale,
-    const uint8_t* __restrict__ zero, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int M, int N, int K,
-    int gshift) {
+__global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(MidArgs args) {
+  const uint16_t* const x = args.x;
+  const uint8_t* const packed = args.packed;
+  const uint16_t* const bias = args.bias;
+  uint16_t* const y = args.y;
+  const int M = args.M, N = args.N, K = args.K, gshift = args.gshift;
+  constexpr bool NF = SC == Scales::NF4;
   using namespace mid;
   using E = Elem<DT>;
   constexpr int FA = BM / 32, FB = 2;
@@ -81,7 +99,8 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
   // Rows past M and columns past N read zeros through the range checks, and so does a step past
   // the end (a descriptor of no bytes at offset 0). A chunk past the end of K in the last step
   // has zeros for x (likewise) and a scale of 0; its weights are the next column's.
-  const uint32_t x_bytes = static_cast<uint32_t>(M) * static_cast<uint32_t>(K) * 2u;
+  const uint32_t x_row = static_cast<uint32_t>(args.x_stride) * 2u;
+  const uint32_t x_bytes = static_cast<uint32_t>(M - 1) * x_row + static_cast<uint32_t>(K) * 2u;
   const uint32_t w_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(K >> 1);
   const uint32_t z_bytes = static_cast<uint32_t>(N) * static_cast<uint32_t>(groups);
 
@@ -89,7 +108,7 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
   // l % 8 holding source column (l % 8) ^ key(row), key = bits 1..3 of the row. Weight load i:
   // columns 8 (wave + 8 i) .. + 7 of the tile, in the same layout.
   const int xrow = 8 * cw + (lane >> 3), wrow = 8 * wave + (lane >> 3);
-  const uint32_t xoff = (static_cast<uint32_t>(m0 + xrow) * K + 64u * kw) * 2u +
+  const uint32_t xoff = static_cast<uint32_t>(m0 + xrow) * x_row + 128u * kw +
                         static_cast<uint32_t>(((lane & 7) ^ ((xrow >> 1) & 7)) * 16);
   const uint32_t woff = static_cast<uint32_t>(n0 + wrow) * static_cast<uint32_t>(K >> 1) +
                         static_cast<uint32_t>(((lane & 7) ^ ((wrow >> 1) & 7)) * 16);
@@ -99,7 +118,7 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
 #pragma unroll
     for (int i = 0; i < BM / 16; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(stage + kw * (BM * 128) + (cw + 2 * i) * 1024), 16,
-                                               xoff + static_cast<uint32_t>(16 * i) * K * 2u, xin ? ks * STEP * 2 : 0, 0, 0);
+                                               xoff + static_cast<uint32_t>(16 * i) * x_row, xin ? ks * STEP * 2 : 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < BN / 64; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr)(stage + XPART + (wave + 8 * i) * 1024), 16,
@@ -110,14 +129,17 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
     u32x4 s;  // BLOCK: 8 scales; else s.x (and s.y: inputs 32 .. 63 of the chunk)
     u32x2 z;
   };
-  constexpr int SLOADS = SC == Scales::TWO ? 4 : 2;
+  constexpr int SLOADS = NF ? 1 : SC == Scales::TWO ? 4 : 2;
   const uint32_t goff = static_cast<uint32_t>(n0 + 64 * cw + lane) * static_cast<uint32_t>(groups);
   auto load_scales = [&](int ks, G& r) {
     const int k0 = ks * STEP + CHUNK * kw;
     const bool in = SC == Scales::BLOCK ? ks < steps : k0 < K;
-    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(scale, in ? 2u * z_bytes : 0u), rz = buffer_rsrc(zero, in ? z_bytes : 0u);
+    const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(args.scale, in ? (NF ? 4u : 2u) * z_bytes : 0u),
+                                 rz = buffer_rsrc(args.zero, in ? z_bytes : 0u);
     const uint32_t at = goff + (in ? static_cast<uint32_t>((SC == Scales::BLOCK ? ks * STEP : k0) >> gshift) : 0u);
-    if constexpr (SC == Scales::BLOCK) {
+    if constexpr (NF) {
+      r.s.x = __builtin_amdgcn_raw_buffer_load_b32(rs, 4u * at, 0, 0);
+    } else if constexpr (SC == Scales::BLOCK) {
       r.s = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, 2u * at, 0, 0));
       r.z = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rz, at, 0, 0));
     } else {
@@ -129,12 +151,14 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
       }
     }
   };
-  // This lane's scale and zero point of column block b, packed (zero << 16 | scale).
+  // This lane's scale and zero point of column block b, packed (zero << 16 | scale); NF4: absmax.
   auto hand_out = [&](const G& r, int j, uint32_t (&o)[FB]) {
     uint32_t v;
     if constexpr (SC == Scales::BLOCK) {  // group 2 j + kw / 2 of the eight
       const uint32_t gs = r.s[j] >> (16 * (kw >> 1)), gz = r.z[j >> 1] >> (16 * (j & 1) + 8 * (kw >> 1));
       v = (gs & 0xffffu) | (gz << 16);
+    } else if constexpr (NF) {
+      v = r.s.x;
     } else {
       v = r.s.x | (r.z.x << 16);
     }
@@ -224,6 +248,7 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
     float s[FB], c[FB], s16[FB], c16[FB];
 #pragma unroll
     for (int b = 0; b < FB; ++b) {
+      if constexpr (NF) continue;
       s[b] = E::to_f32(static_cast<uint16_t>(sz[b]));
       const float z = static_cast<float>((sz[b] >> 16) & 0xffu);
       c[b] = -(1024.f + z) * s[b];
@@ -233,23 +258,45 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
     // Operand i = 2 kk + b: its MFMAs run over operand i + 1's dequantization, half of it
     // behind each (a scheduling region a MFMA pins that).
     u32x4 xa[2][FA], wb[2];
-    auto read_x = [&](int kk, int a) { xa[kk & 1][a] = *reinterpret_cast<const u32x4*>(stage + aoff[kk] + a * 4096); };
+    f32x16 part[NF ? FA : 1][NF ? FB : 1];
+    auto read_x = [&](int kk, int a) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(stage + aoff[kk] + a * 4096);
+      xa[kk & 1][a] = NF ? stream::permute_nf4(v) : v;
+    };
 #pragma unroll
     for (int a = 0; a < FA; ++a) read_x(0, a);
-    wb[0] = dequant_rest(dequant_first(wq[0][0], s[0], c[0], s16[0], c16[0]), s[0], c[0], s16[0], c16[0]);
+    if constexpr (NF) wb[0] = stream::nf4_widen(wq[0][0], args.planes);
+    else wb[0] = dequant_rest(dequant_first(wq[0][0], s[0], c[0], s16[0], c16[0]), s[0], c[0], s16[0], c16[0]);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int kk = i / FB, b = i % FB, nb = (i + 1) % FB, nk = (i + 1) / FB;
       Deq d;
-      acc[0][b] = mid_mfma<DT>(wb[i & 1], xa[kk & 1][0], acc[0][b]);
-      if (i < 7) d = dequant_first(wq[nb][nk], s[nb], c[nb], s16[nb], c16[nb]);
+      auto multiply = [&](int a) {
+        if constexpr (NF) part[a][b] = mid_mfma<DT>(xa[kk & 1][a], wb[i & 1], kk == 0 ? f32x16{} : part[a][b]);
+        else acc[a][b] = mid_mfma<DT>(wb[i & 1], xa[kk & 1][a], acc[a][b]);
+      };
+      multiply(0);
+      if constexpr (!NF)
+        if (i < 7) d = dequant_first(wq[nb][nk], s[nb], c[nb], s16[nb], c16[nb]);
       if (b == 0 && kk < 3) read_x(kk + 1, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      acc[1][b] = mid_mfma<DT>(wb[i & 1], xa[kk & 1][1], acc[1][b]);
-      if (i < 7) wb[(i + 1) & 1] = dequant_rest(d, s[nb], c[nb], s16[nb], c16[nb]);
+      if constexpr (!NF) __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+      if (i < 7) {
+        if constexpr (NF) wb[(i + 1) & 1] = stream::nf4_widen(wq[nb][nk], args.planes);
+        else wb[(i + 1) & 1] = dequant_rest(d, s[nb], c[nb], s16[nb], c16[nb]);
+      }
       if (b == 0 && kk < 3) read_x(kk + 1, 1);
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (NF) {
+#pragma unroll
+      for (int b = 0; b < FB; ++b)
+#pragma unroll
+        for (int a = 0; a < FA; ++a)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[a][b][r] = fmaf(part[a][b][r], __builtin_bit_cast(float, sz[b]), acc[a][b][r]);
     }
   };
 
@@ -297,28 +344,38 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(
   }
   lds_barrier();
   const float* const from = reinterpret_cast<const float*>(kw == 0 ? area[0] : kw == 1 ? area[1] : kw == 2 ? area[2] : area[3]) + 4 * lane;
-  const int m = m0 + 32 * (kw & 1) + lcol;
+  const int mt = m0 + 32 * (kw & 1), nt = n0 + 64 * cw + 32 * (kw >> 1);
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     f32x4 v = *reinterpret_cast<const f32x4*>(from + 256 * q);
 #pragma unroll
     for (int k = 1; k < KW; ++k) v += *reinterpret_cast<const f32x4*>(from + 1024 * k + 256 * q);
-    const int n = n0 + 64 * cw + 32 * (kw >> 1) + 8 * q + 4 * h;
+    // Four features of one row; NF4: four rows of one feature.
     uint16_t out[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      const int n = NF ? nt + lcol : nt + 8 * q + 4 * h + i;
       out[i] = E::from_f32(v[i]);
-      if (bias != nullptr && n + i < N) out[i] = E::from_f32(E::to_f32(out[i]) + E::to_f32(bias[n + i]));
+      if (bias != nullptr && n < N) out[i] = E::from_f32(E::to_f32(out[i]) + E::to_f32(bias[n]));
     }
-    if (m < M) {
-      uint16_t* const yrow = y + static_cast<size_t>(m) * N;
-      if (vec_out && n + 3 < N) {
-        *reinterpret_cast<u32x2*>(yrow + n) = u32x2{static_cast<uint32_t>(out[0]) | (static_cast<uint32_t>(out[1]) << 16),
-                                                    static_cast<uint32_t>(out[2]) | (static_cast<uint32_t>(out[3]) << 16)};
-      } else {
+    if constexpr (NF) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (n + i < N) yrow[n + i] = out[i];
+      for (int i = 0; i < 4; ++i) {
+        const int m = mt + 8 * q + 4 * h + i;
+        if (m < M && nt + lcol < N) y[static_cast<size_t>(m) * args.y_stride + nt + lcol] = out[i];
+      }
+    } else {
+      const int m = mt + lcol, n = nt + 8 * q + 4 * h;
+      if (m < M) {
+        uint16_t* const yrow = y + static_cast<size_t>(m) * args.y_stride;
+        if (vec_out && n + 3 < N) {
+          *reinterpret_cast<u32x2*>(yrow + n) = u32x2{static_cast<uint32_t>(out[0]) | (static_cast<uint32_t>(out[1]) << 16),
+                                                      static_cast<uint32_t>(out[2]) | (static_cast<uint32_t>(out[3]) << 16)};
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (n + i < N) yrow[n + i] = out[i];
+        }
       }
     }
   }
@@ -332,29 +389,36 @@ bool int4_mid_preferred(int M, int N) {
 }
 
 template <int DT, Scales SC>
-static void launch(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero, const void* bias,
-                   void* y, int M, int N, int K, int gshift, hipStream_t stream) {
-  const int tiles = ((M + mid::BM - 1) / mid::BM) * ((N + mid::BN - 1) / mid::BN);
-  hipLaunchKernelGGL((int4_mid_kernel<DT, SC>), dim3(tiles), dim3(mid::THREADS), 0, stream, static_cast<const uint16_t*>(x),
-                     packed, static_cast<const uint16_t*>(scale), zero, static_cast<const uint16_t*>(bias),
-                     static_cast<uint16_t*>(y), M, N, K, gshift);
+static void launch(const MidArgs& a, hipStream_t stream) {
+  const int tiles = ((a.M + mid::BM - 1) / mid::BM) * ((a.N + mid::BN - 1) / mid::BN);
+  hipLaunchKernelGGL((int4_mid_kernel<DT, SC>), dim3(tiles), dim3(mid::THREADS), 0, stream, a);
 }
 
 template <int DT>
-static void launch_scales(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero, const void* bias,
-                          void* y, int M, int N, int K, int G, hipStream_t stream) {
-  const int gshift = __builtin_ctz(static_cast<unsigned>(G));
-  const bool whole = (reinterpret_cast<uintptr_t>(scale) | reinterpret_cast<uintptr_t>(zero)) % 4 == 0;
-  if (G == 128 && K % 1024 == 0 && whole) launch<DT, Scales::BLOCK>(x, packed, scale, zero, bias, y, M, N, K, gshift, stream);
-  else if (G >= 64) launch<DT, Scales::ONE>(x, packed, scale, zero, bias, y, M, N, K, gshift, stream);
-  else launch<DT, Scales::TWO>(x, packed, scale, zero, bias, y, M, N, K, gshift, stream);
+static void launch_scales(const MidArgs& a, int G, hipStream_t stream) {
+  const bool whole = (reinterpret_cast<uintptr_t>(a.scale) | reinterpret_cast<uintptr_t>(a.zero)) % 4 == 0;
+  if (G == 128 && a.K % 1024 == 0 && whole) launch<DT, Scales::BLOCK>(a, stream);
+  else if (G >= 64) launch<DT, Scales::ONE>(a, stream);
+  else launch<DT, Scales::TWO>(a, stream);
 }
 
 LnqStatus launch_int4_mid(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero, const void* bias,
                           void* y, int M, int N, int K, int G, int dtype, hipStream_t stream) {
-  if (dtype == LNQ_BF16) launch_scales<LNQ_BF16>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
-  else launch_scales<LNQ_F16>(x, packed, scale, zero, bias, y, M, N, K, G, stream);
+  const MidArgs a{static_cast<const uint16_t*>(x), packed, scale, zero, static_cast<const uint16_t*>(bias),
+                  static_cast<uint16_t*>(y), M, N, K, __builtin_ctz(static_cast<unsigned>(G)), K, N, {}};
+  if (dtype == LNQ_BF16) launch_scales<LNQ_BF16>(a, G, stream);
+  else launch_scales<LNQ_F16>(a, G, stream);
   return launched("int4_mid");
+}
+
+LnqStatus launch_nf4_mid(const void* x, int x_stride, const uint8_t* codes, const float* absmax, const void* bias, void* y,
+                         int y_stride, int M, int N, int K, int block, const stream::Planes& planes, int dtype,
+                         hipStream_t stream) {
+  const MidArgs a{static_cast<const uint16_t*>(x), codes, absmax, codes, static_cast<const uint16_t*>(bias),
+                  static_cast<uint16_t*>(y), M, N, K, __builtin_ctz(static_cast<unsigned>(block)), x_stride, y_stride, planes};
+  if (dtype == LNQ_BF16) launch<LNQ_BF16, Scales::NF4>(a, stream);
+  else launch<LNQ_F16, Scales::NF4>(a, stream);
+  return launched("nf4_mid");
 }
 
 }  // namespace lnq

@@ -301,6 +301,11 @@ __global__ __launch_bounds__(256) void nf4_repack_kernel(const uint8_t* __restri
   }
 }
 
+// Defined in int4_mid.hip.
+LnqStatus launch_nf4_mid(const void* x, int x_stride, const uint8_t* codes, const float* absmax, const void* bias, void* y,
+                         int y_stride, int M, int N, int K, int block, const stream::Planes& planes, int dtype,
+                         hipStream_t stream);
+
 namespace {
 
 uint32_t bf16_pattern(float f) {
@@ -328,6 +333,25 @@ bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64
                   int64_t y_stride) {
   return rows > (in_features <= nf4::UNIT * nf4::THREADS ? 4 : 2) && rows <= INT32_MAX && (block == 32 || block == 64 || block % 128 == 0) &&
          in_features <= stream::MAX_K && x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
+}
+
+// Whether the 64 x 128 tiles of int4_mid.hip take the call: blocks that hold whole 64-input
+// chunks, a tile a CU at most, and rows whose passes of 32 on the streaming kernel cost more
+// (us, estimates within a fifth of block 64 measured, streaming / tiles: 4096 -> 14336 32 rows
+// 18.7 / 29, 64 rows 32.5 / 29.7, 96 rows 46.9 / 31.2; 14336 -> 4096 64 rows 38.3 / 86, 96 rows
+// 55.8 / 86.5; 3072 -> 9216 32 rows 15.7 / 23, 64 rows 28.5 / 23.1; 4096 -> 4096 96 rows
+// 22.5 / 28.6). Past 96 rows always: the alternative then is the widened weight and its
+// product (128 rows 70.7 / 32.1, 116.2 / 87.0, 40.7 / 24.4, 37.0 / 28.8), not this kernel's
+// fifth pass.
+bool mid_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
+               const void* codes) {
+  if (rows > INT32_MAX || block < 64 || (block & (block - 1)) != 0 || !aligned(codes, 16) || y_stride > INT32_MAX ||
+      x_stride >= (int64_t{1} << 23) || (rows + 63) * x_stride >= (int64_t{1} << 30))
+    return false;
+  if (((rows + 63) / 64) * ((out_features + 127) / 128) > compute_units()) return false;
+  const double tiles = 6 + 1.45 * ((in_features + 255) / 256);
+  const double pass = 3 + static_cast<double>(out_features) * in_features / 4.4e6;
+  return rows > 96 || tiles < ((rows + 31) / 32) * pass;
 }
 
 template <int DT>
@@ -419,6 +443,10 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
   const int slots = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
   const Nf4Planes planes = planes_for(dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mid_takes(rows, out_features, in_features, block, x_stride, y_stride, codes))
+    return launch_nf4_mid(x, static_cast<int>(x_stride), codes, absmax, bias, y, static_cast<int>(y_stride),
+                          static_cast<int>(rows), static_cast<int>(out_features), static_cast<int>(in_features),
+                          static_cast<int>(block), planes, dtype, s);
   if (stream_takes(rows, out_features, in_features, block, x_stride, y_stride)) {
     stream::Args a{};
     a.x = static_cast<const uint16_t*>(x);

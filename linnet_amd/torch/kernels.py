@@ -845,9 +845,20 @@ def nf4_gemv_fits(rows: int, in_features: int, block: int, dtype: torch.dtype) -
             and 0 < in_features <= NF4_GEMV_MAX_IN)
 
 
-# Rows up to which `nf4_linear` reads the stored weight at all: past NF4_GEMV_ROWS on the
-# streaming kernel, 32 rows a pass.
+# Rows up to which `nf4_linear` reads the stored weight at any shape: past NF4_GEMV_ROWS on
+# the streaming kernel, 32 rows a pass, or in tiles. us, block 64, stored / widened at 96 rows:
+# 4096 -> 14336 31.2 / 70.4, 14336 -> 4096 55.8 / 103.2, 2048 -> 2048 15.0 / 16.3.
 NF4_STREAM_ROWS = 96
+# Past those, where 64 x 128 tiles give no compute unit a second one and win by estimates of
+# both (us, from these; 128 rows: 4096 -> 14336 32.1 / 71.6, 4096 -> 4096 28.8 / 37.7, 14336 -> 4096
+# 87.0 / 114.4, but 2048 -> 2048 17.1 / 16.4; 200 rows 4096 -> 14336, 448 tiles: 76 widened).
+NF4_TILES = 256
+
+
+def _nf4_tiles_fit(rows: int, out_features: int, in_features: int, block: int) -> bool:
+    tiles = -(-rows // 64) * -(-out_features // 128)
+    return (block >= 64 and block & (block - 1) == 0 and tiles <= NF4_TILES
+            and 6 + 1.45 * in_features / 256 < 0.9 * (11 + out_features * in_features * 1e-6 + 0.002 * in_features))
 
 
 def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor | None, rows: int, block: int) -> bool:
@@ -858,7 +869,7 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
     out_features, in_features = codes.shape[0], 2 * codes.shape[1]
     if nf4_gemv_fits(rows, in_features, block, x.dtype):
         return True
-    if not (x.dtype in _HALF and rows <= NF4_STREAM_ROWS and (block in (32, 64) or block % 128 == 0)
+    if not (x.dtype in _HALF and (rows <= NF4_STREAM_ROWS or _nf4_tiles_fit(rows, out_features, in_features, block)) and (block in (32, 64) or block % 128 == 0)
             and in_features % block == 0 and 0 < in_features <= NF4_GEMV_MAX_IN
             and out_features * in_features < 1 << 32):
         return False

@@ -125,6 +125,28 @@ def test_nf4(rows: int, out: int, width: int, block: int, dtype: torch.dtype) ->
     _check(got, x, w, np.abs(w), bias)
 
 
+@pytest.mark.parametrize(("rows", "out", "width", "block", "dtype"), [
+    (97, 7003, 1856, 64, BF16),  # 29 chunks of 64: the last step holds one; a partial column tile
+    (130, 4097, 2048, 128, F16),  # odd rows of y, a block over two chunks
+    (64, 14336, 512, 64, BF16),  # the tiles at 33..96 rows
+    (257, 5000, 768, 256, BF16),
+])
+def test_nf4_tiles(rows: int, out: int, width: int, block: int, dtype: torch.dtype) -> None:
+    print(f"nf4 tiles rows={rows} out={out} in={width} block={block} {dtype}", flush=True)
+    rng = np.random.default_rng(rows)
+    codes = rng.integers(0, 256, (out, width // 2)).astype(np.uint8)
+    absmax = (rng.random((out, width // block)) * 0.1 + 0.01).astype(np.float32)
+    x = _x(rows, width, dtype)
+    bias = _x(1, out, dtype)[0] if rows % 2 else None
+    strided = torch.zeros(rows, width + 8, dtype=dtype, device=DEV)
+    strided[:, :width] = x.to(DEV)
+    got = kernels.nf4_linear(strided[:, :width], torch.from_numpy(codes).to(DEV), torch.from_numpy(absmax).to(DEV), block,
+                             None if bias is None else bias.to(DEV))
+    values = torch.from_numpy(quant.NF4_VALUES.copy()).to(dtype).double().numpy()
+    w = values[np.stack([codes & 15, codes >> 4], axis=-1).reshape(out, width)] * np.repeat(absmax.astype(np.float64), block, 1)
+    _check(got, x, w, np.abs(w), bias)
+
+
 @pytest.mark.parametrize("dtype", [BF16, F16])
 @pytest.mark.parametrize(("rows", "chosen", "count", "out", "width", "skew"), [
     (40, 4, 8, 1500, 2880, False),  # In ends inside a step; 20 pairs an expert on average
