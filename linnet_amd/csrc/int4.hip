@@ -766,6 +766,8 @@ static int choose_int4_kernel(int M, int N, int K, int G, int dtype, int kernel,
     // <= 4096 the two are level from 16 to 32 rows (N = 4096: 7.2 / 7.5 us at
     // 16, 11.3 / 11.2 at 32) and the skinny kernel is ahead at 64 (18.6 against
     // 22.5 for two 32-row launches).
+    // GEMV at 5..16 rows and SKINNY stand for the streaming kernel (launch_few_tokens,
+    // lnq_int4_linear), ahead of both there.
     const bool wide = N >= 6144;
     const bool few = M <= 6;
     if (gemv_ok && (M == 1 || few || (M > 4 && wide))) return LNQ_KERNEL_GEMV;

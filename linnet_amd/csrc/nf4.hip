@@ -7,8 +7,9 @@
 // Three kernels:
 // - nf4_dequant_kernel: the weight in T, the f32 product of the code's value and
 //   the scale rounded once (`dequantize_nf4`, quant.linnet:180-187), bit for bit.
-// - nf4_gemv_kernel: y = x W^T (+ bias) for up to 8 rows of x, the weight read
-//   once from HBM as it is stored. NF4's values are no affine function of the
+// - nf4_gemv_kernel: y = x W^T (+ bias), up to 8 rows of x a pass, the weight read
+//   once from HBM as it is stored (lnq_nf4_linear's fewest rows, and the blocks the
+//   streaming product and the tiles do not take: stream_takes, mid_takes). NF4's values are no affine function of the
 //   code, so the widening is a table lookup done in registers: the 16 values'
 //   16-bit patterns (bf16 or f16, x's type) are held as two 16-byte planes (low
 //   bytes, high bytes) in 8 SGPRs, and v_perm_b32 selects four codes' bytes from

@@ -828,11 +828,11 @@ def nf4_dequantize(codes: torch.Tensor, absmax: torch.Tensor, block: int, dtype:
     return out
 
 
-# Rows of x up to which `nf4_linear` reads the stored weight with the NF4 GEMV
-# (8 rows a pass over the weight up to In = 8192, 4 past it); more rows widen
-# the weight and multiply. bf16, graph-replayed, against 57 us for the widened
-# weight and its product: 4096 -> 14336 at 1 / 8 / 16 rows 12.0 / 21.6 / 41.8
-# us; 14336 -> 4096 at 1 / 8 / 12 rows 11.5 / 35.3 / 52.5 us.
+# Rows of x up to which `nf4_linear` reads the stored weight for every block of a multiple
+# of 16 inputs (`lnq_nf4_linear`: its GEMV, 8 rows a pass up to In = 8192 and 4 past it, or
+# the streaming kernel). The GEMV, bf16, graph-replayed, against 57 us for the widened weight
+# and its product: 4096 -> 14336 at 1 / 8 / 16 rows 12.0 / 21.6 / 41.8 us; 14336 -> 4096 at
+# 1 / 8 / 12 rows 11.5 / 35.3 / 52.5 us.
 NF4_GEMV_ROWS = 16
 NF4_GEMV_ROWS_WIDE = 8  # In > 8192
 NF4_GEMV_MAX_IN = 32768
@@ -909,8 +909,8 @@ def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: 
 
 def nf4_linear(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: int,
                bias: torch.Tensor | None = None) -> torch.Tensor:
-    """`linear_nf4` (`stdlib/quant.linnet:189-199`): up to `NF4_GEMV_ROWS` rows of
-    bf16 / f16 x (`NF4_GEMV_ROWS_WIDE` past In = 8192) on the NF4 GEMV; otherwise the weight widened by the HIP
+    """`linear_nf4` (`stdlib/quant.linnet:189-199`): bf16 / f16 x of few rows times the
+    stored weight (`_nf4_reads_stored`); otherwise the weight widened by the HIP
     dequantize kernel, then multiplied in x's type (the reference's own body)."""
     _on_gpu("nf4_linear", x, codes, absmax, bias)
     out_features, in_features = _nf4_operands("nf4_linear", codes, absmax, block)
