@@ -59,7 +59,8 @@ __global__ __launch_bounds__((64 * mm8s::Tile<BM, BN>::WAVES), 2) void mm8_small
   using Op = typename std::conditional<FP8, i32x8, i32x4>::type;
   using Acc = typename std::conditional<FP8, f32x16, i32x16>::type;
   // A stage array each (the compiler tracks loads into LDS by variable).
-  constexpr int STAGE = (BM + BN) * BK;
+  constexpr int OPERANDS = (BM + BN) * BK;
+  constexpr int STAGE = OPERANDS + (BLK ? NW * 512 : 0);  // then each wave's scales
   __shared__ __attribute__((aligned(16))) uint8_t S0[STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t S1[STAGE];
   __shared__ __attribute__((aligned(16))) uint8_t S2[S > 2 ? STAGE : 16];
@@ -119,39 +120,46 @@ __global__ __launch_bounds__((64 * mm8s::Tile<BM, BN>::WAVES), 2) void mm8_small
       aoff[kk][j] = static_cast<uint32_t>((wm * FA * 32 + lrow) * BK) + col;
       boff[kk][j] = static_cast<uint32_t>(BM * BK + (wn * FB * 32 + lrow) * BK) + col;
     }
-  int xs_row[BLK ? FA : 1];
-  // The block form's scales, S - 1 steps ahead like the operands and by vector loads (a
-  // scalar load would share the counter that the LDS reads of a step wait for).
-  float sx[S][BLK ? FA : 1], sw[S];
-  const uint32_t ws_row = static_cast<uint32_t>((n0 + wn * FB * 32) / 128) * static_cast<uint32_t>(steps);
-  const __amdgpu_buffer_rsrc_t rw =
-      buffer_rsrc(scale, static_cast<uint32_t>((N + 127) / 128) * static_cast<uint32_t>(steps) * 4u);
-  if constexpr (BLK) {
-#pragma unroll
-    for (int a = 0; a < FA; ++a) xs_row[a] = min(m0 + (wm * FA + a) * 32 + lrow, M - 1);
-  }
-  auto load_scales = [&](int ks, int slot) {
+  // The block form's scales of a step ride with its operands, by loads into LDS of the wave's
+  // own: its rows' (lane l row l of the wave's; rows past M read row M - 1) and, in every
+  // lane, that of its columns' block. (Loads into registers, which nothing ties to their
+  // place, were moved past the operands' and broke the count that a step waits by. Products
+  // alone, us, so -> now: 256 rows 8192 -> 28672 71 -> 61, 128 rows 45.4 -> 44.5, 4096 -> 14336
+  // 16.8 both; 2048 -> 2048 5.9 -> 6.5, two more LDS loads and reads in each short step.)
+  const uint32_t sx_off = static_cast<uint32_t>(min(m0 + wm * FA * 32 + lane, M - 1)) * 4u;
+  const uint32_t sw_off = static_cast<uint32_t>((n0 + wn * FB * 32) / 128) * static_cast<uint32_t>(steps) * 4u;
+  const uint32_t sx_bytes = static_cast<uint32_t>(M) * 4u;
+  const uint32_t sw_bytes = static_cast<uint32_t>((N + 127) / 128) * static_cast<uint32_t>(steps) * 4u;
+  auto load_scales = [&](int ks, uint8_t* st) {
     if constexpr (BLK) {
-      const int k = min(ks, steps - 1);
-#pragma unroll
-      for (int a = 0; a < FA; ++a) sx[slot][a] = x_scale[static_cast<size_t>(k) * xs_stride + xs_row[a]];
-      sw[slot] = __builtin_bit_cast(
-          float, static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(rw, (ws_row + k) * 4u, 0, 0)));
-      __builtin_amdgcn_sched_barrier(0);
+      const bool in = ks < steps;
+      const int k = in ? ks : 0;
+      uint8_t* const to = st + OPERANDS + wave * 512;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          buffer_rsrc(x_scale + static_cast<size_t>(k) * xs_stride, in ? sx_bytes : 0u), (lds_ptr)to, 4, sx_off, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(buffer_rsrc(scale, in ? sw_bytes : 0u), (lds_ptr)(to + 256), 4, sw_off,
+                                               k * 4, 0, 0);
     }
   };
-  constexpr int LOADS = LA + LB + (BLK ? FA + 1 : 0);  // of a wave a step
+  constexpr int LOADS = LA + LB + (BLK ? 2 : 0);  // of a wave a step
 
-  auto step = [&](int ks, int slot, int nslot, const uint8_t* st, uint8_t* next) {
+  auto step = [&](int ks, const uint8_t* st, uint8_t* next) {
     // This wave's loads of step ks have landed (those of the S - 2 steps after it may be in
     // flight); past the barrier every wave's have, and every wave is done with step
     // ks - 1's stage, which step ks + S - 1 fills.
     wait_vm<(S - 2) * LOADS>();
     __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    load_scales(ks + S - 1, nslot);
     load(ks + S - 1, next);
+    load_scales(ks + S - 1, next);
     __builtin_amdgcn_sched_barrier(0);
     Acc part[BLK ? FA : 1][BLK ? FB : 1];
+    float sx[FA], sw = 0.f;
+    if constexpr (BLK) {
+      const float* const from = reinterpret_cast<const float*>(st + OPERANDS + wave * 512);
+      sw = from[64];
+#pragma unroll
+      for (int a = 0; a < FA; ++a) sx[a] = from[32 * a + lrow];
+    }
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       Op af[FA], bf[FB];
@@ -190,7 +198,7 @@ __global__ __launch_bounds__((64 * mm8s::Tile<BM, BN>::WAVES), 2) void mm8_small
     if constexpr (BLK) {
 #pragma unroll
       for (int a = 0; a < FA; ++a) {
-        const float f = sx[slot][a] * sw[slot];
+        const float f = sx[a] * sw;
 #pragma unroll
         for (int b = 0; b < FB; ++b)
 #pragma unroll
@@ -202,15 +210,15 @@ __global__ __launch_bounds__((64 * mm8s::Tile<BM, BN>::WAVES), 2) void mm8_small
   uint8_t* const st[4] = {S0, S1, S2, S3};
 #pragma unroll
   for (int j = 0; j < S - 1; ++j) {
-    load_scales(j, j);
     load(j, st[j]);
+    load_scales(j, st[j]);
     __builtin_amdgcn_sched_barrier(0);
   }
   for (int ks = 0; ks < steps; ks += S) {
 #pragma unroll
     for (int j = 0; j < S; ++j) {
       if (ks + j >= steps) break;
-      step(ks + j, j, (j + S - 1) % S, st[j], st[(j + S - 1) % S]);
+      step(ks + j, st[j], st[(j + S - 1) % S]);
     }
   }
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
