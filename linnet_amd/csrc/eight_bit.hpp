@@ -51,7 +51,11 @@ __host__ __device__ inline uint32_t f32_to_e4m3(float v) {
 // sums into a partial tile P, which is added to the tile scaled by
 // x_scale[m, step] * scale[n / 128, step] once the step's MFMAs are done: the
 // block-wise product `torch._scaled_mm` computes for the reference. 128-column
-// tiles only (a wave's 64 columns lie in one weight block).
+// tiles only (a wave's 64 columns lie in one weight block). The scales come through
+// LDS two steps ahead, as the operands do: read as their step began, the rows' by a
+// global load and the block's by a scalar one, whose counter the operand reads share,
+// they held the step up (products alone, us, so -> now: 777 rows 4096 -> 14336 68.3 ->
+// 62.7 and 8192 -> 28672 287 -> 244, 2048 rows 14336 -> 4096 122 -> 114).
 namespace mm8 {
 constexpr int BM = 256;
 constexpr int BK = 128;  // bytes (= elements) per step
@@ -117,13 +121,14 @@ __global__ __launch_bounds__(mm8::THREADS, 1) void mm8_kernel(
   using Acc = typename std::conditional<FP8, f32x16, i32x16>::type;
   // Stages per operand: three (loads two steps ahead) where they fit in LDS.
   constexpr int S = BN == 256 ? 2 : 3;
-  constexpr int LPW = 4 + BLOADS;  // loads of a wave per step
+  constexpr int LPW = 4 + BLOADS + (BLK ? 2 : 0);  // loads of a wave per step
+  constexpr int BSTAGE = BN * BK + (BLK ? 8 * 512 : 0);  // BLK: then each wave's scales
   __shared__ __attribute__((aligned(16))) uint8_t A0[BM * BK];
   __shared__ __attribute__((aligned(16))) uint8_t A1[BM * BK];
   __shared__ __attribute__((aligned(16))) uint8_t A2[S > 2 ? BM * BK : 16];
-  __shared__ __attribute__((aligned(16))) uint8_t B0[BN * BK];
-  __shared__ __attribute__((aligned(16))) uint8_t B1[BN * BK];
-  __shared__ __attribute__((aligned(16))) uint8_t B2[S > 2 ? BN * BK : 16];
+  __shared__ __attribute__((aligned(16))) uint8_t B0[BSTAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t B1[BSTAGE];
+  __shared__ __attribute__((aligned(16))) uint8_t B2[S > 2 ? BSTAGE : 16];
   if constexpr (!BLK) LNQ_MFMA_IN_AGPRS();
 
   const int tid = threadIdx.x;
@@ -170,19 +175,24 @@ __global__ __launch_bounds__(mm8::THREADS, 1) void mm8_kernel(
     for (int b = 0; b < FB; ++b)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[a][b][r] = 0;
-  // Block scales: the step's partial tile, the rows' scales of the step (lane
-  // row m = l % 32 of fragment a; rows past M read row M - 1; loaded as the step
-  // starts, they land with its operands), and the weight block row of this
-  // wave's columns.
+  // Block scales: the step's partial tile, and the scales of a step, which ride with its
+  // operands by loads into LDS of the wave's own: its rows' (lane l row l of the wave's
+  // 64; rows past M read row M - 1) and, in every lane, that of its columns' weight block.
   Acc part[BLK ? FA : 1][BLK ? FB : 1];
-  float sx[BLK ? FA : 1];
-  int xs_row[BLK ? FA : 1];
-  const int kblocks = K / BK;
-  const float* wscale = scale + static_cast<size_t>((n0 + wn * FB * 32) / 128) * kblocks;
-  if constexpr (BLK) {
-#pragma unroll
-    for (int a = 0; a < FA; ++a) xs_row[a] = min(m0 + wm * FA * 32 + a * 32 + (lane & 31), M - 1);
-  }
+  const uint32_t sx_off = static_cast<uint32_t>(min(m0 + wm * FA * 32 + lane, M - 1)) * 4u;
+  const uint32_t sw_off = static_cast<uint32_t>((n0 + wn * FB * 32) / 128) * static_cast<uint32_t>(steps) * 4u;
+  auto load_x_scales = [&](uint8_t* b, int ks) {
+    const bool in = ks < steps;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        buffer_rsrc(x_scale + static_cast<size_t>(in ? ks : 0) * xs_stride, in ? static_cast<uint32_t>(M) * 4u : 0u),
+        (lds_ptr)(b + BN * BK + wave * 512), 4, sx_off, 0, 0, 0);
+  };
+  auto load_w_scale = [&](uint8_t* b, int ks) {
+    const bool in = ks < steps;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        buffer_rsrc(scale, in ? static_cast<uint32_t>(N / 128) * static_cast<uint32_t>(steps) * 4u : 0u),
+        (lds_ptr)(b + BN * BK + wave * 512 + 256), 4, sw_off, in ? ks * 4 : 0, 0, 0);
+  };
 
   const int lrow = lane & 31;
   const int lk = lane >> 5;
@@ -262,14 +272,17 @@ __global__ __launch_bounds__(mm8::THREADS, 1) void mm8_kernel(
       for (int i = 0; i < LPW; ++i)
         if (s == (i * NMF) / LPW) {
           if (i < 4) load_a(al, qa, k0, i);
-          else load_b(bl, qb, k0, i - 4);
+          else if (i < 4 + BLOADS) load_b(bl, qb, k0, i - 4);
+          else if (i == 4 + BLOADS) load_x_scales(bl, ks + S - 1);
+          else load_w_scale(bl, ks + S - 1);
         }
     };
+    float sx[BLK ? FA : 1], sw = 0.f;
     if constexpr (BLK) {
+      const float* const from = reinterpret_cast<const float*>(bc + BN * BK + wave * 512);
+      sw = from[64];
 #pragma unroll
-      for (int a = 0; a < FA; ++a) {
-        sx[a] = x_scale[static_cast<size_t>(ks) * xs_stride + xs_row[a]];
-      }
+      for (int a = 0; a < FA; ++a) sx[a] = from[32 * a + lrow];
     }
 #pragma unroll
     for (int kk = 0; kk + 1 < KK; ++kk)
@@ -279,7 +292,6 @@ __global__ __launch_bounds__(mm8::THREADS, 1) void mm8_kernel(
     __builtin_amdgcn_s_barrier();
     region((KK - 1) & 1, an, bn, 0, [&](int) {}, KK == 1);
     if constexpr (BLK) {
-      const float sw = wscale[ks];
 #pragma unroll
       for (int a = 0; a < FA; ++a) {
         const float f = sx[a] * sw;
@@ -304,6 +316,10 @@ __global__ __launch_bounds__(mm8::THREADS, 1) void mm8_kernel(
     for (int i = 0; i < 4; ++i) load_a(a, in ? ra : rnull, in ? j * BK : 0, i);
 #pragma unroll
     for (int i = 0; i < BLOADS; ++i) load_b(b, in ? rb : rnull, in ? j * BK : 0, i);
+    if constexpr (BLK) {
+      load_x_scales(b, j);
+      load_w_scale(b, j);
+    }
   }
   if constexpr (S == 2) __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   else __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * LPW) : "memory");

@@ -249,9 +249,11 @@ def test_mm8_small_tiles(rows: int, out: int, width: int, fp8: bool) -> None:
         assert torch.equal(mm(q, w, xs * 1e-2, ws * 1e-2, dtype), mm(q, w, xs * 1e-2, ws * 1e-2, dtype, tile_n=128))
 
 
-@pytest.mark.parametrize(("rows", "out", "width"), [(33, 128, 128), (65, 4096, 640), (129, 2048, 1152), (200, 7168, 2048), (500, 640, 4096)])
+@pytest.mark.parametrize(("rows", "out", "width"), [(33, 128, 128), (65, 4096, 640), (129, 2048, 1152), (200, 7168, 2048), (500, 640, 4096),
+                                                    # The 256-row form: one step to five of its three stages.
+                                                    (4993, 4096, 128), (4737, 4096, 256), (4993, 4096, 640)])
 def test_fp8_block_small_tiles(rows: int, out: int, width: int) -> None:
-    """Small tiles' block fold. Whole codes up to 8 and scales of powers of two: every sum is
+    """The block fold of both tiles. Whole codes up to 8 and scales of powers of two: every sum is
     exact in f32, so the result is the f64 product rounded once."""
     g = torch.Generator().manual_seed(rows)
     q, w = (torch.randint(-8, 9, (n, width), generator=g).float().to(torch.float8_e4m3fn) for n in (rows, out))
