@@ -350,13 +350,19 @@ __global__ __launch_bounds__(mid::THREADS, 2) void int4_mid_kernel(MidArgs args)
     f32x4 v = *reinterpret_cast<const f32x4*>(from + 256 * q);
 #pragma unroll
     for (int k = 1; k < KW; ++k) v += *reinterpret_cast<const f32x4*>(from + 1024 * k + 256 * q);
-    // Four features of one row; NF4: four rows of one feature.
+    // Four features of one row, the rounded product plus the bias rounded again (the
+    // reference's order); NF4: four rows of one feature, rounded once, as its other kernels do.
     uint16_t out[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int n = NF ? nt + lcol : nt + 8 * q + 4 * h + i;
-      out[i] = E::from_f32(v[i]);
-      if (bias != nullptr && n < N) out[i] = E::from_f32(E::to_f32(out[i]) + E::to_f32(bias[n]));
+      const bool add = bias != nullptr && n < N;
+      if constexpr (NF) {
+        out[i] = E::from_f32(add ? v[i] + E::to_f32(bias[n]) : v[i]);
+      } else {
+        out[i] = E::from_f32(v[i]);
+        if (add) out[i] = E::from_f32(E::to_f32(out[i]) + E::to_f32(bias[n]));
+      }
     }
     if constexpr (NF) {
 #pragma unroll

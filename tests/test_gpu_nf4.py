@@ -270,3 +270,31 @@ def test_widened_where_the_stored_product_refuses(form: str) -> None:
     if form == "grad":
         got.sum().backward()
         assert x.grad is not None and bool(x.grad.abs().sum() > 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(("rows", "out_features", "in_features"), [
+    (2, 72, 512),  # the GEMV
+    (24, 72, 512),  # the streaming kernel
+    (97, 7003, 1856)])  # the 64 x 128 tiles
+def test_a_bias_is_added_before_the_only_rounding(dtype: torch.dtype, rows: int, out_features: int,
+                                                  in_features: int) -> None:
+    """Biases near the products' negatives, so that the sum is small beside the product: the
+    result is within half a unit in the last place of the sum (not of the product), plus 16 f32
+    units of the magnitudes added."""
+    print(f"nf4 bias rows {rows} {out_features}x{in_features} {dtype}", flush=True)
+    codes, absmax = _layer(out_features, in_features, 64, rows)
+    x = torch.randn(1, in_features, generator=torch.Generator().manual_seed(rows)).expand(rows, -1).to(dtype)
+    values = torch.from_numpy(quant.NF4_VALUES.copy()).to(dtype).double().numpy()
+    q = np.stack([codes & 15, codes >> 4], axis=-1).reshape(out_features, in_features)
+    w = values[q] * np.repeat(absmax.astype(np.float64), 64, axis=1)
+    xd = x[:1].double().numpy()
+    product, mag = xd @ w.T, np.abs(xd) @ np.abs(w).T
+    b = torch.from_numpy(-0.97 * product[0]).to(dtype)
+    got = kernels.nf4_linear(x.to(DEV), torch.from_numpy(codes).to(DEV), torch.from_numpy(absmax).to(DEV), 64, b.to(DEV))
+    ref = product + b.double().numpy()
+    half_ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    bound = half_ulp * np.abs(ref) + 2.0 ** -20 * (mag + np.abs(b.double().numpy())) + 2.0 ** -24
+    err = np.abs(got.double().cpu().numpy() - ref)
+    print(f"max err / bound {float((err / bound).max()):.3f}", flush=True)
+    assert np.all(err <= bound)
