@@ -480,6 +480,14 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
                                  int64_t out_features, int64_t in_features, int64_t block,
                                  int32_t dtype, void* stream);
 
+/* The kernel lnq_nf4_linear takes on the current device, for rows of x x_stride elements
+ * apart and 16-byte aligned codes. No counterpart in the reference. */
+#define LNQ_NF4_GEMV 1
+#define LNQ_NF4_STREAM 2
+#define LNQ_NF4_TILES 3
+LNQ_API LnqStatus lnq_nf4_linear_plan(int64_t rows, int64_t x_stride, int64_t out_features,
+                                      int64_t in_features, int64_t block, int32_t* chosen);
+
 /* A bitsandbytes 4-bit NF4 layer as Nf4Linear holds it: `codes` = `packed`
  * ([out * in / 2] bytes, the first code of a pair in the high nibble) with each
  * byte's nibbles swapped; `absmax` [out * in / block] f32 = `absmax_in` (f32)

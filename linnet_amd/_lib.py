@@ -63,6 +63,7 @@ SIGNATURES: dict[str, list[object]] = {
     "lnq_mxfp4_experts": [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i32, _p],
     "lnq_nf4_dequant": [_p, _p, _p, _i64, _i64, _i64, _i32, _p],
     "lnq_nf4_linear": [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p],
+    "lnq_nf4_linear_plan": [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i32)],
     "lnq_nf4_repack": [_p, _p, _p, _p, _i64, _f32, _p, _p, _i64, _i64, _i64, _p],
     "lnq_rmsnorm": [_p, _p, _p, _p, _i64, _i64, ctypes.c_float, _p],
     "lnq_rmsnorm_tiles": [_p, _p, _p, _p, _i64, _i64, ctypes.c_float, _p],

@@ -337,7 +337,10 @@ bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64
 }
 
 // Whether the 64 x 128 tiles of int4_mid.hip take the call: blocks that hold whole 64-input
-// chunks, a tile a CU at most, and rows whose passes of 32 on the streaming kernel cost more
+// chunks, a tile a CU at most, and more than 16 rows, whose passes of 32 on the streaming kernel
+// cost more (up to 16 rows that kernel's narrower forms and the GEMV cost less than such a pass:
+// 4096 -> 28672 1 / 4 / 8 / 16 rows 18.2 / 25.7 / 26.3 / 27.2 on them, 30 in tiles; 24 rows 33.7
+// / 31.5; 8192 -> 28672 1 / 16 rows 33.1 / 46.1, 55)
 // (us, estimates within a fifth of block 64 measured, streaming / tiles: 4096 -> 14336 32 rows
 // 18.7 / 29, 64 rows 32.5 / 29.7, 96 rows 46.9 / 31.2; 14336 -> 4096 64 rows 38.3 / 86, 96 rows
 // 55.8 / 86.5; 3072 -> 9216 32 rows 15.7 / 23, 64 rows 28.5 / 23.1; 4096 -> 4096 96 rows
@@ -346,7 +349,7 @@ bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64
 // fifth pass.
 bool mid_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
                const void* codes) {
-  if (rows > INT32_MAX || block < 64 || (block & (block - 1)) != 0 || !aligned(codes, 16) || y_stride > INT32_MAX ||
+  if (rows <= 16 || rows > INT32_MAX || block < 64 || (block & (block - 1)) != 0 || !aligned(codes, 16) || y_stride > INT32_MAX ||
       x_stride >= (int64_t{1} << 23) || (rows + 63) * x_stride >= (int64_t{1} << 30))
     return false;
   if (((rows + 63) / 64) * ((out_features + 127) / 128) > compute_units()) return false;
@@ -361,6 +364,13 @@ void launch_stream(stream::Args& a, int block, hipStream_t s) {
   if (block == 32) stream::launch<DT, stream::NF4, 4>(a, s);
   else if (block == 64) stream::launch<DT, stream::NF4, 2>(a, s);
   else stream::launch<DT, stream::NF4, 1, stream::SPAN>(a, s);
+}
+
+// The kernel of a call that lnq_nf4_linear's checks let through.
+int kernel_for(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
+               const void* codes) {
+  if (mid_takes(rows, out_features, in_features, block, x_stride, y_stride, codes)) return LNQ_NF4_TILES;
+  return stream_takes(rows, out_features, in_features, block, x_stride, y_stride) ? LNQ_NF4_STREAM : LNQ_NF4_GEMV;
 }
 
 }  // namespace
@@ -444,11 +454,12 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
   const int slots = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
   const Nf4Planes planes = planes_for(dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (mid_takes(rows, out_features, in_features, block, x_stride, y_stride, codes))
+  const int kernel = kernel_for(rows, out_features, in_features, block, x_stride, y_stride, codes);
+  if (kernel == LNQ_NF4_TILES)
     return launch_nf4_mid(x, static_cast<int>(x_stride), codes, absmax, bias, y, static_cast<int>(y_stride),
                           static_cast<int>(rows), static_cast<int>(out_features), static_cast<int>(in_features),
                           static_cast<int>(block), planes, dtype, s);
-  if (stream_takes(rows, out_features, in_features, block, x_stride, y_stride)) {
+  if (kernel == LNQ_NF4_STREAM) {
     stream::Args a{};
     a.x = static_cast<const uint16_t*>(x);
     a.w = codes;
@@ -518,6 +529,20 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
     const LnqStatus st = launched("nf4_gemv");
     if (st != LNQ_OK) return st;
   }
+  return LNQ_OK;
+}
+
+LNQ_API LnqStatus lnq_nf4_linear_plan(int64_t rows, int64_t x_stride, int64_t out_features, int64_t in_features,
+                                      int64_t block, int32_t* chosen) {
+  LNQ_REQUIRE(chosen != nullptr, "lnq_nf4_linear_plan: null pointer");
+  LNQ_REQUIRE(rows > 0 && out_features > 0 && in_features > 0 && block > 0 && block % nf4::UNIT == 0 &&
+                  in_features % block == 0,
+              "lnq_nf4_linear_plan: bad shape rows=%lld in=%lld out=%lld block=%lld", static_cast<long long>(rows),
+              static_cast<long long>(in_features), static_cast<long long>(out_features), static_cast<long long>(block));
+  // Any 16-byte aligned address stands for the codes.
+  *chosen = kernel_for(rows, out_features, in_features, block, x_stride, out_features,
+                       reinterpret_cast<const void*>(static_cast<uintptr_t>(256)));
+  clear_error();
   return LNQ_OK;
 }
 

@@ -298,3 +298,20 @@ def test_a_bias_is_added_before_the_only_rounding(dtype: torch.dtype, rows: int,
     err = np.abs(got.double().cpu().numpy() - ref)
     print(f"max err / bound {float((err / bound).max()):.3f}", flush=True)
     assert np.all(err <= bound)
+
+
+@pytest.mark.parametrize("rows", [1, 8])
+def test_few_rows_over_a_wide_output(rows: int) -> None:
+    """4096 -> 28672 with a bias: the kernels of few rows (one rounding)."""
+    print(f"nf4 wide output rows {rows}", flush=True)
+    codes, absmax = _layer(28672, 4096, 64, rows)
+    gen = torch.Generator().manual_seed(rows)
+    x, b = torch.randn(rows, 4096, generator=gen).to(torch.bfloat16), torch.randn(28672, generator=gen).to(torch.bfloat16)
+    got = kernels.nf4_linear(x.to(DEV), torch.from_numpy(codes).to(DEV), torch.from_numpy(absmax).to(DEV), 64, b.to(DEV))
+    values = torch.from_numpy(quant.NF4_VALUES.copy()).to(torch.bfloat16).double().numpy()
+    q = np.stack([codes & 15, codes >> 4], axis=-1).reshape(28672, 4096)
+    w = values[q] * np.repeat(absmax.astype(np.float64), 64, axis=1)
+    xd, bd = x.double().numpy(), b.double().numpy()
+    ref = xd @ w.T + bd
+    bound = 2.0 ** -8 * np.abs(ref) + 2.0 ** -20 * (np.abs(xd) @ np.abs(w).T + np.abs(bd)) + 2.0 ** -24
+    assert np.all(np.abs(got.double().cpu().numpy() - ref) <= bound)
