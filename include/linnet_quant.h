@@ -481,7 +481,10 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
                                  int32_t dtype, void* stream);
 
 /* The kernel lnq_nf4_linear takes on the current device, for rows of x x_stride elements
- * apart and 16-byte aligned codes. No counterpart in the reference. */
+ * apart and 16-byte aligned codes; LNQ_NF4_WIDENED where lnq_nf4_dequant and a library product
+ * are the faster (by estimates of both) or lnq_nf4_linear refuses the shape. No counterpart in
+ * the reference, whose generated module always widens. */
+#define LNQ_NF4_WIDENED 0
 #define LNQ_NF4_GEMV 1
 #define LNQ_NF4_STREAM 2
 #define LNQ_NF4_TILES 3

@@ -25,6 +25,7 @@ BF16, F16, F32 = 0, 1, 2
  KERNEL_SPLIT) = range(8)
 PROLOGUE_RMSNORM, PROLOGUE_SILU_MUL = 1, 2
 PACKING_GPTQ, PACKING_AWQ = 0, 1
+NF4_WIDENED, NF4_GEMV, NF4_STREAM, NF4_TILES = range(4)
 
 _p = ctypes.c_void_p
 _i64 = ctypes.c_int64

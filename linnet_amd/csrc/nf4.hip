@@ -336,26 +336,65 @@ bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64
          in_features <= stream::MAX_K && x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
 }
 
-// Whether the 64 x 128 tiles of int4_mid.hip take the call: blocks that hold whole 64-input
-// chunks, a tile a CU at most, and more than 16 rows, whose passes of 32 on the streaming kernel
-// cost more (up to 16 rows that kernel's narrower forms and the GEMV cost less than such a pass:
-// 4096 -> 28672 1 / 4 / 8 / 16 rows 18.2 / 25.7 / 26.3 / 27.2 on them, 30 in tiles; 24 rows 33.7
-// / 31.5; 8192 -> 28672 1 / 16 rows 33.1 / 46.1, 55)
-// (us, estimates within a fifth of block 64 measured, streaming / tiles: 4096 -> 14336 32 rows
-// 18.7 / 29, 64 rows 32.5 / 29.7, 96 rows 46.9 / 31.2; 14336 -> 4096 64 rows 38.3 / 86, 96 rows
-// 55.8 / 86.5; 3072 -> 9216 32 rows 15.7 / 23, 64 rows 28.5 / 23.1; 4096 -> 4096 96 rows
-// 22.5 / 28.6). Past 96 rows always: the alternative then is the widened weight and its
-// product (128 rows 70.7 / 32.1, 116.2 / 87.0, 40.7 / 24.4, 37.0 / 28.8), not this kernel's
-// fifth pass.
-bool mid_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
-               const void* codes) {
-  if (rows <= 16 || rows > INT32_MAX || block < 64 || (block & (block - 1)) != 0 || !aligned(codes, 16) || y_stride > INT32_MAX ||
+// Whether the 64 x 128 tiles of int4_mid.hip can take the call: blocks that hold whole 64-input
+// chunks, a tile a CU at most.
+bool tiles_take(int64_t rows, int64_t out_features, int64_t block, int64_t x_stride, int64_t y_stride, const void* codes) {
+  if (rows > INT32_MAX || block < 64 || (block & (block - 1)) != 0 || !aligned(codes, 16) || y_stride > INT32_MAX ||
       x_stride >= (int64_t{1} << 23) || (rows + 63) * x_stride >= (int64_t{1} << 30))
     return false;
-  if (((rows + 63) / 64) * ((out_features + 127) / 128) > compute_units()) return false;
-  const double tiles = 6 + 1.45 * ((in_features + 255) / 256);
-  const double pass = 3 + static_cast<double>(out_features) * in_features / 4.4e6;
-  return rows > 96 || tiles < ((rows + 31) / 32) * pass;
+  return ((rows + 63) / 64) * ((out_features + 127) / 128) <= compute_units();
+}
+
+// Estimated us past 16 rows, fitted to 17 to 512 rows of 27 layers from 512 -> 4096 to 14336 ->
+// 28672 (nine in ten within 10, 7 and 15 percent). The streaming kernel: whole rounds of its
+// workgroups, 32 rows of x each (16 where the scales of a wide layer take the LDS), by the 16-row
+// tiles that a workgroup holds. Measured streaming / tiles / widened, block 64: 64 rows 4096 ->
+// 14336 32.8 / 30.2 / 60.6, 4096 -> 4096 14.6 / 29.3 / 30.7; 96 rows 4096 -> 14336 48.3 / 30.9 /
+// 60.8, 14336 -> 4096 53.3 / 86.9 / 85.1; 128 rows 4096 -> 4096 26.7 / 29.3 / 37.4, 14336 -> 4096
+// 69.7 / 87.3 / 95.1; 256 rows 2048 -> 8192 - / 19.4 / 37.8.
+double stream_us(int64_t rows, int64_t out_features, int64_t in_features, int64_t block) {
+  stream::Args a{};
+  a.cols = static_cast<int>(in_features / block);
+  a.row_block = 1;
+  int most = stream::fitting_rows<stream::NF4, 2, 2, 8, stream::ONE_STEP>(a), x_rows = 32;
+  if (most < 16) most = stream::fitting_rows<stream::NF4, 2, 1, 4, stream::ONE_STEP>(a), x_rows = 16;
+  const int r = stream::rows_per_block(static_cast<int>(out_features), most);
+  const int64_t groups = (out_features + r - 1) / r * ((rows + x_rows - 1) / x_rows);
+  const double k = static_cast<double>(in_features) / 1024;
+  const double round = r <= 16 ? 2.5 + 0.95 * k : r <= 32 ? 2.5 + 1.5 * k : 4.5 + 2.55 * k;
+  return (2.5 + round * ((groups + compute_units() - 1) / compute_units())) * (block == 32 ? 1.1 : 1.0);
+}
+
+double tiles_us(int64_t in_features) { return 6 + 1.45 * ((in_features + 255) / 256); }
+
+// The widened weight and the library's product of it.
+double widened_us(int64_t rows, int64_t out_features, int64_t in_features) {
+  const double weights = static_cast<double>(out_features) * in_features;
+  return 10.4 + weights * (0.9e-6 + 1.33e-9 * rows) + 0.86 / 1024 * in_features;
+}
+
+// The kernel of a call that lnq_nf4_linear's checks let through. No tiles up to 16 rows, where
+// the streaming kernel's narrower forms and the GEMV cost less than the pass of 17 to 32 rows
+// that the estimate is of (4096 -> 28672 1 / 4 / 8 / 16 rows 18.2 / 25.7 / 26.3 / 27.2, in tiles
+// 30; 24 rows 33.7 / 31.5; 8192 -> 28672 1 / 16 rows 33.1 / 46.1, in tiles 55).
+int kernel_for(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
+               const void* codes) {
+  const bool streams = stream_takes(rows, out_features, in_features, block, x_stride, y_stride);
+  if (rows > 16 && tiles_take(rows, out_features, block, x_stride, y_stride, codes) &&
+      (!streams || tiles_us(in_features) < stream_us(rows, out_features, in_features, block)))
+    return LNQ_NF4_TILES;
+  return streams ? LNQ_NF4_STREAM : LNQ_NF4_GEMV;
+}
+
+// Whether the stored weight is the faster one for that kernel: always up to 64 rows, by the
+// estimates above that, and past 96 rows only in tiles (the library's product gains on further
+// passes: 160 rows 4096 -> 14336 77.8 streamed, 66.9 widened). The GEMV keeps 16 rows (8 past In =
+// 8192); more are its passes over the weight again.
+bool stored_preferred(int kernel, int64_t rows, int64_t out_features, int64_t in_features, int64_t block) {
+  if (kernel == LNQ_NF4_GEMV) return rows <= (in_features <= 8192 ? 16 : 8);
+  if (rows <= 64) return true;
+  const double us = kernel == LNQ_NF4_TILES ? tiles_us(in_features) : stream_us(rows, out_features, in_features, block);
+  return (rows <= 96 || kernel == LNQ_NF4_TILES) && us < widened_us(rows, out_features, in_features);
 }
 
 template <int DT>
@@ -364,13 +403,6 @@ void launch_stream(stream::Args& a, int block, hipStream_t s) {
   if (block == 32) stream::launch<DT, stream::NF4, 4>(a, s);
   else if (block == 64) stream::launch<DT, stream::NF4, 2>(a, s);
   else stream::launch<DT, stream::NF4, 1, stream::SPAN>(a, s);
-}
-
-// The kernel of a call that lnq_nf4_linear's checks let through.
-int kernel_for(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride, int64_t y_stride,
-               const void* codes) {
-  if (mid_takes(rows, out_features, in_features, block, x_stride, y_stride, codes)) return LNQ_NF4_TILES;
-  return stream_takes(rows, out_features, in_features, block, x_stride, y_stride) ? LNQ_NF4_STREAM : LNQ_NF4_GEMV;
 }
 
 }  // namespace
@@ -535,13 +567,15 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
 LNQ_API LnqStatus lnq_nf4_linear_plan(int64_t rows, int64_t x_stride, int64_t out_features, int64_t in_features,
                                       int64_t block, int32_t* chosen) {
   LNQ_REQUIRE(chosen != nullptr, "lnq_nf4_linear_plan: null pointer");
-  LNQ_REQUIRE(rows > 0 && out_features > 0 && in_features > 0 && block > 0 && block % nf4::UNIT == 0 &&
-                  in_features % block == 0,
-              "lnq_nf4_linear_plan: bad shape rows=%lld in=%lld out=%lld block=%lld", static_cast<long long>(rows),
-              static_cast<long long>(in_features), static_cast<long long>(out_features), static_cast<long long>(block));
-  // Any 16-byte aligned address stands for the codes.
-  *chosen = kernel_for(rows, out_features, in_features, block, x_stride, out_features,
-                       reinterpret_cast<const void*>(static_cast<uintptr_t>(256)));
+  *chosen = LNQ_NF4_WIDENED;
+  if (rows > 0 && out_features > 0 && in_features > 0 && block > 0 && block % nf4::UNIT == 0 && in_features % block == 0 &&
+      in_features <= nf4::UNIT * nf4::THREADS * nf4::MAX_SLOTS && out_features <= INT32_MAX &&
+      out_features * (in_features / 2) < (int64_t{1} << 31) && x_stride >= in_features && x_stride % 8 == 0) {
+    // Any 16-byte aligned address stands for the codes.
+    const int kernel = kernel_for(rows, out_features, in_features, block, x_stride, out_features,
+                                  reinterpret_cast<const void*>(static_cast<uintptr_t>(256)));
+    if (stored_preferred(kernel, rows, out_features, in_features, block)) *chosen = kernel;
+  }
   clear_error();
   return LNQ_OK;
 }

@@ -845,22 +845,6 @@ def nf4_gemv_fits(rows: int, in_features: int, block: int, dtype: torch.dtype) -
             and 0 < in_features <= NF4_GEMV_MAX_IN)
 
 
-# Rows up to which `nf4_linear` reads the stored weight at any shape: past NF4_GEMV_ROWS on
-# the streaming kernel, 32 rows a pass, or in tiles. us, block 64, stored / widened at 96 rows:
-# 4096 -> 14336 31.2 / 70.4, 14336 -> 4096 55.8 / 103.2, 2048 -> 2048 15.0 / 16.3.
-NF4_STREAM_ROWS = 96
-# Past those, where 64 x 128 tiles give no compute unit a second one and win by estimates of
-# both (us, from these; 128 rows: 4096 -> 14336 32.1 / 71.6, 4096 -> 4096 28.8 / 37.7, 14336 -> 4096
-# 87.0 / 114.4, but 2048 -> 2048 17.1 / 16.4; 200 rows 4096 -> 14336, 448 tiles: 76 widened).
-NF4_TILES = 256
-
-
-def _nf4_tiles_fit(rows: int, out_features: int, in_features: int, block: int) -> bool:
-    tiles = -(-rows // 64) * -(-out_features // 128)
-    return (block >= 64 and block & (block - 1) == 0 and tiles <= NF4_TILES
-            and 6 + 1.45 * in_features / 256 < 0.9 * (11 + out_features * in_features * 1e-6 + 0.002 * in_features))
-
-
 def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor | None, rows: int, block: int) -> bool:
     """Whether `nf4_linear` multiplies by the stored weight (`lnq_nf4_linear`) rather than
     the widened one. Past the GEMV's rows the widened product takes whatever that entry
@@ -869,16 +853,22 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
     out_features, in_features = codes.shape[0], 2 * codes.shape[1]
     if nf4_gemv_fits(rows, in_features, block, x.dtype):
         return True
-    if not (x.dtype in _HALF and (rows <= NF4_STREAM_ROWS or _nf4_tiles_fit(rows, out_features, in_features, block)) and (block in (32, 64) or block % 128 == 0)
-            and in_features % block == 0 and 0 < in_features <= NF4_GEMV_MAX_IN
-            and out_features * in_features < 1 << 32):
+    if x.dtype not in _HALF or x.shape[-1] != in_features:
         return False
     if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
         return False
     if torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0:
         return False
-    return (bias is None or (bias.dtype == x.dtype and bias.numel() == out_features)) and (
-        (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))
+    if not ((bias is None or (bias.dtype == x.dtype and bias.numel() == out_features)) and (
+            (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))):
+        return False
+    # The rows as `nf4_gemv` passes them: a view where they lie evenly, else a copy.
+    stride = in_features if x.is_contiguous() else x.reshape(-1, in_features).stride(0)
+    chosen = ctypes.c_int32(0)
+    with _on(x.device):
+        _lib.call("lnq_nf4_linear_plan", rows, max(stride, in_features) if stride % 8 == 0 else in_features, out_features,
+                  in_features, block, ctypes.byref(chosen))
+    return chosen.value != _lib.NF4_WIDENED
 
 
 def nf4_gemv(x: torch.Tensor, codes: torch.Tensor, absmax: torch.Tensor, block: int,

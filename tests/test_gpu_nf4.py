@@ -315,3 +315,12 @@ def test_few_rows_over_a_wide_output(rows: int) -> None:
     ref = xd @ w.T + bd
     bound = 2.0 ** -8 * np.abs(ref) + 2.0 ** -20 * (np.abs(xd) @ np.abs(w).T + np.abs(bd)) + 2.0 ** -24
     assert np.all(np.abs(got.double().cpu().numpy() - ref) <= bound)
+
+
+def test_rows_far_apart_are_widened() -> None:
+    """Rows of x 32 MB apart: past the GEMV, no kernel of the stored weight takes them in one pass."""
+    codes, absmax = (torch.from_numpy(t).to(DEV) for t in _layer(64, 256, 64, 4))
+    x = torch.empty(20 << 24, dtype=torch.bfloat16, device=DEV).view(20, 1 << 24)[:, :256]
+    x.copy_(torch.randn(20, 256, generator=torch.Generator().manual_seed(3)))
+    want = torch.nn.functional.linear(x, kernels.nf4_dequantize(codes, absmax, 64, torch.bfloat16))
+    assert torch.equal(kernels.nf4_linear(x, codes, absmax, 64), want)

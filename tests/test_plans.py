@@ -9,7 +9,7 @@ import pytest
 
 from linnet_amd import _lib
 
-GEMV, STREAM, TILES = 1, 2, 3
+WIDENED, GEMV, STREAM, TILES = _lib.NF4_WIDENED, _lib.NF4_GEMV, _lib.NF4_STREAM, _lib.NF4_TILES
 
 
 def _nf4(rows: int, out: int, width: int, block: int = 64, stride: int | None = None) -> int:
@@ -27,3 +27,24 @@ def test_nf4_few_rows_over_wide_outputs_take_no_tiles(out: int, width: int, bloc
     for rows in (5, 8, 16):
         assert _nf4(rows, out, width, block) == STREAM
     assert _nf4(64, out, width, block) == TILES
+
+
+@pytest.mark.parametrize(("rows", "out", "width", "block", "want"), [
+    (17, 4096, 4096, 64, STREAM), (64, 14336, 4096, 64, TILES), (96, 4096, 14336, 64, STREAM),
+    (128, 14336, 4096, 64, TILES), (97, 4096, 14336, 64, WIDENED),  # 88 us in tiles, 77 widened
+    (96, 9216, 3072, 32, WIDENED),  # blocks of 32 have no tiles: 47 us streamed, 39 widened
+    (64, 9216, 3072, 32, STREAM), (96, 14336, 4096, 32, STREAM), (200, 14336, 4096, 64, WIDENED),  # two tiles a unit
+    (17, 64, 65536, 64, WIDENED), (17, 1 << 20, 8192, 64, WIDENED),  # lnq_nf4_linear refuses
+    (16, 64, 1024, 16, GEMV), (17, 64, 1024, 16, WIDENED),  # blocks that only the GEMV takes
+    (9, 64, 16384, 16, WIDENED)])
+def test_nf4_reads_the_stored_weight_where_it_is_faster(rows: int, out: int, width: int, block: int, want: int) -> None:
+    assert _nf4(rows, out, width, block) == want
+
+
+def test_nf4_rows_far_apart_are_widened() -> None:
+    """Past the streaming kernel's and the tiles' strides the stored weight would be read
+    again for every 8 rows, or the call refused."""
+    for stride in (1 << 23, 1 << 28):
+        assert _nf4(16, 4096, 4096, 64, stride) == GEMV
+        for rows in (17, 64, 128):
+            assert _nf4(rows, 4096, 4096, 64, stride) == WIDENED
