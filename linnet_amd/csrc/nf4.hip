@@ -9,7 +9,7 @@
 //   the scale rounded once (`dequantize_nf4`, quant.linnet:180-187), bit for bit.
 // - nf4_gemv_kernel: y = x W^T (+ bias), up to 8 rows of x a pass, the weight read
 //   once from HBM as it is stored (lnq_nf4_linear's fewest rows, and the blocks the
-//   streaming product and the tiles do not take: stream_takes, mid_takes). NF4's values are no affine function of the
+//   streaming product and the tiles do not take: gemv_preferred, kernel_for). NF4's values are no affine function of the
 //   code, so the widening is a table lookup done in registers: the 16 values'
 //   16-bit patterns (bf16 or f16, x's type) are held as two 16-byte planes (low
 //   bytes, high bytes) in 8 SGPRs, and v_perm_b32 selects four codes' bytes from
@@ -325,15 +325,39 @@ Nf4Planes planes_for(int dtype) {
   return p;
 }
 
-// Whether the streaming product (stream.hpp) takes the call: past 4 rows (2 where In > 4096
-// gives the GEMV's lanes several units; 4096 -> 14336, block 64: 4 rows 14.0 us on the GEMV
-// against 14.9, 5 rows 20.9 against 14.1, 16 rows 42.9 against 15.4; 14336 -> 4096: 2 rows
-// 13.9 against 14.1, 4 rows 19.1 against 14.5), blocks its
-// steps hold whole (32, 64 or 128 k inputs), 32 rows of x below 1 GiB.
+// Slots of 256 units a GEMV lane has over a row, and the rows of x of a pass (x's registers
+// grow with rows x slots).
+int gemv_slots(int64_t in_features) {
+  const int64_t need = (in_features / nf4::UNIT + nf4::THREADS - 1) / nf4::THREADS;
+  return need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+}
+
+int gemv_pass(int slots) { return slots <= 2 ? nf4::MAX_ROWS_X : 4; }
+
+// Whether the GEMV is faster than the streaming kernel: up to 4 rows (2 where In > 4096 gives
+// its lanes several units; us GEMV / streaming, block 64: 4096 -> 14336 4 rows 14.0 / 14.9, 5
+// rows 20.9 / 14.1, 16 rows 42.9 / 15.4; 14336 -> 4096 2 rows 13.9 / 14.1, 4 rows 19.1 / 14.5),
+// and a single pass over a narrow output, whose workgroups are at most one a CU (two from In =
+// 12288 on), where the streaming kernel's prologue and steps along In are the longer: 4096 ->
+// 1024 5 rows 5.0 / 5.9, 4096 -> 1152 (two rounds) 6.2 / 5.8; 8192 -> 1024 8 rows 7.0 / 8.1; 8192
+// -> 2048 4 rows 7.4 / 8.0; 14336 -> 2048 3 rows 10.4 / 11.2. Not up to In = 2048 (2048 -> 1024 5
+// rows 4.6 / 4.4), nor 3 and 4 rows where a lane's second slot is partly empty (6144 -> 1536
+// 7.1 / 6.6).
+bool gemv_preferred(int64_t rows, int64_t out_features, int64_t in_features) {
+  const int slots = gemv_slots(in_features);
+  if (rows <= (slots == 1 ? 4 : 2)) return true;
+  if (rows > gemv_pass(slots) || in_features <= 2048 || (rows <= 4 && slots == 2 && in_features <= 6144)) return false;
+  const int r = nf4_rows(rows <= 4 ? 4 : 8, slots);
+  return (out_features + r - 1) / r <= static_cast<int64_t>(compute_units()) * (in_features >= 12288 ? 2 : 1);
+}
+
+// Whether the streaming product (stream.hpp) takes the call: blocks its steps hold whole (32, 64
+// or 128 k inputs), 32 rows of x below 1 GiB, and not the GEMV's.
 bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride,
                   int64_t y_stride) {
-  return rows > (in_features <= nf4::UNIT * nf4::THREADS ? 4 : 2) && rows <= INT32_MAX && (block == 32 || block == 64 || block % 128 == 0) &&
-         in_features <= stream::MAX_K && x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
+  return !gemv_preferred(rows, out_features, in_features) && rows <= INT32_MAX &&
+         (block == 32 || block == 64 || block % 128 == 0) && in_features <= stream::MAX_K &&
+         x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
 }
 
 // Whether the 64 x 128 tiles of int4_mid.hip can take the call: blocks that hold whole 64-input
@@ -481,9 +505,7 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
               "lnq_nf4_linear: row strides shorter than a row");
   LNQ_REQUIRE(aligned(x, 16) && x_stride % 8 == 0 && aligned(codes, 8),
               "lnq_nf4_linear: x (with its row stride) must be 16-byte aligned and the codes 8-byte aligned");
-  const int units = static_cast<int>(in_features / nf4::UNIT);
-  const int need = (units + nf4::THREADS - 1) / nf4::THREADS;
-  const int slots = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
+  const int slots = gemv_slots(in_features);
   const Nf4Planes planes = planes_for(dtype);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int kernel = kernel_for(rows, out_features, in_features, block, x_stride, y_stride, codes);
@@ -514,8 +536,7 @@ LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, 
   const int O = static_cast<int>(out_features), K = static_cast<int>(in_features), B = static_cast<int>(block);
   // Up to 8 rows of x a launch (4 past In = 8192); more rows take more launches
   // over the same weight.
-  // x's registers grow with rows x slots: 8 rows a pass up to 2 slots, else 4.
-  const int per_pass = slots <= 2 ? nf4::MAX_ROWS_X : 4;
+  const int per_pass = gemv_pass(slots);
   for (int64_t r0 = 0; r0 < rows; r0 += per_pass) {
     const int part = static_cast<int>(rows - r0 < per_pass ? rows - r0 : per_pass);
     const int mr = part == 1 ? 1 : part == 2 ? 2 : part <= 4 ? 4 : 8;

@@ -48,3 +48,13 @@ def test_nf4_rows_far_apart_are_widened() -> None:
         assert _nf4(16, 4096, 4096, 64, stride) == GEMV
         for rows in (17, 64, 128):
             assert _nf4(rows, 4096, 4096, 64, stride) == WIDENED
+
+
+@pytest.mark.parametrize(("rows", "out", "width", "want"), [
+    (5, 1024, 4096, GEMV), (8, 1024, 8192, GEMV), (9, 1024, 4096, STREAM), (5, 1025, 4096, STREAM), (5, 1024, 2048, STREAM),
+    (3, 2048, 8192, GEMV), (4, 2049, 8192, STREAM), (3, 1536, 6144, STREAM), (8, 1024, 6144, GEMV),
+    (3, 2048, 14336, GEMV), (4, 2049, 14336, STREAM), (5, 512, 14336, STREAM), (3, 1024, 11008, GEMV),
+    (3, 1152, 11008, STREAM), (4, 14336, 4096, GEMV), (3, 4096, 14336, STREAM)])
+def test_nf4_narrow_outputs_keep_the_gemv(rows: int, out: int, width: int, want: int) -> None:
+    """One GEMV pass of at most a workgroup a unit: 4096 -> 1024 at 5 rows 5.0 us, streamed 5.9."""
+    assert _nf4(rows, out, width) == want
