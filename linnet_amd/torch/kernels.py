@@ -859,7 +859,7 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
         return False
     if torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0:
         return False
-    if not ((bias is None or (bias.dtype == x.dtype and bias.numel() == out_features)) and (
+    if not ((bias is None or (bias.dtype == x.dtype and bias.shape == (out_features,))) and (
             (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))):
         return False
     # The rows as `nf4_gemv` passes them: a view where they lie evenly, else a copy.

@@ -324,3 +324,21 @@ def test_rows_far_apart_are_widened() -> None:
     x.copy_(torch.randn(20, 256, generator=torch.Generator().manual_seed(3)))
     want = torch.nn.functional.linear(x, kernels.nf4_dequantize(codes, absmax, 64, torch.bfloat16))
     assert torch.equal(kernels.nf4_linear(x, codes, absmax, 64), want)
+
+
+def _few_rows_past_the_gemv(rows: int, out: int, dtype: torch.dtype = torch.bfloat16) -> tuple[torch.Tensor, ...]:
+    codes, absmax = (torch.from_numpy(t).to(DEV) for t in _layer(out, 256, 64, rows))
+    x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows)).to(dtype).to(DEV)
+    return x, codes, absmax, kernels.nf4_dequantize(codes, absmax, 64, dtype)
+
+
+@pytest.mark.parametrize("shape", [(64, 1), (1, 64), (8, 8)])
+def test_a_bias_of_another_shape_broadcasts_as_the_widened_product_does(shape: tuple[int, int]) -> None:
+    """A column per row, a row per column, or refused: not as many values in any shape."""
+    x, codes, absmax, weight = _few_rows_past_the_gemv(64, 64)
+    bias = torch.randn(shape, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(DEV)
+    if shape == (8, 8):
+        with pytest.raises(RuntimeError):
+            kernels.nf4_linear(x, codes, absmax, 64, bias)
+        return
+    assert torch.equal(kernels.nf4_linear(x, codes, absmax, 64, bias), torch.nn.functional.linear(x, weight, bias))
