@@ -859,6 +859,9 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
         return False
     if torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0:
         return False
+    # Under autocast to the other 16-bit type the product and its result are of that type.
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype:
+        return False
     if not ((bias is None or (bias.dtype == x.dtype and bias.shape == (out_features,))) and (
             (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))):
         return False

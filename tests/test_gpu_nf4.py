@@ -342,3 +342,12 @@ def test_a_bias_of_another_shape_broadcasts_as_the_widened_product_does(shape: t
             kernels.nf4_linear(x, codes, absmax, 64, bias)
         return
     assert torch.equal(kernels.nf4_linear(x, codes, absmax, 64, bias), torch.nn.functional.linear(x, weight, bias))
+
+
+@pytest.mark.parametrize("to", [torch.bfloat16, torch.float16])
+def test_autocast_multiplies_in_its_type(to: torch.dtype) -> None:
+    x, codes, absmax, weight = _few_rows_past_the_gemv(24, 72)
+    with torch.autocast("cuda", dtype=to):
+        got, want = kernels.nf4_linear(x, codes, absmax, 64), torch.nn.functional.linear(x, weight)
+    assert got.dtype == want.dtype == to
+    torch.testing.assert_close(got, want, rtol=1e-2, atol=1e-2 * want.abs().max().item())
