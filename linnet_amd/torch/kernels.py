@@ -849,7 +849,7 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
     """Whether `nf4_linear` multiplies by the stored weight (`lnq_nf4_linear`) rather than
     the widened one. Past the GEMV's rows the widened product takes whatever that entry
     refuses (wide or huge weights, operands off their alignment, a broadcast bias) and what
-    needs an operator that autograd and vmap know."""
+    needs an operator that autograd, vmap, tensor subclasses and modes see."""
     out_features, in_features = codes.shape[0], 2 * codes.shape[1]
     if nf4_gemv_fits(rows, in_features, block, x.dtype):
         return True
@@ -858,6 +858,8 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
     if torch.is_grad_enabled() and (x.requires_grad or (bias is not None and bias.requires_grad)):
         return False
     if torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0:
+        return False
+    if torch.overrides.has_torch_function_variadic(x, bias) or torch._C._len_torch_dispatch_stack():
         return False
     # Under autocast to the other 16-bit type the product and its result are of that type.
     if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype:

@@ -351,3 +351,24 @@ def test_autocast_multiplies_in_its_type(to: torch.dtype) -> None:
         got, want = kernels.nf4_linear(x, codes, absmax, 64), torch.nn.functional.linear(x, weight)
     assert got.dtype == want.dtype == to
     torch.testing.assert_close(got, want, rtol=1e-2, atol=1e-2 * want.abs().max().item())
+
+
+def test_subclasses_and_modes_see_the_product() -> None:
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Named(torch.Tensor):
+        pass
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):  # type: ignore[no-untyped-def]
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    names: list[str] = []
+    x, codes, absmax, weight = _few_rows_past_the_gemv(24, 72)
+    want = torch.nn.functional.linear(x, weight)
+    got = kernels.nf4_linear(x.as_subclass(Named), codes, absmax, 64)
+    assert type(got) is Named and torch.equal(got.as_subclass(torch.Tensor), want)
+    with Seen():
+        got = kernels.nf4_linear(x, codes, absmax, 64)
+    assert torch.equal(got, want) and any("mm" in n or "linear" in n for n in names)
