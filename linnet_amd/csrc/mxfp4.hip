@@ -199,7 +199,7 @@ __global__ __launch_bounds__(64 * mx::GROUP_WAVES, MT == 1 ? 4 : 2) void mxfp4_g
   for (int m0 = 0; m0 < count; m0 += ROWS) {
     const int live = min(count - m0, ROWS);
     stream::product<mx::GROUP_WAVES, DT, stream::FP4, 4, MT, XI, NT, stream::ONE_STEP>(
-        a, n0, n_end, a.x, g.x_bytes, X0, X1, X2, X3, SC,
+        a, n0, n_end, a.x, g.x_bytes, X0, X1, SC,
         [&](int i) -> int {
           if (i >= live) return -1;
           const int p = list[m0 + i], r = p / g.chosen;

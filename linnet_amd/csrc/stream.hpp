@@ -58,16 +58,14 @@ constexpr bool eight(int f) { return f == INT8 || f == FP8; }
 // f16 the offset comes off exactly), which sums of x undo.
 constexpr bool needs_xsum(int f, int dt) { return f == INT4 || (f == INT8 && dt == LNQ_BF16); }
 
-// Steps whose x and weights a wave has in flight: four (K = 4096: all of a wave's), two
-// where 32 rows of x a step leave LDS for no more.
-constexpr int depth(int) { return 2; }
+// Steps whose x a wave has in flight, a stage each.
+constexpr int DEPTH = 2;
 // x values of a wave's stage of one step: the 4 xi rows that are moved.
 // (the stages hold the waves' sums at the end: 512 values a unit of 16 x 16 outputs).
 constexpr int stage_values(int xi, int mt, int nt) {
-  const int sums = 512 * ((mt * nt + depth(mt) - 1) / depth(mt));
+  const int sums = 512 * ((mt * nt + DEPTH - 1) / DEPTH);
   return 4 * xi * STEP > sums ? 4 * xi * STEP : sums;
 }
-constexpr int stage_array(int nw, int xi, int mt, int nt, int i) { return i < depth(mt) ? nw * stage_values(xi, mt, nt) : 8; }
 
 // NF4's 16 values in x's type as byte planes (see nf4.hip).
 struct Planes {
@@ -208,7 +206,7 @@ inline int scale_lds(int f, bool per_row, bool blocks, int rows, int cols, int r
 // GPS: groups a step (0: one scale a row). NW: the workgroup's waves, which
 // all call it.
 template <int NW, int DT, int F, int GPS, int MT, int XI, int NT, int KIND, class RowOf, class Put>
-__device__ inline void product(const Args& a, int n0, int n_end, const uint16_t* xbase, uint32_t xbytes, uint16_t* X0, uint16_t* X1, uint16_t* X2, uint16_t* X3,
+__device__ inline void product(const Args& a, int n0, int n_end, const uint16_t* xbase, uint32_t xbytes, uint16_t* X0, uint16_t* X1,
                                uint8_t* SC, RowOf row_of, Put put) {
   using E = Elem<DT>;
   constexpr bool XS = needs_xsum(F, DT);
@@ -216,7 +214,7 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   constexpr int US = eight(F) ? 1 : 2;         // steps of a weight unit (128 bytes of a row)
   constexpr int GP = GPS == 0 ? 1 : GPS;       // MFMA chains of a step
   constexpr int TPG = 4 / GP;                  // MFMAs of a chain
-  constexpr int D = depth(MT);                 // steps in flight
+  constexpr int D = DEPTH;                     // steps in flight
   constexpr int XW = stage_values(XI, MT, NT);         // x values of a wave's stage
 
   const int lane = threadIdx.x & 63;
@@ -227,8 +225,7 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   const int per = (units + NW - 1) / NW;
   const int u0 = min(units, wave * per), u1 = min(units, u0 + per);
   const int s0 = u0 * US, s1 = min(steps, u1 * US);
-  uint16_t* const xw[4] = {X0 + wave * XW, X1 + wave * XW, D > 2 ? X2 + wave * XW : nullptr,
-                           D > 2 ? X3 + wave * XW : nullptr};
+  uint16_t* const xw[D] = {X0 + wave * XW, X1 + wave * XW};
 
   // Per-workgroup buffers: the rows' own bytes, so that offsets stay below 1 GiB.
   const int rows = n_end - n0;
@@ -505,7 +502,7 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   constexpr int PER_ARRAY = XW * 2 / 1024;  // units of a wave an array holds
   static_assert(PER_ARRAY * D >= UNITS, "the sums fit the stages");
   auto unit = [&](int q, int wv) -> f32x4* {
-    uint16_t* const base = q / PER_ARRAY == 0 ? X0 : q / PER_ARRAY == 1 ? X1 : q / PER_ARRAY == 2 ? X2 : X3;
+    uint16_t* const base = q / PER_ARRAY == 0 ? X0 : X1;
     return reinterpret_cast<f32x4*>(base + wv * XW + (q % PER_ARRAY) * 512);
   };
 #pragma unroll
@@ -537,12 +534,11 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
 }
 
 // The x stages, an LDS array each: the compiler tracks the loads into LDS by variable, so
-// a stage's reads wait for that stage's loads alone.
-#define LNQ_STREAM_STAGES(NW, XI, MT, NT)                                                             \
-  __shared__ __attribute__((aligned(16))) uint16_t X0[stream::stage_array(NW, XI, MT, NT, 0)];        \
-  __shared__ __attribute__((aligned(16))) uint16_t X1[stream::stage_array(NW, XI, MT, NT, 1)];        \
-  __shared__ __attribute__((aligned(16))) uint16_t X2[stream::stage_array(NW, XI, MT, NT, 2)];        \
-  __shared__ __attribute__((aligned(16))) uint16_t X3[stream::stage_array(NW, XI, MT, NT, 3)]
+// a stage's reads wait for that stage's loads alone. They are all of a dense workgroup's LDS
+// beside its scales: fitting_rows fills what they leave to the last byte.
+#define LNQ_STREAM_STAGES(NW, XI, MT, NT)                                                       \
+  __shared__ __attribute__((aligned(16))) uint16_t X0[NW * stream::stage_values(XI, MT, NT)];   \
+  __shared__ __attribute__((aligned(16))) uint16_t X1[NW * stream::stage_values(XI, MT, NT)]
 
 // x [M, K] row-major, outputs [M, N]; blocks of R output rows and chunks of 16 MT rows of
 // x. The chunks of one block sit 8 workgroups apart, on one XCD (workgroups go to the 8
@@ -563,7 +559,7 @@ __global__ __launch_bounds__(64 * WAVES) void dense_kernel(Args a) {
   const uint16_t* x = a.x + static_cast<int64_t>(m0) * a.x_stride;
   const uint32_t xbytes = static_cast<uint32_t>(((live - 1) * a.x_stride + a.K) * 2);
   product<WAVES, DT, F, GPS, MT, XI, NT, KIND>(
-      a, n0, n_end, x, xbytes, X0, X1, X2, X3, SC, [&](int i) -> int { return i < live ? i * a.x_stride : -1; },
+      a, n0, n_end, x, xbytes, X0, X1, SC, [&](int i) -> int { return i < live ? i * a.x_stride : -1; },
       [&](int m, int n, float v) {
         if (m < live) {
           if constexpr (F == INT4) {
@@ -604,7 +600,7 @@ template <int F, int GPS, int MT, int XI, int KIND>
 inline int fitting_rows(const Args& a) {
   int most = MAX_R;
   while (most > 0 && scale_lds(F, GPS == 0, KIND == BLOCK, most, a.cols, a.row_block) +
-                             depth(MT) * WAVES * stage_values(XI, MT, most <= 16 ? 1 : most <= 32 ? 2 : 4) * 2 > LDS_BYTES)
+                             DEPTH * WAVES * stage_values(XI, MT, most <= 16 ? 1 : most <= 32 ? 2 : 4) * 2 > LDS_BYTES)
     most -= 8;
   return most;
 }

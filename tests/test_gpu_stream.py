@@ -73,6 +73,24 @@ def test_int4(rows: int, out: int, width: int, group: int, dtype: torch.dtype) -
     _check(got, x, ((q - z) * s).reshape(out, width), ((q + z + 2 * offset) * s).reshape(out, width), bias)
 
 
+@pytest.mark.parametrize(("out", "width"), [(8192, 48640), (8192, 49024), (6144, 64896), (6144, 65408)])
+def test_int4_scales_that_fill_the_lds(out: int, width: int) -> None:
+    """Groups of 32 at 4 rows whose scales and zero points take all the LDS that the stages
+    leave, against the skinny kernel (f32 sums in another order, one rounding each)."""
+    print(f"int4 stream full LDS out={out} in={width}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(width)
+    packed = torch.randint(0, 256, (out, width // 32, 16), generator=g, dtype=torch.uint8, device=DEV)
+    scale = (torch.rand(out, width // 32, generator=g, device=DEV) * 0.02 + 0.001).to(BF16)
+    zero = torch.randint(0, 16, (out, width // 32), generator=g, dtype=torch.uint8, device=DEV)
+    x = torch.randn(4, width, generator=g, device=DEV).to(BF16)
+    got = kernels.int4_linear(x, packed, scale, zero).double()
+    want = kernels.int4_linear(x, packed, scale, zero, kernel="skinny").double()
+    # Half a unit in the last place each, and 16 f32 units of the magnitudes added: |x| times
+    # codes that carry 128 and the zero point, at most (2 * 128 + 30) * 0.021.
+    carried = x.double().abs().sum(1, keepdim=True) * (286 * 0.021)
+    assert bool(((got - want).abs() <= 2 * ULP[BF16] * want.abs() + 2.0**-19 * carried).all())
+
+
 @pytest.mark.parametrize("fp8", [True, False])
 @pytest.mark.parametrize(("rows", "out", "width", "group", "row_block", "dtype"), [
     (1, 72, 640, 0, 1, BF16),  # one row, a scale a row, 5 steps
