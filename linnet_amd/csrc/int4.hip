@@ -651,6 +651,7 @@ LnqStatus launch_int4_mid(const void* x, const uint8_t* packed, const void* scal
 
 // Defined in int4_stream.hip: the streaming few-row product.
 bool int4_stream_supports(int K);
+bool int4_skinny_preferred(int M, int N, int K, int G);
 LnqStatus launch_int4_stream(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
                              const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
 
@@ -767,7 +768,7 @@ static int choose_int4_kernel(int M, int N, int K, int G, int dtype, int kernel,
     // 16, 11.3 / 11.2 at 32) and the skinny kernel is ahead at 64 (18.6 against
     // 22.5 for two 32-row launches).
     // GEMV at 5..16 rows and SKINNY stand for the streaming kernel (launch_few_tokens,
-    // lnq_int4_linear), ahead of both there.
+    // lnq_int4_linear), ahead of both there but for short layers (int4_skinny_preferred).
     const bool wide = N >= 6144;
     const bool few = M <= 6;
     if (gemv_ok && (M == 1 || few || (M > 4 && wide))) return LNQ_KERNEL_GEMV;
@@ -847,8 +848,9 @@ LNQ_API LnqStatus lnq_int4_linear(const void* x, const uint8_t* packed, const vo
     return launch_int4_tiled(x, packed, scale, zero, bias, y, M, N, K, G, dtype,
                              code == LNQ_KERNEL_TILED_256 ? 256 : 128, s);
   // The rest of the few-row calls (LNQ_KERNEL_SKINNY as the plan names them) stream; the
-  // skinny kernel runs when it is asked for, and past the streaming kernel's widest layer.
-  if (kernel == LNQ_KERNEL_AUTO && int4_stream_supports(K))
+  // skinny kernel runs when it is asked for, where it is the faster one, and past the streaming
+  // kernel's widest layer.
+  if (kernel == LNQ_KERNEL_AUTO && int4_stream_supports(K) && !int4_skinny_preferred(M, N, K, G))
     return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
   if (dtype == LNQ_BF16)
     return launch_skinny<LNQ_BF16>(x, packed, scale, zero, bias, y, M, N, K, G, s);

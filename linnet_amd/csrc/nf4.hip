@@ -380,13 +380,11 @@ double stream_us(int64_t rows, int64_t out_features, int64_t in_features, int64_
   stream::Args a{};
   a.cols = static_cast<int>(in_features / block);
   a.row_block = 1;
-  int most = stream::fitting_rows<stream::NF4, 2, 2, 8, stream::ONE_STEP>(a), x_rows = 32;
-  if (most < 16) most = stream::fitting_rows<stream::NF4, 2, 1, 4, stream::ONE_STEP>(a), x_rows = 16;
-  const int r = stream::rows_per_block(static_cast<int>(out_features), most);
-  const int64_t groups = (out_features + r - 1) / r * ((rows + x_rows - 1) / x_rows);
+  int r = 0;
+  const int rounds = stream::rounds<stream::NF4, 2, stream::ONE_STEP>(a, rows, out_features, r);
   const double k = static_cast<double>(in_features) / 1024;
   const double round = r <= 16 ? 2.5 + 0.95 * k : r <= 32 ? 2.5 + 1.5 * k : 4.5 + 2.55 * k;
-  return (2.5 + round * ((groups + compute_units() - 1) / compute_units())) * (block == 32 ? 1.1 : 1.0);
+  return (2.5 + round * rounds) * (block == 32 ? 1.1 : 1.0);
 }
 
 double tiles_us(int64_t in_features) { return 6 + 1.45 * ((in_features + 255) / 256); }

@@ -619,6 +619,24 @@ inline void launch_nt(Args& a, int chunks, hipStream_t stream) {
 // 1 GiB, and the scales of 8 rows (groups of 32) fit beside the stages of 16 rows of x.
 constexpr int MAX_K = 65536;
 
+// Whole rounds of workgroups, one a CU, over `rows` > 16 rows of x (32 each, 16 where the scales
+// leave no room for more); r: the output rows of a workgroup.
+template <int F, int GPS, int KIND>
+inline int rounds(const Args& a, int64_t rows, int64_t out_features, int& r) {
+  int most = fitting_rows<F, GPS, 2, 8, KIND>(a), x_rows = 32;
+  if (most < 16) most = fitting_rows<F, GPS, 1, 4, KIND>(a), x_rows = 16;
+  r = rows_per_block(static_cast<int>(out_features), most);
+  const int64_t groups = (out_features + r - 1) / r * ((rows + x_rows - 1) / x_rows);
+  return static_cast<int>((groups + compute_units() - 1) / compute_units());
+}
+
+// Past about 4 MB of x the rows that every workgroup reads leave the L2s: measured over the
+// estimate of a round, 1.2 at 7 MB, 1.5 at 11, 2.0 at 29.
+inline double x_past_l2(int64_t rows, int64_t in_features) {
+  const double mb = static_cast<double>(rows) * in_features * 2e-6;
+  return mb > 4 ? 1 + (mb - 4) / 28 : 1.0;
+}
+
 // The dense product of M rows (a.R is set here): 4, 8, 16 or 32 rows of x a workgroup, 16
 // where the scales of very wide layers leave no room for more.
 template <int DT, int F, int GPS, int KIND = ONE_STEP>

@@ -91,6 +91,20 @@ def test_int4_scales_that_fill_the_lds(out: int, width: int) -> None:
     assert bool(((got - want).abs() <= 2 * ULP[BF16] * want.abs() + 2.0**-19 * carried).all())
 
 
+@pytest.mark.parametrize(("rows", "out", "width", "group"), [
+    (16, 2048, 512, 128), (24, 4096, 512, 64), (17, 1000, 1024, 128), (64, 4096, 1024, 128), (36, 2048, 2048, 256),
+    (48, 4096, 512, 32), (64, 8192, 256, 64), (65, 2048, 1536, 384), (600, 1024, 2176, 2176)])
+def test_int4_short_layers_keep_the_skinny_kernel(rows: int, out: int, width: int, group: int) -> None:
+    """Where the skinny kernel is the faster one the automatic choice has its bits."""
+    print(f"int4 short layer rows={rows} out={out} in={width} group={group}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    packed = torch.randint(0, 256, (out, width // group, group // 2), generator=g, dtype=torch.uint8, device=DEV)
+    scale = (torch.rand(out, width // group, generator=g, device=DEV) * 0.02 + 0.001).to(F16)
+    zero = torch.randint(0, 16, (out, width // group), generator=g, dtype=torch.uint8, device=DEV)
+    x = torch.randn(rows, width, generator=g, device=DEV).to(F16)
+    assert torch.equal(kernels.int4_linear(x, packed, scale, zero), kernels.int4_linear(x, packed, scale, zero, kernel="skinny"))
+
+
 @pytest.mark.parametrize("fp8", [True, False])
 @pytest.mark.parametrize(("rows", "out", "width", "group", "row_block", "dtype"), [
     (1, 72, 640, 0, 1, BF16),  # one row, a scale a row, 5 steps
