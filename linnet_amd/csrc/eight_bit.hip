@@ -613,7 +613,7 @@ LNQ_API LnqStatus lnq_w8a16(const void* x, const uint8_t* weight, const float* s
   // One row at K = 4096 over a narrow output keeps the row kernel, which loads a wave's
   // whole share at once (N = 4096 int8 5.9 against 6.4 us, N = 6144 FP8 7.9 against 7.1).
   const bool row_kernel = M == 1 && K == 4096 && N <= 4096 && G % 128 == 0;
-  if (!row_kernel && K <= stream::MAX_K)
+  if (!row_kernel && K <= stream::MAX_K && N <= stream::MAX_N)
     return (fp8 ? launch_fp8_stream : launch_int8_stream)(x, weight, scale, y, M, N, K, (int)group, rb, dtype, s);
   if (dtype == LNQ_BF16) {
     if (fp8) launch_w8_few<LNQ_BF16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);

@@ -650,7 +650,7 @@ LnqStatus launch_int4_mid(const void* x, const uint8_t* packed, const void* scal
                           void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
 
 // Defined in int4_stream.hip: the streaming few-row product.
-bool int4_stream_supports(int K);
+bool int4_stream_supports(int N, int K);
 bool int4_skinny_preferred(int M, int N, int K, int G);
 LnqStatus launch_int4_stream(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
                              const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t stream);
@@ -799,7 +799,8 @@ static int choose_int4_kernel(int M, int N, int K, int G, int dtype, int kernel,
 // 32-row GEMV, whose products the x-tile entry repeats bit for bit.
 static LnqStatus launch_few_tokens(const void* x, const uint8_t* packed, const void* scale, const uint8_t* zero,
                                    const void* bias, void* y, int M, int N, int K, int G, int dtype, hipStream_t s) {
-  if (M >= 5 && M <= 16) return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
+  if (M >= 5 && M <= 16 && int4_stream_supports(N, K))
+    return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
   return launch_int4_gemv(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
 }
 
@@ -850,7 +851,7 @@ LNQ_API LnqStatus lnq_int4_linear(const void* x, const uint8_t* packed, const vo
   // The rest of the few-row calls (LNQ_KERNEL_SKINNY as the plan names them) stream; the
   // skinny kernel runs when it is asked for, where it is the faster one, and past the streaming
   // kernel's widest layer.
-  if (kernel == LNQ_KERNEL_AUTO && int4_stream_supports(K) && !int4_skinny_preferred(M, N, K, G))
+  if (kernel == LNQ_KERNEL_AUTO && int4_stream_supports(N, K) && !int4_skinny_preferred(M, N, K, G))
     return launch_int4_stream(x, packed, scale, zero, bias, y, M, N, K, G, dtype, s);
   if (dtype == LNQ_BF16)
     return launch_skinny<LNQ_BF16>(x, packed, scale, zero, bias, y, M, N, K, G, s);

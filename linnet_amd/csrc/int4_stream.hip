@@ -4,7 +4,7 @@
 
 namespace lnq {
 
-bool int4_stream_supports(int K) { return K <= stream::MAX_K; }
+bool int4_stream_supports(int N, int K) { return K <= stream::MAX_K && N <= stream::MAX_N; }
 
 // Whether the skinny kernel is faster than the streaming one, for the calls that both take. It
 // gives 16 outputs and all the rows (64 of them past 64) a workgroup of four waves: less to do

@@ -356,7 +356,7 @@ bool gemv_preferred(int64_t rows, int64_t out_features, int64_t in_features) {
 bool stream_takes(int64_t rows, int64_t out_features, int64_t in_features, int64_t block, int64_t x_stride,
                   int64_t y_stride) {
   return !gemv_preferred(rows, out_features, in_features) && rows <= INT32_MAX &&
-         (block == 32 || block == 64 || block % 128 == 0) && in_features <= stream::MAX_K &&
+         (block == 32 || block == 64 || block % 128 == 0) && in_features <= stream::MAX_K && out_features <= stream::MAX_N &&
          x_stride < (int64_t{1} << 23) && y_stride <= INT32_MAX;
 }
 

@@ -618,6 +618,8 @@ inline void launch_nt(Args& a, int chunks, hipStream_t stream) {
 // In up to which the kernel takes any call: 32 rows of x and 64 of the weight stay below
 // 1 GiB, and the scales of 8 rows (groups of 32) fit beside the stages of 16 rows of x.
 constexpr int MAX_K = 65536;
+// Out up to which the grid's y holds the blocks of 8 or more outputs, eight a step.
+constexpr int MAX_N = 65535 * 64;
 
 // Whole rounds of workgroups, one a CU, over `rows` > 16 rows of x (32 each, 16 where the scales
 // leave no room for more); r: the output rows of a workgroup.

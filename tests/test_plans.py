@@ -58,3 +58,10 @@ def test_nf4_rows_far_apart_are_widened() -> None:
 def test_nf4_narrow_outputs_keep_the_gemv(rows: int, out: int, width: int, want: int) -> None:
     """One GEMV pass of at most a workgroup a unit: 4096 -> 1024 at 5 rows 5.0 us, streamed 5.9."""
     assert _nf4(rows, out, width) == want
+
+
+def test_nf4_outputs_past_the_streaming_grid() -> None:
+    """The grid's y holds 65535 steps of eight blocks."""
+    assert _nf4(16, 65535 * 64, 64) == STREAM
+    assert _nf4(16, 65535 * 64 + 1, 64) == GEMV
+    assert _nf4(17, 65535 * 64 + 1, 64) == WIDENED
