@@ -361,6 +361,13 @@ LNQ_API LnqStatus lnq_w8a16(const void* x, const uint8_t* weight, const float* s
                             int32_t fp8, int64_t group, int64_t row_block, int32_t dtype,
                             void* stream);
 
+/* The kernel lnq_w8a16 takes on the current device. No counterpart in the reference. */
+#define LNQ_W8_ROW 1
+#define LNQ_W8_STREAM 2
+#define LNQ_W8_SKINNY 3
+LNQ_API LnqStatus lnq_w8a16_plan(int64_t rows, int64_t out_features, int64_t in_features,
+                                 int64_t group, int64_t row_block, int32_t* chosen);
+
 /* The 8-bit weight dequantized: out[o, i] = widen(w[o, i]) * scale, f32 product
  * rounded once to `dtype`. Replaces: kernels.py:595-666 `dequantize8`. */
 LNQ_API LnqStatus lnq_dequantize8(const uint8_t* weight, const float* scale, void* out,

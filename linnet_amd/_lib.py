@@ -25,6 +25,7 @@ BF16, F16, F32 = 0, 1, 2
  KERNEL_SPLIT) = range(8)
 PROLOGUE_RMSNORM, PROLOGUE_SILU_MUL = 1, 2
 PACKING_GPTQ, PACKING_AWQ = 0, 1
+W8_ROW, W8_STREAM, W8_SKINNY = 1, 2, 3
 NF4_WIDENED, NF4_GEMV, NF4_STREAM, NF4_TILES = range(4)
 
 _p = ctypes.c_void_p
@@ -54,6 +55,7 @@ SIGNATURES: dict[str, list[object]] = {
     "lnq_int4_repack": [_p, _p, _p, _i32, _i32, _i64, _i64, _i64, _p, _p, _p],
     "lnq_int8_quantize": [_p, _p, _p, _i64, _i64, _i64, _i32, _p],
     "lnq_w8a16": [_p, _p, _p, _p, _i64, _i64, _i64, _i32, _i64, _i64, _i32, _p],
+    "lnq_w8a16_plan": [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i32)],
     "lnq_dequantize8": [_p, _p, _p, _i64, _i64, _i32, _i64, _i64, _i32, _p],
     "lnq_rows8": [_p, _p, _p, _i64, _i64, _i32, _i32, _p],
     "lnq_mm8": [_p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _i32, _p],

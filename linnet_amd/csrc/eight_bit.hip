@@ -534,19 +534,58 @@ LnqStatus launch_fp8_stream(const void* x, const uint8_t* w, const float* scale,
 LnqStatus launch_int8_stream(const void* x, const uint8_t* w, const float* scale, void* y, int M, int N, int K, int group,
                              int row_block, int dtype, hipStream_t stream);
 
-// The row kernel (one row, K = 4096, scales of 128 k inputs), or the skinny kernel where
-// the streaming product does not reach (stream::MAX_K).
+// The kernel of a call. One row at K = 4096 over a narrow output keeps the row kernel, which
+// loads a wave's whole share at once (N = 4096 int8 5.9 against 6.4 us streamed, N = 6144 FP8 7.9
+// against 7.1). The rest streams (stream.hpp; 8 rows 8192 -> 28672 FP8 39 us against 69 on the
+// skinny kernel, 24 rows 4096 -> 14336 int8 in groups of 128 16 against 46) but for layers past its
+// sizes, and from 33 rows on where estimates of both, fitted to 33 to 1024 rows of 12 layers, say
+// that the skinny kernel's 64 rows a workgroup take fewer rounds (us skinny / streaming, FP8, a
+// scale a row: 1024 -> 4096 33 rows 7.2 / 9.0; 2048 -> 2048 128 / 512 rows 12.2 / 19.3, 36 / 70; 4096
+// -> 4096 64 / 512 / 1024 rows 20.5 / 16.2, 131 / 115, 261 / 318; 14336 -> 1024 128 / 512 rows 59 /
+// 36, 115 / 158). Smaller groups cost the skinny kernel a fold each.
+static int w8_kernel(int M, int N, int K, int group, int row_block) {
+  const bool by_128 = group == 0 || group % 128 == 0;
+  if (M == 1 && K == 4096 && N <= 4096 && by_128) return LNQ_W8_ROW;
+  if (K > stream::MAX_K || N > stream::MAX_N) return LNQ_W8_SKINNY;
+  if (M <= 32) return LNQ_W8_STREAM;
+  const double k = K / 1024.0;
+  const int chunks = (M + 63) / 64, cus = compute_units();
+  const int64_t groups = static_cast<int64_t>((N + 15) / 16) * chunks;
+  const double fold = group == 0 ? 0 : by_128 ? 0.4 : 0.8;
+  const double skinny = 4 + static_cast<double>((groups + cus - 1) / cus) * (1.9 + 0.034 * M / chunks + fold) * k;
+  stream::Args a{};
+  a.cols = group == 0 ? 1 : K / group;
+  a.row_block = row_block;
+  int r = 0;
+  const int rounds = group == 0 ? stream::rounds<stream::FP8, 0, stream::ONE_STEP>(a, M, N, r)
+                                : stream::rounds<stream::FP8, 1, stream::BLOCK>(a, M, N, r);
+  const double round = r <= 16 ? 2.3 + 1.05 * k : r <= 32 ? 2.6 + 1.4 * k : 3.3 + 2.1 * k;
+  return skinny < 0.97 * (1.7 + round * rounds) * stream::x_past_l2(M, K) ? LNQ_W8_SKINNY : LNQ_W8_STREAM;
+}
+
+// The skinny kernel keeps more chunks in flight the fewer rows it has (K = 98304, N = 2048, FP8, one
+// row 105 us; in the form of 64 rows 215).
 template <int DT, int FP8>
-static void launch_w8_few(const void* x, const uint8_t* w, const float* s, void* y, int M,
+static void launch_w8_skinny(const void* x, const uint8_t* w, const float* s, void* y, int M,
                              int N, int K, int G, int rb, int cols, hipStream_t stream) {
   const auto* xs = static_cast<const uint16_t*>(x);
   auto* ys = static_cast<uint16_t*>(y);
-  if (M == 1 && K == 4096)
-    hipLaunchKernelGGL((w8_row_slices_kernel<DT, FP8>), dim3((N + 15) / 16), dim3(1024), 0, stream, xs, w, s, ys, N, G,
-                       rb, cols);
+  if (M <= 16)
+    hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 1>), dim3((N + 15) / 16, 1), dim3(256), 0, stream,
+                       xs, w, s, ys, M, N, K, G, rb, cols);
+  else if (M <= 32)
+    hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 2>), dim3((N + 15) / 16, 1), dim3(256), 0, stream,
+                       xs, w, s, ys, M, N, K, G, rb, cols);
   else
     hipLaunchKernelGGL((w8_skinny_kernel<DT, FP8, 4>), dim3((N + 15) / 16, (M + 63) / 64), dim3(256),
                        0, stream, xs, w, s, ys, M, N, K, G, rb, cols);
+}
+
+template <int DT, int FP8>
+static void launch_w8_row(const void* x, const uint8_t* w, const float* s, void* y, int N, int G, int rb, int cols,
+                          hipStream_t stream) {
+  hipLaunchKernelGGL((w8_row_slices_kernel<DT, FP8>), dim3((N + 15) / 16), dim3(1024), 0, stream,
+                     static_cast<const uint16_t*>(x), w, s, static_cast<uint16_t*>(y), N, G, rb, cols);
 }
 
 }  // namespace lnq
@@ -607,22 +646,40 @@ LNQ_API LnqStatus lnq_w8a16(const void* x, const uint8_t* weight, const float* s
   const int rb = group == 0 ? 1 : (int)row_block;
   const int cols = group == 0 ? 1 : (int)(in_features / group);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // Several rows, and one where the row kernels do not take it, on the streaming product (a
-  // decode batch of 8 at 8192 -> 28672 FP8 69 us on the skinny kernel, 24 rows at 4096 ->
-  // 14336 int8 in groups 46: it reads all of x for each 16 outputs).
-  // One row at K = 4096 over a narrow output keeps the row kernel, which loads a wave's
-  // whole share at once (N = 4096 int8 5.9 against 6.4 us, N = 6144 FP8 7.9 against 7.1).
-  const bool row_kernel = M == 1 && K == 4096 && N <= 4096 && G % 128 == 0;
-  if (!row_kernel && K <= stream::MAX_K && N <= stream::MAX_N)
+  const int kernel = w8_kernel(M, N, K, (int)group, rb);
+  if (kernel == LNQ_W8_STREAM)
     return (fp8 ? launch_fp8_stream : launch_int8_stream)(x, weight, scale, y, M, N, K, (int)group, rb, dtype, s);
-  if (dtype == LNQ_BF16) {
-    if (fp8) launch_w8_few<LNQ_BF16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
-    else launch_w8_few<LNQ_BF16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
-  } else {
-    if (fp8) launch_w8_few<LNQ_F16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
-    else launch_w8_few<LNQ_F16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+  if (kernel == LNQ_W8_ROW) {
+    if (dtype == LNQ_BF16) {
+      if (fp8) launch_w8_row<LNQ_BF16, 1>(x, weight, scale, y, N, G, rb, cols, s);
+      else launch_w8_row<LNQ_BF16, 0>(x, weight, scale, y, N, G, rb, cols, s);
+    } else {
+      if (fp8) launch_w8_row<LNQ_F16, 1>(x, weight, scale, y, N, G, rb, cols, s);
+      else launch_w8_row<LNQ_F16, 0>(x, weight, scale, y, N, G, rb, cols, s);
+    }
+    return launched("w8_row");
   }
-  return launched("w8_few");
+  if (dtype == LNQ_BF16) {
+    if (fp8) launch_w8_skinny<LNQ_BF16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    else launch_w8_skinny<LNQ_BF16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+  } else {
+    if (fp8) launch_w8_skinny<LNQ_F16, 1>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+    else launch_w8_skinny<LNQ_F16, 0>(x, weight, scale, y, M, N, K, G, rb, cols, s);
+  }
+  return launched("w8_skinny");
+}
+
+LNQ_API LnqStatus lnq_w8a16_plan(int64_t rows, int64_t out_features, int64_t in_features, int64_t group,
+                                 int64_t row_block, int32_t* chosen) {
+  LNQ_REQUIRE(chosen != nullptr, "lnq_w8a16_plan: null pointer");
+  LNQ_REQUIRE(rows > 0 && out_features > 0 && in_features > 0 && in_features % 128 == 0 && rows <= INT32_MAX &&
+                  out_features <= INT32_MAX && in_features <= INT32_MAX && group % 64 == 0 &&
+                  check_scales(out_features, in_features, group, row_block) == nullptr,
+              "lnq_w8a16_plan: bad shape rows=%lld in=%lld out=%lld group=%lld", (long long)rows, (long long)in_features,
+              (long long)out_features, (long long)group);
+  *chosen = w8_kernel((int)rows, (int)out_features, (int)in_features, (int)group, group == 0 ? 1 : (int)row_block);
+  clear_error();
+  return LNQ_OK;
 }
 
 LNQ_API LnqStatus lnq_dequantize8(const uint8_t* weight, const float* scale, void* out,

@@ -114,6 +114,10 @@ def test_int4_short_layers_keep_the_skinny_kernel(rows: int, out: int, width: in
     (31, 48, 3840, 384, 1, BF16),  # a group of three steps
     (33, 60, 1152, 192, 5, F16),  # groups of 1.5 steps, a scale row for 5 weight rows
     (64, 1024, 1024, 128, 128, BF16),  # block scales
+    (1, 24, 65664, 0, 1, BF16),  # past the streaming kernel's inputs: the skinny kernel's 16-,
+    (20, 40, 65664, 128, 1, F16),  # 32-
+    (40, 24, 65664, 64, 1, BF16),  # and 64-row forms
+    (130, 300, 1024, 128, 1, F16),  # past 64 rows, where the skinny kernel is the faster one
 ])
 def test_eight_bit(fp8: bool, rows: int, out: int, width: int, group: int, row_block: int, dtype: torch.dtype) -> None:
     print(f"w8 stream fp8={fp8} rows={rows} out={out} in={width} group={group}/{row_block} {dtype}", flush=True)
@@ -141,6 +145,7 @@ def test_eight_bit(fp8: bool, rows: int, out: int, width: int, group: int, row_b
     (17, 130, 1024, 128, F16),
     (24, 72, 14336, 64, BF16),
     (96, 1000, 1536, 512, BF16),
+    (9, 40, 8256, 64, BF16),  # In ends inside a step, long
 ])
 def test_nf4(rows: int, out: int, width: int, block: int, dtype: torch.dtype) -> None:
     print(f"nf4 stream rows={rows} out={out} in={width} block={block} {dtype}", flush=True)

@@ -65,3 +65,22 @@ def test_nf4_outputs_past_the_streaming_grid() -> None:
     assert _nf4(16, 65535 * 64, 64) == STREAM
     assert _nf4(16, 65535 * 64 + 1, 64) == GEMV
     assert _nf4(17, 65535 * 64 + 1, 64) == WIDENED
+
+
+@pytest.mark.parametrize(("rows", "out", "width", "group", "row_block", "want"), [
+    (1, 4096, 4096, 0, 1, _lib.W8_ROW), (1, 4096, 4096, 64, 1, _lib.W8_STREAM), (1, 4112, 4096, 128, 128, None),
+    (1, 6144, 4096, 0, 1, _lib.W8_STREAM), (32, 2048, 2048, 0, 1, _lib.W8_STREAM), (33, 4096, 1024, 0, 1, _lib.W8_SKINNY),
+    (64, 4096, 4096, 128, 128, _lib.W8_STREAM), (128, 2048, 2048, 128, 1, _lib.W8_SKINNY),
+    (512, 14336, 4096, 0, 1, _lib.W8_STREAM), (512, 1024, 14336, 64, 1, _lib.W8_SKINNY),
+    (1, 64, 65536, 0, 1, _lib.W8_STREAM), (1, 64, 65664, 0, 1, _lib.W8_SKINNY),
+    (1, 65535 * 64 + 1, 128, 0, 1, _lib.W8_SKINNY)])
+def test_eight_bit_kernels(rows: int, out: int, width: int, group: int, row_block: int, want: int | None) -> None:
+    """`want` None: scale blocks that do not tile the weight are refused."""
+    chosen = ctypes.c_int32(-1)
+    args = ("lnq_w8a16_plan", rows, out, width, group, row_block, ctypes.byref(chosen))
+    if want is None:
+        with pytest.raises(_lib.LinnetError):
+            _lib.call(*args)
+        return
+    _lib.call(*args)
+    assert chosen.value == want
