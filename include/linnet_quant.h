@@ -456,6 +456,12 @@ LNQ_API LnqStatus lnq_mxfp4_experts(const void* x, int64_t x_row_stride, int64_t
                                     int64_t num_experts, int64_t out_features,
                                     int64_t in_features, int32_t dtype, void* stream);
 
+/* How lnq_mxfp4_experts takes a call on the current device (x within its limits): 8, 16 or
+ * 32 of an expert's pairs a pass over its weights, or 0 for a pass a pair. No counterpart in
+ * the reference. */
+LNQ_API LnqStatus lnq_mxfp4_experts_plan(int64_t rows, int64_t chosen, int64_t num_experts,
+                                         int64_t out_features, int64_t in_features, int32_t* pass);
+
 /* ------------------------------------------------------------------------- NF4
  * std.quant::Nf4Linear (stdlib/quant.linnet:177-215): codes [out, in/2] bytes of
  * QLoRA's 4-bit NormalFloat, the first input of a pair in the low nibble, and

@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list[object]] = {
     "lnq_fp8_groups": [_p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p],
     "lnq_mm8_block": [_p, _p, _p, _i64, _p, _p, _i64, _i64, _i64, _i32, _p],
     "lnq_mxfp4_experts": [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _i32, _p],
+    "lnq_mxfp4_experts_plan": [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i32)],
     "lnq_nf4_dequant": [_p, _p, _p, _i64, _i64, _i64, _i32, _p],
     "lnq_nf4_linear": [_p, _i64, _i64, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _p],
     "lnq_nf4_linear_plan": [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i32)],

@@ -221,12 +221,39 @@ static void launch_grouped(const ExpertArgs& g, hipStream_t stream) {
 }
 
 template <int DT>
-static void launch_grouped_dt(const ExpertArgs& g, hipStream_t stream) {
-  // Rows of x a pass by the pairs an expert has on average.
-  if (g.pairs <= g.num_experts) launch_grouped<DT, 1, 1>(g, stream);
-  else if (g.pairs <= 3 * g.num_experts) launch_grouped<DT, 1, 2>(g, stream);
-  else if (g.pairs <= 12 * g.num_experts) launch_grouped<DT, 1, 4>(g, stream);
+static void launch_grouped_dt(const ExpertArgs& g, int pass, hipStream_t stream) {
+  if (pass == 8) launch_grouped<DT, 1, 2>(g, stream);
+  else if (pass == 16) launch_grouped<DT, 1, 4>(g, stream);
   else launch_grouped<DT, 2, 8>(g, stream);
+}
+
+// The pairs of an expert that the grouped kernel multiplies a pass (8, 16 or 32, by the pairs an
+// expert has on average; 16 at least for one choice a token, where a single expert may hold them
+// all), or 0 for a workgroup a pair. Estimates of both in us, for routers that spread their choices,
+// fitted to 1 to 1024 tokens of 1 to 8 choices over 4 to 128 experts in eight layers from 1024 ->
+// 1024 to 4096 -> 14336. A pair costs its expert's bytes again, from the caches past the first, and
+// each wave's lane slots. The grouped kernel costs a pass of an expert its units of 256 inputs,
+// whatever the pairs in it, their longest chain first, and the listing in every workgroup.
+// us, pair / grouped: 2880 -> 5760, 32 experts, top 4: 4 tokens 32.4 / 38.8, 8 59.4 / 54.9, 32 227 / 80,
+// 256 1590 / 190; top 1: 16 tokens 32.9 / 44.7; 4096 -> 1536, 128 experts, top 1: 64 tokens 40.2 / 60.3,
+// 256 145 / 106; 1024 -> 1024, 8 of 128: 8 tokens 8.5 / 17. Routers that send every token to the same
+// experts are not what is estimated: over a narrow layer the pair kernel's reads of one expert then
+// come from the caches, and the grouped kernel has few workgroups (4096 -> 1536, 128 experts, top 1,
+// 1024 tokens to one expert 368 / 608; of wide layers the grouped kernel is ahead there too, 2880 ->
+// 5760, 32 tokens 55 / 29).
+static int mxfp4_pass(int64_t rows, int64_t chosen, int64_t num_experts, int64_t out_features, int64_t in_features) {
+  const double pairs = static_cast<double>(rows) * chosen, experts = static_cast<double>(num_experts);
+  const int pass = pairs > 12 * experts ? 32 : chosen == 1 || pairs > 3 * experts ? 16 : 8;
+  const double named = experts * (1 - std::pow(1 - std::fmin(1.0, chosen / experts), static_cast<double>(rows)));
+  const int64_t groups = in_features / 32, slots = (groups + 63) / 64;
+  const double mb = static_cast<double>(out_features) * groups * 17e-6;
+  const double pair = 3.5 + mb * (0.05 * pairs + 0.018 * named) +
+                      1.74e-3 * pairs * ((out_features + 15) / 16) * slots + 0.33 * slots;
+  const double units = 0.5 * ((in_features + 127) / 128);
+  const double blocks = static_cast<double>((out_features + stream::MAX_R - 1) / stream::MAX_R) / compute_units();
+  const double passes = named + 1.5 * std::fmax(0.0, pairs / pass - 0.5 * named);
+  const double grouped = 4.04 + 1.58 * std::ceil(std::ceil(units) / mx::GROUP_WAVES) + blocks * (0.49 * passes * units + 0.19 * (experts + 1));
+  return grouped < 0.97 * pair ? pass : 0;
 }
 
 }  // namespace lnq
@@ -258,19 +285,13 @@ LNQ_API LnqStatus lnq_mxfp4_experts(const void* x, int64_t x_row_stride, int64_t
   hipStream_t s = static_cast<hipStream_t>(stream);
   const auto* xs = static_cast<const uint16_t*>(x);
   auto* ys = static_cast<uint16_t*>(y);
-  const int64_t pairs = rows * chosen;
-  // The grouped kernel costs about 4 us more than this one for what it reads once (the
-  // list, its barriers), so it is taken where it saves 16 MB of weights read again: the
-  // pairs past the experts that evenly spread choices would name (2880 -> 5760, 32
-  // experts, top 4: 6 tokens 45.2 against 48.6 us, 8 53.8 / 61.9, 16 66.8 / 113, 32 79 /
-  // 214, 64 93 / 409; 1056 -> 1501, 8 experts, top 2: 8 tokens 8.1 / 7.1, 16 8.6 / 11.4).
   // x as the range-checked buffers need it: below 1 GiB, rows and slots forward.
   const int64_t x_span = (rows - 1) * x_row_stride + (chosen - 1) * x_slot_stride + in_features;
-  const double named = static_cast<double>(num_experts) * (1.0 - std::pow(1.0 - 1.0 / static_cast<double>(num_experts), static_cast<double>(pairs)));
-  const double again = (static_cast<double>(pairs) - named) * static_cast<double>(out_features * groups * 17);
-  if (in_features >= 32 && again > 16e6 && x_row_stride >= 0 && x_slot_stride >= 0 &&
-      x_span < (int64_t{1} << 29) && num_experts < 65535 && out_features <= (1 << 24) &&
-      chosen <= mx::MAX_PAIRS) {
+  const int pass = in_features >= 32 && x_row_stride >= 0 && x_slot_stride >= 0 && x_span < (int64_t{1} << 29) &&
+                           num_experts < 65535 && out_features <= (1 << 24) && chosen <= mx::MAX_PAIRS
+                       ? mxfp4_pass(rows, chosen, num_experts, out_features, in_features)
+                       : 0;
+  if (pass) {
     ExpertArgs g{};
     g.a.w = blocks;
     g.a.scale = scales;
@@ -293,8 +314,8 @@ LNQ_API LnqStatus lnq_mxfp4_experts(const void* x, int64_t x_row_stride, int64_t
       g.a.y = ys + r0 * chosen * out_features;
       g.experts = experts + r0 * chosen;
       g.pairs = static_cast<int>(rc * chosen);
-      if (dtype == LNQ_BF16) launch_grouped_dt<LNQ_BF16>(g, s);
-      else launch_grouped_dt<LNQ_F16>(g, s);
+      if (dtype == LNQ_BF16) launch_grouped_dt<LNQ_BF16>(g, pass, s);
+      else launch_grouped_dt<LNQ_F16>(g, pass, s);
       const LnqStatus st = launched("mxfp4_grouped");
       if (st != LNQ_OK) return st;
     }
@@ -324,6 +345,18 @@ LNQ_API LnqStatus lnq_mxfp4_experts(const void* x, int64_t x_row_stride, int64_t
 #undef LNQ_MX_S
 #undef LNQ_MX
   return launched("mxfp4_experts");
+}
+
+LNQ_API LnqStatus lnq_mxfp4_experts_plan(int64_t rows, int64_t chosen, int64_t num_experts, int64_t out_features,
+                                         int64_t in_features, int32_t* pass) {
+  LNQ_REQUIRE(pass != nullptr, "lnq_mxfp4_experts_plan: null pointer");
+  LNQ_REQUIRE(rows > 0 && chosen > 0 && num_experts > 0 && out_features > 0 && in_features > 0 && in_features % 32 == 0,
+              "lnq_mxfp4_experts_plan: bad shape rows=%lld chosen=%lld experts=%lld in=%lld out=%lld",
+              static_cast<long long>(rows), static_cast<long long>(chosen), static_cast<long long>(num_experts),
+              static_cast<long long>(in_features), static_cast<long long>(out_features));
+  *pass = mxfp4_pass(rows, chosen, num_experts, out_features, in_features);
+  clear_error();
+  return LNQ_OK;
 }
 
 }  // extern "C"

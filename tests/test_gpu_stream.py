@@ -189,7 +189,8 @@ def test_nf4_tiles(rows: int, out: int, width: int, block: int, dtype: torch.dty
     (40, 4, 8, 1500, 2880, False),  # In ends inside a step; 20 pairs an expert on average
     (24, 2, 4, 3000, 1056, True),  # one expert takes most pairs (several passes), some are out of range
     (600, 4, 2, 70, 256, False),  # more pairs than a launch lists
-    (16, 4, 16, 2048, 2048, False),  # 4 pairs an expert: the 8-row form
+    (16, 4, 16, 2048, 2048, False),  # 4 pairs an expert: 16 a pass
+    (11, 4, 16, 2050, 2880, True),  # 8 a pass, several passes of one expert
 ])
 def test_mxfp4_grouped(dtype: torch.dtype, rows: int, chosen: int, count: int, out: int, width: int, skew: bool) -> None:
     print(f"mxfp4 grouped rows={rows} chosen={chosen} E={count} out={out} in={width} {dtype}", flush=True)
