@@ -413,6 +413,11 @@ LNQ_API LnqStatus lnq_mm8_tiles(const uint8_t* q, const uint8_t* weight, const f
 LNQ_API LnqStatus lnq_mm8_plan(int64_t rows, int64_t out_features, int64_t in_features,
                                int32_t fp8, int32_t* tile_n);
 
+/* The rows of lnq_mm8's tiles for that call, or of lnq_mm8_block's (block_scaled 1): 32, 64
+ * or 128 (by 64 columns), or 256. No counterpart in the reference. */
+LNQ_API LnqStatus lnq_mm8_rows_plan(int64_t rows, int64_t out_features, int64_t in_features,
+                                    int32_t fp8, int32_t block_scaled, int32_t* tile_rows);
+
 /* Each 128 inputs (group = 128) of each row of x [rows, in] (`dtype`: bf16, f16 or f32)
  * rounded to FP8 E4M3 with a scale of their own: scale = max(max|x|, 1e-12) / 448
  * (f32, IEEE divide), q = E4M3 round-to-nearest-even of clamp(x / scale, +-448); rows

@@ -852,4 +852,19 @@ LNQ_API LnqStatus lnq_mm8_plan(int64_t rows, int64_t out_features, int64_t in_fe
   return LNQ_OK;
 }
 
+LNQ_API LnqStatus lnq_mm8_rows_plan(int64_t rows, int64_t out_features, int64_t in_features, int32_t fp8,
+                                    int32_t block_scaled, int32_t* tile_rows) {
+  LNQ_REQUIRE(tile_rows != nullptr, "lnq_mm8_rows_plan: null pointer");
+  LNQ_REQUIRE(rows > 0 && out_features > 0 && in_features > 0 && in_features % 128 == 0 && rows <= INT32_MAX &&
+                  out_features <= INT32_MAX && in_features <= INT32_MAX,
+              "lnq_mm8_rows_plan: bad shape rows=%lld in=%lld out=%lld", (long long)rows, (long long)in_features,
+              (long long)out_features);
+  const int M = static_cast<int>(rows), N = static_cast<int>(out_features), K = static_cast<int>(in_features);
+  const int bn = block_scaled ? 128 : mm8_kernel_for(M, N, K, fp8 != 0);
+  const int bm = bn == 128 || bn == LNQ_MM8_STREAM ? mm8_small_rows(M, N, K, block_scaled != 0) : 0;
+  *tile_rows = bm ? bm : 256;
+  clear_error();
+  return LNQ_OK;
+}
+
 }  // extern "C"

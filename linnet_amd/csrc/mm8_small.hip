@@ -274,27 +274,29 @@ static LnqStatus launch_tile(int bm, const uint8_t* qx, const uint8_t* weight, c
   return launch<DT, FP8, 128, 64, BLK>(qx, weight, x_scale, scale, y, M, N, K, xs_stride, s);
 }
 
-// Rows of the tile to take, or 0 for the 256 x 128 tiles. Estimates in us, fitted to calls of
-// 48 to 777 rows of 2048 -> 2048, 3072 -> 9216, 4096 -> 14336, 14336 -> 4096 and 8192 -> 28672
-// (within a fifth of those). A small tile's step takes its latency or, where several
-// workgroups share a CU, their work in turn; the weights' own time from memory (4.87 bytes a
-// picosecond) adds in where the two are alike. A large tile's step takes 0.7 us where the
-// tiles share few columns of the weight (14336 -> 4096) and 1 us where each reads its own
-// (4096 -> 14336), its block form 1.05 and 1.2, and the rounds are whole. Small tiles have to
-// win by a twentieth.
+// Rows of the tile to take, or 0 for the 256 x 128 tiles: the least of estimates in us, fitted to
+// the fastest of the four at 16 to 1500 rows of 19 layers from 1024 -> 1024 to 8192 -> 28672 (in the
+// mean 0.5 percent off that). A large tile costs its steps a round, or the weights' own time from
+// memory (4.87 bytes a picosecond); a small tile's step its latency or, where several workgroups share
+// a CU, their work in turn, a partial second round half a whole one. Small tiles have to win by 4
+// percent. us large / 32 / 64 / 128 rows: int8 48 rows 4096 -> 14336 27.7 / 18.8 / 17.6 / 20.4, 160 rows
+// 6144 -> 12288 45.1 / 53.8 / 44.8 / 37.0, 777 rows 1024 -> 4096 16.7 / 16.4 / 13.9 / 12.1, 513 rows
+// 14336 -> 4096 72.3 / 97.4 / 79.6 / 80.4; block-scaled 300 rows 8192 -> 28672 115 / 199 / 154 / 137.
 int mm8_small_rows(int M, int N, int K, bool blk) {
   const double cus = compute_units(), steps = K / 128;
   const double memory = static_cast<double>(N) * K / 4.87e6;
-  const double columns = std::ceil(N / 128.0), rounds = std::ceil(std::ceil(M / 256.0) * columns / cus);
-  const double shared = std::min(columns, 128.0);
-  const double step256 = blk ? 1.0 + 0.0015 * shared : 0.62 + 0.0032 * shared;
-  double best = 0.95 * (4 + steps * step256 * rounds);
+  const double tiles = std::ceil(M / 256.0) * std::ceil(N / 128.0) / cus;
+  const double large = steps * (blk ? 0.85 * std::ceil(tiles) + 0.05 * tiles : 0.8 * std::ceil(tiles) + 0.09 * tiles);
+  double best = 0.96 * ((blk ? 5.65 : 6.27) + std::max(large, 1.07 * memory));
   int rows = 0;
-  constexpr struct { int bm; double latency, work; } kinds[] = {{32, 0.27, 0.155}, {64, 0.36, 0.235}, {128, 0.46, 0.42}};
-  for (const auto& k : kinds) {
+  struct Kind { int bm; double base, latency, work; };
+  static constexpr Kind plain[] = {{32, 2.7, 0.19, 0.21}, {64, 2.73, 0.29, 0.29}, {128, 4.3, 0.48, 0.38}};
+  static constexpr Kind block[] = {{32, 2.7, 0.22, 0.21}, {64, 2.73, 0.32, 0.3}, {128, 4.3, 0.5, 0.38}};
+  for (const Kind& k : blk ? block : plain) {
     double c = std::ceil(static_cast<double>(M) / k.bm) * std::ceil(N / 64.0) / cus;
-    if (c > 2) c = (c + std::ceil(c)) / 2;  // past the two a CU holds, a partial round costs half a whole one
-    const double t = 4 + std::hypot(steps * std::max(k.latency, c * k.work), memory);
+    if (c > 2) c = std::ceil(c);
+    else if (c > 1) c = (c + std::ceil(c)) / 2;
+    const double t = k.base + steps * std::max(k.latency, c * k.work);
     if (t < best) best = t, rows = k.bm;
   }
   return rows;
