@@ -236,10 +236,10 @@ static void launch_grouped_dt(const ExpertArgs& g, int pass, hipStream_t stream)
 // whatever the pairs in it, their longest chain first, and the listing in every workgroup.
 // us, pair / grouped: 2880 -> 5760, 32 experts, top 4: 4 tokens 32.4 / 38.8, 8 59.4 / 54.9, 32 227 / 80,
 // 256 1590 / 190; top 1: 16 tokens 32.9 / 44.7; 4096 -> 1536, 128 experts, top 1: 64 tokens 40.2 / 60.3,
-// 256 145 / 106; 1024 -> 1024, 8 of 128: 8 tokens 8.5 / 17. Routers that send every token to the same
+// 256 145 / 106; 1024 -> 1024, 32 experts, top 4: 2 tokens 4.6 / 7.6, 16 14.4 / 8.5. Routers that send every token to the same
 // experts are not what is estimated: over a narrow layer the pair kernel's reads of one expert then
 // come from the caches, and the grouped kernel has few workgroups (4096 -> 1536, 128 experts, top 1,
-// 1024 tokens to one expert 368 / 608; of wide layers the grouped kernel is ahead there too, 2880 ->
+// 1024 tokens to one expert 366 / 793; of wide layers the grouped kernel is ahead there too, 2880 ->
 // 5760, 32 tokens 55 / 29).
 static int mxfp4_pass(int64_t rows, int64_t chosen, int64_t num_experts, int64_t out_features, int64_t in_features) {
   const double pairs = static_cast<double>(rows) * chosen, experts = static_cast<double>(num_experts);

@@ -370,7 +370,7 @@ bool tiles_take(int64_t rows, int64_t out_features, int64_t block, int64_t x_str
 }
 
 // Estimated us past 16 rows, fitted to 17 to 512 rows of 27 layers from 512 -> 4096 to 14336 ->
-// 28672 (nine in ten within 10, 7 and 15 percent). The streaming kernel: whole rounds of its
+// 28672 (nine in ten within 13, 10 and 20 percent). The streaming kernel: whole rounds of its
 // workgroups, 32 rows of x each (16 where the scales of a wide layer take the LDS), by the 16-row
 // tiles that a workgroup holds. Measured streaming / tiles / widened, block 64: 64 rows 4096 ->
 // 14336 32.8 / 30.2 / 60.6, 4096 -> 4096 14.6 / 29.3 / 30.7; 96 rows 4096 -> 14336 48.3 / 30.9 /

@@ -632,8 +632,8 @@ inline int rounds(const Args& a, int64_t rows, int64_t out_features, int& r) {
   return static_cast<int>((groups + compute_units() - 1) / compute_units());
 }
 
-// Past about 4 MB of x the rows that every workgroup reads leave the L2s: measured over the
-// estimate of a round, 1.2 at 7 MB, 1.5 at 11, 2.0 at 29.
+// Past about 4 MB of x the rows that every workgroup reads leave the L2s: calls took 1.1 to 1.5
+// times the estimate by rounds at 8 MB, 1.3 to 1.7 at 15, 1.9 to 2.1 at 29.
 inline double x_past_l2(int64_t rows, int64_t in_features) {
   const double mb = static_cast<double>(rows) * in_features * 2e-6;
   return mb > 4 ? 1 + (mb - 4) / 28 : 1.0;
