@@ -560,7 +560,7 @@ static int w8_kernel(int M, int N, int K, int group, int row_block) {
   const int rounds = group == 0 ? stream::rounds<stream::FP8, 0, stream::ONE_STEP>(a, M, N, r)
                                 : stream::rounds<stream::FP8, 1, stream::BLOCK>(a, M, N, r);
   const double round = r <= 16 ? 2.3 + 1.05 * k : r <= 32 ? 2.6 + 1.4 * k : 3.3 + 2.1 * k;
-  return skinny < 0.97 * (1.7 + round * rounds) * stream::x_past_l2(M, K) ? LNQ_W8_SKINNY : LNQ_W8_STREAM;
+  return skinny < 0.97 * (1.7 + round * rounds) * stream::x_past_l2(M, K, r) ? LNQ_W8_SKINNY : LNQ_W8_STREAM;
 }
 
 // The skinny kernel keeps more chunks in flight the fewer rows it has (K = 98304, N = 2048, FP8, one

@@ -36,7 +36,7 @@ bool int4_skinny_preferred(int M, int N, int K, int G) {
   int r = 0;
   const int rounds = stream::rounds<stream::INT4, 4, stream::ONE_STEP>(a, M, N, r);
   const double round = r <= 16 ? 2.45 + 0.9 * k : r <= 32 ? 2.95 + 1.15 * k : 3 + 1.85 * k;
-  return skinny < 0.97 * (1.75 + round * rounds) * stream::x_past_l2(M, K);
+  return skinny < 0.97 * (1.75 + round * rounds) * stream::x_past_l2(M, K, r);
 }
 
 template <int DT>

@@ -632,11 +632,12 @@ inline int rounds(const Args& a, int64_t rows, int64_t out_features, int& r) {
   return static_cast<int>((groups + compute_units() - 1) / compute_units());
 }
 
-// Past about 4 MB of x the rows that every workgroup reads leave the L2s: calls took 1.1 to 1.5
-// times the estimate by rounds at 8 MB, 1.3 to 1.7 at 15, 1.9 to 2.1 at 29.
-inline double x_past_l2(int64_t rows, int64_t in_features) {
+// Past about 4 MB of x the rows that every workgroup reads leave the L2s: calls of 16 outputs a
+// workgroup took 1.1 to 1.5 times the estimate by rounds at 8 MB, 1.3 to 1.7 at 15, 1.9 to 2.1 at 29;
+// of r outputs, 16 / r of the excess (14336 -> 14336 2048 rows, 56 a workgroup, 59 MB: 1.3).
+inline double x_past_l2(int64_t rows, int64_t in_features, int r) {
   const double mb = static_cast<double>(rows) * in_features * 2e-6;
-  return mb > 4 ? 1 + (mb - 4) / 28 : 1.0;
+  return mb > 4 ? 1 + (mb - 4) / 24 * 16 / (r > 16 ? r : 16) : 1.0;
 }
 
 // The dense product of M rows (a.R is set here): 4, 8, 16 or 32 rows of x a workgroup, 16
