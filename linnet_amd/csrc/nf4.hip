@@ -409,14 +409,15 @@ int kernel_for(int64_t rows, int64_t out_features, int64_t in_features, int64_t 
 }
 
 // Whether the stored weight is the faster one for that kernel: always up to 64 rows, by the
-// estimates above that, and past 96 rows only in tiles (the library's product gains on further
-// passes: 160 rows 4096 -> 14336 77.8 streamed, 66.9 widened). The GEMV keeps 16 rows (8 past In =
-// 8192); more are its passes over the weight again.
-bool stored_preferred(int kernel, int64_t rows, int64_t out_features, int64_t in_features, int64_t block) {
+// estimates above past them, and past 96 rows only where the tiles could take it too (the library's
+// product gains on further passes: 160 rows 4096 -> 14336 77.8 streamed, 66.9 widened; 128 rows 14336
+// -> 4096 69.7 streamed, 87.3 in tiles, 95.1 widened). The GEMV keeps 16 rows (8 past In = 8192); more
+// are its passes over the weight again.
+bool stored_preferred(int kernel, int64_t rows, int64_t out_features, int64_t in_features, int64_t block, bool tiles) {
   if (kernel == LNQ_NF4_GEMV) return rows <= (in_features <= 8192 ? 16 : 8);
   if (rows <= 64) return true;
   const double us = kernel == LNQ_NF4_TILES ? tiles_us(in_features) : stream_us(rows, out_features, in_features, block);
-  return (rows <= 96 || kernel == LNQ_NF4_TILES) && us < widened_us(rows, out_features, in_features);
+  return (rows <= 96 || tiles) && us < widened_us(rows, out_features, in_features);
 }
 
 template <int DT>
@@ -591,9 +592,10 @@ LNQ_API LnqStatus lnq_nf4_linear_plan(int64_t rows, int64_t x_stride, int64_t ou
       in_features <= nf4::UNIT * nf4::THREADS * nf4::MAX_SLOTS && out_features <= INT32_MAX &&
       out_features * (in_features / 2) < (int64_t{1} << 31) && x_stride >= in_features && x_stride % 8 == 0) {
     // Any 16-byte aligned address stands for the codes.
-    const int kernel = kernel_for(rows, out_features, in_features, block, x_stride, out_features,
-                                  reinterpret_cast<const void*>(static_cast<uintptr_t>(256)));
-    if (stored_preferred(kernel, rows, out_features, in_features, block)) *chosen = kernel;
+    const void* const codes = reinterpret_cast<const void*>(static_cast<uintptr_t>(256));
+    const int kernel = kernel_for(rows, out_features, in_features, block, x_stride, out_features, codes);
+    const bool tiles = tiles_take(rows, out_features, block, x_stride, out_features, codes);
+    if (stored_preferred(kernel, rows, out_features, in_features, block, tiles)) *chosen = kernel;
   }
   clear_error();
   return LNQ_OK;
