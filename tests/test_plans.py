@@ -91,7 +91,7 @@ def test_eight_bit_kernels(rows: int, out: int, width: int, group: int, row_bloc
     (1, 4, 32, 5760, 2880, 0), (4, 4, 32, 5760, 2880, 0),  # 32 us a pass a pair, 39 grouped
     (16, 1, 32, 5760, 2880, 0), (12, 1, 32, 5760, 2880, 0), (64, 1, 128, 1536, 4096, 0),  # 40 and 60
     (16, 4, 128, 1536, 4096, 0), (8, 2, 8, 1536, 4096, 0), (8, 8, 128, 1024, 1024, 0), (4, 8, 128, 2880, 2880, 0),
-    (12, 4, 32, 5760, 2880, 8), (32, 4, 32, 5760, 2880, 16), (256, 4, 32, 5760, 2880, 32), (64, 1, 32, 5760, 2880, 16),
+    (12, 4, 32, 5760, 2880, 8), (32, 4, 32, 5760, 2880, 16), (256, 4, 32, 5760, 2880, 32), (64, 1, 32, 5760, 2880, 8),
     (64, 2, 8, 1501, 1056, 32), (64, 4, 128, 1536, 4096, 8), (1024, 1, 4, 1024, 1024, 32)])
 def test_mxfp4_pairs_a_pass(rows: int, chosen: int, experts: int, out: int, width: int, want: int) -> None:
     got = ctypes.c_int32(-1)
