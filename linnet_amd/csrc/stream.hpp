@@ -47,11 +47,8 @@ enum Format { INT4 = 0, NF4 = 1, FP4 = 2, INT8 = 3, FP8 = 4 };
 constexpr int STEP = 128;   // inputs of a step
 constexpr int WAVES = 8;    // waves of a dense workgroup
 constexpr int MAX_R = 64;   // output rows of a workgroup
-constexpr int RING = 1;     // weight units a wave has in flight
-// Offsets past every buffer's range (each spans less than 1 GiB): a row that does not
-// exist, and a step past the wave's end; their sum stays outside too.
+// An offset past every buffer's range (each spans less than 1 GiB): a row that does not exist.
 constexpr uint32_t NO_ROW = 0x40000000u;
-constexpr uint32_t NO_STEP = 0x80000000u;
 
 constexpr bool eight(int f) { return f == INT8 || f == FP8; }
 // Formats whose widened codes are offset (int4 by MAGIC + zero, int8 in bf16 by 128; in
@@ -286,7 +283,7 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   __builtin_amdgcn_sched_barrier(0);
   // The step rides in the scalar offset; a step past the wave's end reads through a
   // descriptor of no bytes (at offset 0), which returns zeros and moves nothing.
-  u32x4 wr[RING][NT][2];
+  u32x4 wr[NT][2];
   auto load_w = [&](int u, int T, u32x4 (&dst)[2]) {
     const bool live = u < u1;
     const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(wbase, live ? wbytes : 0u);
@@ -342,10 +339,10 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   // land, and its next unit asked for as soon as it is widened.
   auto compute = [&](int u, int d0, u32x4 (&w)[NT][2]) {
     // The unit's stages have landed: all but the loads issued after theirs, the other
-    // stages' and the ring's (loads retire in order; the order of issue is held by the
+    // stages' and the weights' (loads retire in order; the order of issue is held by the
     // scheduling barriers below). The wait is explicit: the compiler's own tracking of
     // loads into LDS let a read of the second stage pass ahead of its loads.
-    wait_vm<(D - US) * XI + 2 * NT * RING>();
+    wait_vm<(D - US) * XI + 2 * NT>();
     u32x4 xa[US][MT][4];
 #pragma unroll
     for (int h = 0; h < US; ++h)
@@ -459,7 +456,7 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
           }
         }
       }
-      load_w(u + RING, T, w[T]);
+      load_w(u + 1, T, w[T]);
     }
   };
 
@@ -471,25 +468,22 @@ __device__ inline void product(const Args& a, int n0, int n_end, const uint16_t*
   // first waves' weights (a bare barrier: nothing has to land).
   __asm__ volatile("s_barrier" ::: "memory");
 #pragma unroll
-  for (int d = 0; d < RING; ++d)
-#pragma unroll
-    for (int T = 0; T < NT; ++T) {
-      load_w(u0 + d, T, wr[d][T]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
+  for (int T = 0; T < NT; ++T) {
+    load_w(u0, T, wr[T]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if constexpr (GPS > 0) {
     // The scales, issued before everything else, have landed; again a bare barrier (a fence
     // would wait for the x stages too).
-    wait_vm<D * XI + 2 * RING * NT>();
+    wait_vm<D * XI + 2 * NT>();
     __asm__ volatile("s_barrier" ::: "memory");
   }
-  constexpr int TURN = US == 2 ? RING : 2;  // units until the stages and the ring both come round
-  static_assert(US * TURN % D == 0 && TURN % RING == 0, "stages and ring repeat with the loop");
+  constexpr int TURN = D / US;  // units until the stages come round
   for (int u = u0; u < u1; u += TURN) {
 #pragma unroll
     for (int d = 0; d < TURN; ++d) {
       if (u + d >= u1) break;
-      compute(u + d, d * US, wr[d % RING]);
+      compute(u + d, d * US, wr);
     }
   }
 
