@@ -34,6 +34,8 @@
 // sums (ROWS x rows of x) go through LDS, [output][lane] with the lanes
 // contiguous, and 256 / (ROWS * MR) lanes add each output's 256 partial sums in
 // a fixed order.
+#include <cmath>
+
 #include "stream.hpp"
 
 namespace lnq {
@@ -384,15 +386,19 @@ double stream_us(int64_t rows, int64_t out_features, int64_t in_features, int64_
   const int rounds = stream::rounds<stream::NF4, 2, stream::ONE_STEP>(a, rows, out_features, r);
   const double k = static_cast<double>(in_features) / 1024;
   const double round = r <= 16 ? 2.5 + 0.95 * k : r <= 32 ? 2.5 + 1.5 * k : 4.5 + 2.55 * k;
-  return (2.5 + round * rounds) * (block == 32 ? 1.1 : 1.0);
+  return (2.5 + round * rounds) * (block != 32 ? 1.0 : r <= 32 ? 1.1 : 1.25);
 }
 
 double tiles_us(int64_t in_features) { return 6 + 1.45 * ((in_features + 255) / 256); }
 
-// The widened weight and the library's product of it.
+// The widened weight and the library's product of it: up to 96 rows its bytes (past 80 M weights
+// the 16-bit weight leaves the last-level cache between the two), then the rows' products too. The
+// library's own choices scatter it: 96 rows 3584 -> 18944 69 us with the stored weight in memory, 59
+// with it in the cache, 14336 -> 4096 128 / 192 / 256 rows 95 / 115 / 86.
 double widened_us(int64_t rows, int64_t out_features, int64_t in_features) {
-  const double weights = static_cast<double>(out_features) * in_features;
-  return 10.4 + weights * (0.9e-6 + 1.33e-9 * rows) + 0.86 / 1024 * in_features;
+  const double millions = 1e-6 * static_cast<double>(out_features) * in_features, k = in_features / 1024.0;
+  if (rows <= 96) return 11.5 + 0.74 * millions + k + 0.45 * std::fmax(0.0, millions - 80);
+  return 10.4 + millions * (0.9 + 1.33e-3 * rows) + 0.86 * k;
 }
 
 // The kernel of a call that lnq_nf4_linear's checks let through. No tiles up to 16 rows, where

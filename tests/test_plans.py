@@ -34,7 +34,7 @@ def test_nf4_few_rows_over_wide_outputs_take_no_tiles(out: int, width: int, bloc
     (128, 14336, 4096, 64, TILES), (97, 4096, 14336, 64, STREAM),  # 67 us streamed, 88 in tiles, 75 widened
     (97, 2048, 14336, 64, WIDENED),  # 63 us streamed, 48 widened
     (96, 9216, 3072, 32, WIDENED),  # blocks of 32 have no tiles: 47 us streamed, 39 widened
-    (64, 9216, 3072, 32, STREAM), (96, 14336, 4096, 32, STREAM), (200, 14336, 4096, 64, WIDENED),  # two tiles a unit
+    (64, 9216, 3072, 32, STREAM), (96, 18944, 3584, 64, WIDENED), (96, 14336, 4096, 32, STREAM), (200, 14336, 4096, 64, WIDENED),  # two tiles a unit
     (17, 64, 65536, 64, WIDENED), (17, 1 << 20, 8192, 64, WIDENED),  # lnq_nf4_linear refuses
     (16, 64, 1024, 16, GEMV), (17, 64, 1024, 16, WIDENED),  # blocks that only the GEMV takes
     (9, 64, 16384, 16, WIDENED)])
