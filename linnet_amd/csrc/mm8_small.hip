@@ -275,30 +275,31 @@ static LnqStatus launch_tile(int bm, const uint8_t* qx, const uint8_t* weight, c
 }
 
 // Rows of the tile to take, or 0 for the 256 x 128 tiles: the least of estimates in us, fitted to
-// the fastest of the four at 16 to 1500 rows of 35 layers from 1024 -> 1024 to 8192 -> 28672 (in the
-// mean 0.6 percent off that). A large tile costs its steps a round, or the weights' own time from
-// memory (4.87 bytes a picosecond). A small tile's step costs its latency or, where several workgroups
-// share a CU, their work in turn, a partial second round 0.6 of a whole one, or all of it where one row
-// of tiles reads each weight but once; the weights' time adds in where the two are alike. Small tiles
-// have to win by 4 percent. us large / 32 / 64 / 128 rows: int8 48 rows 4096 -> 14336 27.7 / 18.8 / 17.6 /
-// 20.4, 160 rows 6144 -> 12288 45.1 / 53.8 / 44.8 / 37.0, 777 rows 1024 -> 4096 16.7 / 16.4 / 13.9 / 12.1, 513
-// rows 14336 -> 4096 72.3 / 97.4 / 79.6 / 80.4; block-scaled 128 rows 5120 -> 25600 42.0 / 69.4 / 60.0 /
-// 51.5, 300 rows 8192 -> 28672 115 / 199 / 154 / 137.
+// the fastest of the four at 16 to 1500 rows of 35 layers from 1024 -> 1024 to 8192 -> 28672, with the
+// weights in memory and in the last-level cache alike (in the mean 0.8 and 0.5 percent off the
+// fastest). A large tile costs its steps a round, or the weights' own time from memory (4.87 bytes a
+// picosecond). A small tile's step costs its latency or, where several workgroups share a CU, their
+// work in turn; a partial second round costs 0.55 of a whole one, further ones all of it. Small tiles
+// have to win by 3 percent. us large / 32 / 64 / 128 rows, weights from memory: int8 48 rows 4096 ->
+// 14336 27.7 / 18.8 / 17.6 / 20.4, 160 rows 6144 -> 12288 45.1 / 53.8 / 44.8 / 37.0, 777 rows 1024 ->
+// 4096 16.7 / 16.4 / 13.9 / 12.1; block-scaled 300 rows 8192 -> 28672 115 / 199 / 154 / 137, 128 rows
+// 4096 -> 14336 29.3 / 33.2 / 25.0 / 22.6 (from the cache 28.2 / 26.1 / 17.5 / 19.8). Between 16384 and
+// 28672 outputs one row of tiles reads every weight once, and the large tiles have them from memory the
+// faster (block-scaled 128 rows 5120 -> 25600 42.0 / 69.4 / 60.0 / 51.5, from the cache 36.7 / 50.0 / 41.4 / 35.8).
 int mm8_small_rows(int M, int N, int K, bool blk) {
   const double cus = compute_units(), steps = K / 128;
   const double memory = static_cast<double>(N) * K / 4.87e6;
   const double rounds = std::ceil(std::ceil(M / 256.0) * std::ceil(N / 128.0) / cus);
-  double best = 0.96 * ((blk ? 3.13 : 5.49) + std::max(steps * rounds * (blk ? 0.85 : 0.75), 1.07 * memory));
+  double best = 0.97 * ((blk ? 2.96 : 3.77) + std::max(steps * rounds * (blk ? 0.84 : 0.83), 1.16 * memory));
   int rows = 0;
   struct Kind { int bm; double base, latency, work; };
-  static constexpr Kind plain[] = {{32, 1.3, 0.2, 0.2}, {64, 1.42, 0.28, 0.27}, {128, 2.67, 0.45, 0.34}};
-  static constexpr Kind block[] = {{32, 1.3, 0.23, 0.22}, {64, 1.42, 0.32, 0.29}, {128, 2.67, 0.49, 0.37}};
+  static constexpr Kind plain[] = {{32, 0.1, 0.21, 0.2}, {64, 0.1, 0.28, 0.27}, {128, 1.56, 0.47, 0.36}};
+  static constexpr Kind block[] = {{32, 0.1, 0.24, 0.22}, {64, 0.1, 0.32, 0.3}, {128, 1.56, 0.64, 0.36}};
   for (const Kind& k : blk ? block : plain) {
-    const bool one = M <= k.bm;
     double c = std::ceil(static_cast<double>(M) / k.bm) * std::ceil(N / 64.0) / cus;
-    if (c > 2 || (one && c > 1)) c = std::ceil(c);
-    else if (c > 1) c += 0.6 * (2 - c);
-    const double t = k.base + std::hypot(steps * std::max(k.latency, c * k.work), (one ? 0.74 : 0.83) * memory);
+    if (c > 2) c = std::ceil(c);
+    else if (c > 1) c += 0.55 * (2 - c);
+    const double t = k.base + steps * std::max(k.latency, c * k.work);
     if (t < best) best = t, rows = k.bm;
   }
   return rows;

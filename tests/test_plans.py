@@ -100,10 +100,10 @@ def test_mxfp4_pairs_a_pass(rows: int, chosen: int, experts: int, out: int, widt
 
 
 @pytest.mark.parametrize(("rows", "out", "width", "block", "want"), [
-    (48, 14336, 4096, 0, 64), (16, 14336, 4096, 0, 32), (128, 14336, 4096, 0, 128), (256, 4096, 14336, 0, 64), (512, 4096, 14336, 0, 128),
+    (48, 14336, 4096, 0, 64), (16, 14336, 4096, 0, 32), (128, 14336, 4096, 0, 64), (256, 4096, 14336, 0, 64), (512, 4096, 14336, 0, 128),
     (160, 12288, 6144, 0, 128),  # 45 us in 256 rows, 54 in 32, 37 in 128
     (1500, 12288, 6144, 0, 256), (777, 14336, 4096, 1, 256), (300, 28672, 8192, 1, 256),  # 115 us, 154 in 64
-    (128, 25600, 5120, 1, 256), (64, 28672, 4096, 0, 64), (128, 18944, 3584, 0, 128),
+    (128, 25600, 5120, 1, 128), (64, 28672, 4096, 0, 64), (128, 18944, 3584, 0, 128),
     (257, 28672, 4096, 1, 256), (257, 12288, 6144, 1, 256), (640, 14336, 4096, 1, 256), (33, 2048, 2048, 1, 32)])
 def test_eight_bit_tile_rows(rows: int, out: int, width: int, block: int, want: int) -> None:
     got = ctypes.c_int32(-1)
