@@ -487,12 +487,13 @@ LNQ_API LnqStatus lnq_nf4_dequant(const uint8_t* codes, const float* absmax, voi
 /* y[r, o] = sum_i x[r, i] * weight[o, i] (+ bias[o]) for `rows` rows of x
  * (row strides in elements), x / bias / y of `dtype` (bf16 or f16). The weight
  * is read as stored: each code's value, rounded once to `dtype`, meets x in an
- * f32 dot product; a block's sum is scaled by its absmax and the blocks added in
- * f32, the row rounded once. Up to 8 rows of x a pass over the weight (4 past
- * in = 8192). block %
- * 16 == 0, in % block == 0, in <= 32768, the codes under 2 GiB; x 16-byte aligned
- * with x_stride % 8 == 0. Replaces: `linear_nf4`'s body, the widened weight and
- * its product (stdlib/quant.linnet:189-199), for the few-row calls. */
+ * f32 dot product; a block's sum is scaled by its absmax and the blocks and the bias
+ * added in f32, the row rounded once. Any number of rows: the fewest on a GEMV (8 a
+ * pass over the weight, 4 past in = 8192), more on the streaming product (32 a pass)
+ * or 64 x 128 tiles (lnq_nf4_linear_plan names which). block % 16 == 0, in % block ==
+ * 0, in <= 32768, the codes under 2 GiB; x 16-byte aligned with x_stride % 8 == 0.
+ * Replaces: `linear_nf4`'s body, the widened weight and its product
+ * (stdlib/quant.linnet:189-199). */
 LNQ_API LnqStatus lnq_nf4_linear(const void* x, int64_t x_stride, int64_t rows, const uint8_t* codes,
                                  const float* absmax, const void* bias, void* y, int64_t y_stride,
                                  int64_t out_features, int64_t in_features, int64_t block,

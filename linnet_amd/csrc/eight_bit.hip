@@ -1,7 +1,8 @@
 // 8-bit weights (std.quant::Int8Linear / Int8GroupLinear / Fp8Linear / Fp8BlockLinear)
 // on gfx950:
-//   - w8_skinny:  weight-only product for few rows (gemv8 / w8a16), weights
-//                 widened in registers and multiplied on MFMA, x unrounded;
+//   - w8_skinny:  weight-only product (w8a16) where the streaming one (stream.hpp) takes
+//                 more rounds or does not reach (w8_kernel), weights widened in registers
+//                 and multiplied on MFMA, x unrounded; w8_row_slices: one row, short K;
 //   - dequant8:   the weight widened and scaled, rounded to the output dtype;
 //   - rows8:      dynamic per-token FP8 / int8 rounding of activations;
 //   - mm8:        int8 x int8 (int32 sums) or FP8 x FP8 (f32 sums) tiled MFMA GEMM

@@ -11,7 +11,8 @@
 // block's sum times its scale (v_ldexp_f32, exact) is added to the row's sum in
 // f32, as the reference applies the scale after the block's products.
 //
-// Layout of the work: one workgroup per (row, chosen slot) pair and 16 output
+// Layout of the work (the pair kernel; calls whose pairs share experts take the grouped
+// one, mxfp4_pass): one workgroup per (row, chosen slot) pair and 16 output
 // rows of its expert, 4 waves of 4 rows. Lane l owns blocks l, l + 64, ... of
 // every row it visits, so its 32 inputs of x per block stay in registers across
 // the rows and a wave's weight loads read 64 consecutive blocks (1 KB) of a row.
@@ -228,18 +229,19 @@ static void launch_grouped_dt(const ExpertArgs& g, int pass, hipStream_t stream)
 }
 
 // The pairs of an expert that the grouped kernel multiplies a pass (8, 16 or 32, by the pairs an
-// expert has on average), or 0 for a workgroup a pair. Estimates of both in us, for routers that spread their choices,
-// fitted to 1 to 1024 tokens of 1 to 8 choices over 4 to 128 experts in eight layers from 1024 ->
-// 1024 to 4096 -> 14336. A pair costs its expert's bytes again, from the caches past the first, and
-// each wave's lane slots. The grouped kernel costs a pass of an expert its units of 256 inputs,
-// whatever the pairs in it, their longest chain first, and the listing in every workgroup.
+// expert has on average), or 0 for a workgroup a pair. Estimates of both in us, for routers that
+// spread their choices, fitted to 1 to 1024 tokens of 1 to 8 choices over 4 to 128 experts in eight
+// layers from 1024 -> 1024 to 4096 -> 14336. A pair costs its expert's bytes again, from the caches
+// past the first, and each wave's lane slots. The grouped kernel costs a pass of an expert its units
+// of 256 inputs, whatever the pairs in it, their longest chain first, and the listing in every
+// workgroup.
 // us, pair / grouped: 2880 -> 5760, 32 experts, top 4: 4 tokens 32.4 / 38.8, 8 59.4 / 54.9, 32 227 / 80,
 // 256 1590 / 190; top 1: 16 tokens 32.9 / 43.3; 4096 -> 1536, 128 experts, top 1: 64 tokens 40.2 / 66.0,
-// 256 145 / 101; 1024 -> 1024, 32 experts, top 4: 2 tokens 4.6 / 7.6, 16 14.4 / 8.5. Routers that send every token to the same
-// experts are not what is estimated: over a narrow layer the pair kernel's reads of one expert then
-// come from the caches, and the grouped kernel has few workgroups (4096 -> 1536, 128 experts, top 1,
-// 1024 tokens to one expert 366 / 793; of wide layers the grouped kernel is ahead there too, 2880 ->
-// 5760, 32 tokens of top 1 to one of 32 experts 55 / 44).
+// 256 145 / 101; 1024 -> 1024, 32 experts, top 4: 2 tokens 4.6 / 7.6, 16 14.4 / 8.5. Routers that
+// send every token to the same experts are not what is estimated: over a narrow layer the pair
+// kernel's reads of one expert then come from the caches, and the grouped kernel has few workgroups
+// (4096 -> 1536, 128 experts, top 1, 1024 tokens to one expert 366 / 793; of wide layers the grouped
+// kernel is ahead there too, 2880 -> 5760, 32 tokens of top 1 to one of 32 experts 55 / 44).
 static int mxfp4_pass(int64_t rows, int64_t chosen, int64_t num_experts, int64_t out_features, int64_t in_features) {
   const double pairs = static_cast<double>(rows) * chosen, experts = static_cast<double>(num_experts);
   const int pass = pairs > 12 * experts ? 32 : pairs > 3 * experts ? 16 : 8;

@@ -4,13 +4,15 @@
 // `block` consecutive inputs of a row, absmax [Out, In / block]:
 //     weight[o, i] = nf4(q[o, i]) * absmax[o, i / block].
 //
-// Three kernels:
+// Three kernels here, and two more that lnq_nf4_linear launches (kernel_for): the streaming
+// product (stream.hpp) and the 64 x 128 tiles (int4_mid.hip).
 // - nf4_dequant_kernel: the weight in T, the f32 product of the code's value and
 //   the scale rounded once (`dequantize_nf4`, quant.linnet:180-187), bit for bit.
 // - nf4_gemv_kernel: y = x W^T (+ bias), up to 8 rows of x a pass, the weight read
 //   once from HBM as it is stored (lnq_nf4_linear's fewest rows, and the blocks the
-//   streaming product and the tiles do not take: gemv_preferred, kernel_for). NF4's values are no affine function of the
-//   code, so the widening is a table lookup done in registers: the 16 values'
+//   streaming product and the tiles do not take: gemv_preferred, kernel_for). NF4's
+//   values are no affine function of the code, so the widening is a table lookup done
+//   in registers: the 16 values'
 //   16-bit patterns (bf16 or f16, x's type) are held as two 16-byte planes (low
 //   bytes, high bytes) in 8 SGPRs, and v_perm_b32 selects four codes' bytes from
 //   a plane at once (two perms over the 8-entry halves, v_bfi_b32 on the code's

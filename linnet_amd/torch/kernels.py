@@ -829,8 +829,9 @@ def nf4_dequantize(codes: torch.Tensor, absmax: torch.Tensor, block: int, dtype:
 
 
 # Rows of x up to which `nf4_linear` reads the stored weight for every block of a multiple
-# of 16 inputs (`lnq_nf4_linear`: its GEMV, 8 rows a pass up to In = 8192 and 4 past it, or
-# the streaming kernel). The GEMV, bf16, graph-replayed, against 57 us for the widened weight
+# of 16 inputs, also where the streaming kernel does not take the block and the GEMV serves
+# the call (8 rows a pass up to In = 8192 and 4 past it; past these rows the library is asked,
+# `lnq_nf4_linear_plan`). The GEMV, bf16, graph-replayed, against 57 us for the widened weight
 # and its product: 4096 -> 14336 at 1 / 8 / 16 rows 12.0 / 21.6 / 41.8 us; 14336 -> 4096 at
 # 1 / 8 / 12 rows 11.5 / 35.3 / 52.5 us.
 NF4_GEMV_ROWS = 16
@@ -839,7 +840,7 @@ NF4_GEMV_MAX_IN = 32768
 
 
 def nf4_gemv_fits(rows: int, in_features: int, block: int, dtype: torch.dtype) -> bool:
-    """Whether `nf4_linear` takes the GEMV for this call."""
+    """Whether `nf4_linear` reads the stored weight for this call without asking the library."""
     limit = NF4_GEMV_ROWS if in_features <= 8192 else NF4_GEMV_ROWS_WIDE
     return (dtype in _HALF and rows <= limit and block % 16 == 0 and in_features % block == 0
             and 0 < in_features <= NF4_GEMV_MAX_IN)

@@ -4,9 +4,9 @@ The layer holds what `linnet_amd.quant.import_quantized` writes for a
 bitsandbytes NF4 checkpoint: `weight` [Out, In/2] uint8 (QLoRA's 4-bit
 NormalFloat codes, the first input of a pair in the low nibble), `absmax`
 [Out, In/block] float32 and an optional `bias` in the activation dtype. Its
-forward is `linear_nf4`: bf16 / f16 x of up to 96 rows, and of more where 64 x 128
-tiles fit (`kernels.nf4_linear`), meets the weight as stored; other calls widen the
-weight with the HIP dequantize kernel (bit for bit the reference's
+forward is `linear_nf4`: bf16 / f16 x of few rows, and of more where the library
+estimates it the faster (`kernels.nf4_linear`), meets the weight as stored; other
+calls widen the weight with the HIP dequantize kernel (bit for bit the reference's
 `dequantize_nf4`) and multiply in x's type, as the reference's body does.
 """
 

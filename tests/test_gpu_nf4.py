@@ -3,16 +3,17 @@
 - `lnq_nf4_dequant` is bit-exact against the oracle's `dequantize_nf4` (the f32
   product of the code's value and its block's absmax, rounded once) for bf16,
   f16 and f32, with rows whose bytes do and do not split in 8.
-- The NF4 GEMV (`lnq_nf4_linear`, 1-16 rows of bf16 / f16 x, 8 a pass up to In = 8192) is checked against
-  the oracle's f64 product over the exact f32 weight, within 1e-2 of the
+- The product with the stored weight (`lnq_nf4_linear`, bf16 / f16 x; the GEMV, the
+  streaming product or 64 x 128 tiles) is checked at 1-16 rows against the oracle's f64 product over the exact f32 weight, within 1e-2 of the
   largest output plus the 16-bit rounding of each one (the reference's
   tolerance for its quantized products, `python/linnet/tests/test_quant_groups.py:165-195`):
   the kernel rounds each code's value to x's type, as the reference's body
   rounds the scaled weight to T. Shapes cover In below one unit a lane, a
   ragged last unit slot, In = 32768 (8 slots), blocks of 16 to 256, a bias,
   and Llama-3.1-8B's 4096 -> 14336 and 14336 -> 4096.
-- More rows (past 16, or 8 past In = 8192), f32 and blocks the GEMV does not take go through the dequantize
-  kernel and the product in x's type (the reference's body); f32 is held to
+- f32, blocks that are no multiple of 16 and, of more rows, what the stored weight is not
+  estimated the faster for go through the dequantize kernel and the product in x's type
+  (the reference's body); f32 is held to
   1e-5 as the reference's NF4 test holds its f32 layer
   (`python/linnet/tests/test_nf4.py:103-115`).
 - `import_quantized` on a bitsandbytes NF4 checkpoint built as the reference's
@@ -82,7 +83,8 @@ def test_gemv_against_f64(dtype: torch.dtype, rows: int, out_features: int, in_f
     gen = torch.Generator().manual_seed(rows + in_features)
     x = torch.randn(rows, in_features, generator=gen).to(dtype)
     b = torch.randn(out_features, generator=gen).to(dtype) if bias else None
-    # The GEMV itself at every row count (several passes past 8 rows), whatever nf4_linear picks.
+    # The stored weight at every row count, whatever nf4_linear picks: the GEMV up to 4 rows (2 past
+    # In = 4096) and, in several passes past 8, with blocks of 16; the streaming product else.
     got = kernels.nf4_gemv(x.to(DEV), torch.from_numpy(codes).to(DEV), torch.from_numpy(absmax).to(DEV), block,
                            None if b is None else b.to(DEV))
     want = linear.nf4_reference_f64(x.float().numpy(), codes, absmax, block, None if b is None else b.float().numpy())
@@ -94,7 +96,7 @@ def test_gemv_against_f64(dtype: torch.dtype, rows: int, out_features: int, in_f
     (1, 64, 16, 16), (4, 40, 48, 16), (16, 72, 4096, 64), (3, 1000, 14336, 128)])
 def test_gemv_uses_the_rounded_nf4_values(dtype: torch.dtype, rows: int, out_features: int, in_features: int,
                                           block: int) -> None:
-    """The GEMV's arithmetic, pinned tightly: each code's value rounded to x's
+    """The stored product's arithmetic, pinned tightly: each code's value rounded to x's
     type, products summed in f32, each block's sum scaled by its absmax, the
     output rounded once. Against the f64 sum over the rounded values: half a unit
     in the last place of the output's type plus 16 f32 units of the row's
@@ -130,6 +132,8 @@ def test_gemv_takes_strided_rows_and_leading_axes() -> None:
     (torch.bfloat16, 17, 64), (torch.float16, 33, 64), (torch.bfloat16, 3, 8), (torch.float32, 1, 64),
     (torch.float32, 40, 64)])
 def test_wider_calls_widen_then_multiply(dtype: torch.dtype, rows: int, block: int) -> None:
+    # Of these the 17 and 33 rows take what the library estimates the faster (the stored weight);
+    # the blocks of 8 and the f32 rows are widened.
     print(f"nf4 linear rows {rows} block {block} {dtype}", flush=True)
     assert not kernels.nf4_gemv_fits(rows, 1024, block, dtype)
     codes, absmax = _layer(200, 1024, block, rows)
