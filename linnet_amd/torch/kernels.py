@@ -868,8 +868,13 @@ def _nf4_reads_stored(x: torch.Tensor, codes: torch.Tensor, bias: torch.Tensor |
     if not ((bias is None or (bias.dtype == x.dtype and bias.shape == (out_features,))) and (
             (x.data_ptr() % 16 == 0 or not x.is_contiguous()) and (codes.data_ptr() % 16 == 0 or not codes.is_contiguous()))):
         return False
-    # The rows as `nf4_gemv` passes them: a view where they lie evenly, else a copy.
-    stride = in_features if x.is_contiguous() else x.reshape(-1, in_features).stride(0)
+    # The rows as `nf4_gemv` passes them: a view where they lie evenly, else a copy of its own.
+    stride = in_features
+    if not x.is_contiguous():
+        try:
+            stride = x.view(-1, in_features).stride(0)
+        except RuntimeError:
+            pass
     chosen = ctypes.c_int32(0)
     with _on(x.device):
         _lib.call("lnq_nf4_linear_plan", rows, max(stride, in_features) if stride % 8 == 0 else in_features, out_features,

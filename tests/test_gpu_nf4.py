@@ -376,3 +376,14 @@ def test_subclasses_and_modes_see_the_product() -> None:
     with Seen():
         got = kernels.nf4_linear(x, codes, absmax, 64)
     assert torch.equal(got, want) and any("mm" in n or "linear" in n for n in names)
+
+
+def test_rows_that_are_no_view_are_copied_once() -> None:
+    """x whose leading axes do not fold into one: the choice of the kernel takes no copy of it."""
+    _, codes, absmax, weight = _few_rows_past_the_gemv(24, 72)
+    x = torch.randn(8, 3, 256, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV).transpose(0, 1)
+    want = torch.nn.functional.linear(x, weight)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    assert kernels._nf4_reads_stored(x, codes, None, 24, 64)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+    torch.testing.assert_close(kernels.nf4_linear(x, codes, absmax, 64), want, rtol=1e-2, atol=1e-2 * want.abs().max().item())
